@@ -132,6 +132,14 @@ struct qhg_pop {
     uint32_t *d_wave_part = nullptr;
     uint64_t *d_scan_part = nullptr;   // 3 per k_cell_scan wave (grid <= ntiles blocks)
     unsigned long long *d_digest = nullptr;   // 2 sums of qhg_gpu_state_digest (allocated at its first call)
+    // reading agents back: the live ids' bitmap with its prefixes (rank_bytes,
+    // allocated at the first read, doubled as the ids grow), and a pinned
+    // host buffer for small reads (its first word is the read's error flag)
+    char *d_rank = nullptr;
+    int64_t rank_bytes = 0;
+    char *h_read = nullptr, *d_read = nullptr;
+    size_t read_bytes = 0;
+    std::mutex read_mu;       // readers on several threads share the scratch above
     DevStatus *d_st = nullptr;
 
     // Navigate: the navigation as set (ports in cell order, each port's
@@ -296,6 +304,7 @@ int64_t device_bytes(const qhg_pop *p) {
     if (p->d_coastal) per_cell += 1;
     b += nc * per_cell + 3 * 4;
     if (p->has_nav) b += nc * (4 + 4 + 8 + 4) + 8 + (int64_t)p->nnav * (4 + 8 + 4 + 4 + 4 + 4);
+    b += p->rank_bytes;
     b += 2 * (int64_t)p->ntiles * 8 + (int64_t)p->ntiles * 4 + (int64_t)p->num_cu * kMaxBlocksPerCu * kParts * 4 +
          (int64_t)p->ntiles * (kScanBlock / kWave) * 3 * 8 +
          (int64_t)sizeof(DevStatus);
@@ -734,6 +743,195 @@ int refresh_known(qhg_pop *p) {
     if (rc) return rc;
     p->known = s;
     p->known_step = p->steps_enqueued;
+    return 0;
+}
+
+// ids below this are ordered by their bitmap (at most 256 MB of it); a host
+// that numbers its agents sparsely beyond that takes the sorting path
+constexpr int64_t kRankIdLimit = (int64_t)1 << 31;
+// reads up to this size are written by the kernel straight into pinned host
+// memory and copied out by the CPU: nine copies cost ~12 us each however
+// small, this path one wait
+constexpr size_t kReadPinned = (size_t)4 << 20;
+
+// the bitmap and its prefixes for ids up to max_id
+int rank_map(qhg_pop *p, int64_t max_id, RankMap *m) {
+    m->words = max_id / 64 + 1;
+    m->tiles = (int32_t)((m->words + kRankTile - 1) / kRankTile);
+    const int64_t need = m->words * 12 + (int64_t)m->tiles * 4;
+    if (need > p->rank_bytes) {
+        HIPCHK(hipStreamSynchronize(p->stream));
+        if (p->d_rank) (void)hipFree(p->d_rank);
+        p->d_rank = nullptr;
+        p->rank_bytes = 0;
+        int64_t bytes = 65536;
+        while (bytes < need) bytes *= 2;
+        if (hipMalloc(&p->d_rank, (size_t)bytes) != hipSuccess) return fail(QHG_ERR_NOMEM, "read-back bitmap");
+        p->rank_bytes = bytes;
+    }
+    m->bits = reinterpret_cast<unsigned long long *>(p->d_rank);
+    m->pre = reinterpret_cast<uint32_t *>(p->d_rank + m->words * 8);
+    m->base = m->pre + m->words;
+    return 0;
+}
+
+// pinned host memory of at least `bytes`, with its device address
+int read_buffer(qhg_pop *p, size_t bytes) {
+    if (bytes <= p->read_bytes) return 0;
+    if (p->h_read) (void)hipHostFree(p->h_read);
+    p->h_read = p->d_read = nullptr;
+    p->read_bytes = 0;
+    size_t cap = 4096;
+    while (cap < bytes) cap *= 2;
+    if (hipHostMalloc((void **)&p->h_read, cap, hipHostMallocMapped) != hipSuccess)
+        return fail(QHG_ERR_NOMEM, "pinned read-back buffer");
+    HIPCHK(hipHostGetDevicePointer((void **)&p->d_read, p->h_read, 0));
+    p->read_bytes = cap;
+    return 0;
+}
+
+// The live agents in id order, ordered on the device (aux_kernels.hpp).  The
+// buffer the next step writes is free between steps and takes the arrays;
+// the list scratch takes the order and the cells.
+int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
+    std::lock_guard<std::mutex> lock(p->read_mu);
+    const int b = p->cur();
+    const int64_t n = s.n_alive[b];
+    struct Field { const void *host; size_t size; void *dev; };
+    const AgentBuf &nx = p->buf[1 - b];
+    const Field fields[9] = {{a->id, 8, nx.id},          {a->mate_id, 8, nx.mate_id}, {a->birth_time, 8, nx.birth},
+                             {a->age, 8, nx.age},        {a->last_birth, 8, nx.lastb}, {a->cell, 4, p->d_gfu},
+                             {a->num_babies, 4, nx.nbabies}, {a->life, 1, nx.life},   {a->gender, 1, nx.gender}};
+    size_t want = 0;
+    for (const Field &f : fields)
+        if (f.host) want += (f.size * (size_t)n + 63) / 64 * 64;
+    const bool genomes = a->genome && p->gwords;
+    const bool pinned = want + 64 <= kReadPinned;
+    int rc = read_buffer(p, pinned ? want + 64 : 64);
+    if (rc) return rc;
+    RankMap m{};
+    rc = rank_map(p, s.max_id[b], &m);
+    if (rc) return rc;
+    // the pool a compaction writes next takes the ordered genome rows
+    uint64_t *&rows = p->d_gpool[1 - p->gp_cur];
+    if (genomes && !rows && hipMalloc(&rows, (size_t)p->gcap * p->gwords * 8) != hipSuccess)
+        return fail(QHG_ERR_NOMEM, "second genome pool");
+    void *to[9];
+    size_t at = 64;
+    for (int k = 0; k < 9; k++) {
+        to[k] = !fields[k].host ? nullptr : pinned ? (void *)(p->d_read + at) : fields[k].dev;
+        if (fields[k].host) at += (fields[k].size * (size_t)n + 63) / 64 * 64;
+    }
+    volatile int32_t *bad = reinterpret_cast<volatile int32_t *>(p->h_read);
+    *bad = 0;
+    int32_t *d_bad = reinterpret_cast<int32_t *>(p->d_read);
+    const AgentBuf &d = p->buf[b];
+    uint32_t *slot_of = reinterpret_cast<uint32_t *>(p->d_gfs);
+    const dim3 blk(kRankBlock);
+    const int ga = grid_for(n, p->num_cu * 8);
+    hipStream_t st = p->stream;
+    hipLaunchKernelGGL(k_rank_clear, dim3(grid_for(m.words, p->num_cu * 8)), blk, 0, st, m);
+    hipLaunchKernelGGL(k_rank_mark, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n);
+    hipLaunchKernelGGL(k_rank_tiles, dim3(std::min(m.tiles, p->num_cu * 8)), blk, 0, st, m);
+    hipLaunchKernelGGL(k_rank_base, dim3(1), blk, 0, st, m);
+    hipLaunchKernelGGL(k_rank_slots, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n, slot_of, d_bad);
+    ReadOut o{(int64_t *)to[0], (int64_t *)to[1], (int32_t *)to[5], (int32_t *)to[6], (uint8_t *)to[7],
+              (uint8_t *)to[8], (double *)to[2],  (double *)to[3],  (double *)to[4]};
+    hipLaunchKernelGGL(k_read_agents, dim3(ga), blk, 0, st, m, d, (const OccCell *)p->d_occ[b], s.n_occ[b], p->ncells,
+                       (const uint32_t *)slot_of, n, o, d_bad);
+    if (genomes)
+        hipLaunchKernelGGL(k_read_genomes, dim3(grid_for(n * p->gwords, p->num_cu * 16)), blk, 0, st,
+                           (const int32_t *)d.ghandle, (const uint64_t *)p->d_gpool[p->gp_cur], s.gpool[b], p->gwords,
+                           (const uint32_t *)slot_of, n, rows, d_bad);
+    HIPCHK(hipGetLastError());
+    if (!pinned)
+        for (const Field &f : fields)
+            if (f.host)
+                HIPCHK(hipMemcpyAsync(const_cast<void *>(f.host), f.dev, f.size * (size_t)n, hipMemcpyDeviceToHost, st));
+    if (genomes)
+        HIPCHK(hipMemcpyAsync(a->genome, rows, (size_t)n * p->gwords * 8, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (*bad) return fail(QHG_ERR_STATE, "download: the agents, the cell list or the genome handles disagree");
+    if (pinned) {
+        at = 64;
+        for (const Field &f : fields) {
+            if (!f.host) continue;
+            std::memcpy(const_cast<void *>(f.host), p->h_read + at, f.size * (size_t)n);
+            at += (f.size * (size_t)n + 63) / 64 * 64;
+        }
+    }
+    return 0;
+}
+
+// Ids too large for the bitmap, or no device memory left for it: everything
+// is copied and ordered on the host.
+int read_agents_sorted(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
+    const int b = p->cur();
+    const int64_t n = s.n_alive[b];
+    const int64_t np = p->gwords ? s.gpool[b] : 0;
+    const AgentBuf &d = p->buf[b];
+    std::vector<int64_t> id(n), mate(n);
+    std::vector<int32_t> nbab(n), gh(n);
+    std::vector<OccCell> occ((size_t)std::max<int64_t>(0, s.n_occ[b]));
+    std::vector<uint8_t> life(n), gender(n);
+    std::vector<double> birth(n), age(n), lastb(n);
+    std::vector<uint64_t> pool;
+    hipStream_t st = p->stream;
+    if (!occ.empty())
+        HIPCHK(hipMemcpyAsync(occ.data(), p->d_occ[b], occ.size() * sizeof(OccCell), hipMemcpyDeviceToHost, st));
+    if (n > 0) {
+        HIPCHK(hipMemcpyAsync(id.data(), d.id, n * 8, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(mate.data(), d.mate_id, n * 8, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(nbab.data(), d.nbabies, n * 4, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(life.data(), d.life, n, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(gender.data(), d.gender, n, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(birth.data(), d.birth, n * 8, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(age.data(), d.age, n * 8, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(lastb.data(), d.lastb, n * 8, hipMemcpyDeviceToHost, st));
+        if (p->gwords && a->genome) {
+            HIPCHK(hipMemcpyAsync(gh.data(), d.ghandle, n * 4, hipMemcpyDeviceToHost, st));
+            pool.resize((size_t)np * p->gwords);
+            if (np > 0)
+                HIPCHK(hipMemcpyAsync(pool.data(), p->d_gpool[p->gp_cur], (size_t)np * p->gwords * 8,
+                                      hipMemcpyDeviceToHost, st));
+        }
+    }
+    HIPCHK(hipStreamSynchronize(st));
+    // every agent's cell from the occupied-cell list (cell, first slot, count)
+    std::vector<int32_t> cell(n, -1);
+    int64_t covered = 0;
+    for (const OccCell &e : occ) {
+        if (e.c < 0 || e.c >= p->ncells || (int64_t)e.s + e.n > n) return fail(QHG_ERR_STATE, "download: bad cell list");
+        for (uint32_t i = e.s; i < e.s + e.n; i++) cell[i] = e.c;
+        covered += e.n;
+    }
+    if (covered != n) return fail(QHG_ERR_STATE, "download: the cell list disagrees with the count");
+    std::vector<int64_t> order(n);
+    std::iota(order.begin(), order.end(), 0);
+    std::sort(order.begin(), order.end(), [&](int64_t x, int64_t y) { return id[x] < id[y]; });
+    std::vector<int64_t> sorted_ids(n);
+    for (int64_t k = 0; k < n; k++) sorted_ids[k] = id[order[k]];
+    for (int64_t k = 0; k < n; k++) {
+        const int64_t i = order[k];
+        if (a->id) a->id[k] = id[i];
+        if (a->cell) a->cell[k] = cell[i];
+        if (a->life) a->life[k] = life[i];
+        if (a->gender) a->gender[k] = gender[i];
+        if (a->birth_time) a->birth_time[k] = birth[i];
+        if (a->age) a->age[k] = age[i];
+        if (a->last_birth) a->last_birth[k] = lastb[i];
+        if (a->num_babies) a->num_babies[k] = nbab[i];
+        if (a->mate_id) {
+            // the partner's id while it lives, -1 once it has died
+            const int64_t m = mate[i];
+            a->mate_id[k] = (m >= 0) ? (std::binary_search(sorted_ids.begin(), sorted_ids.end(), m) ? m : -1) : m;
+        }
+        if (a->genome && p->gwords) {
+            const int64_t h = gh[i];
+            if (h < 0 || h >= np) return fail(QHG_ERR_STATE, "download: genome handle out of range");
+            std::memcpy(a->genome + (size_t)k * p->gwords, &pool[(size_t)h * p->gwords], (size_t)p->gwords * 8);
+        }
+    }
     return 0;
 }
 
@@ -1183,13 +1381,14 @@ int qhg_gpu_destroy(qhg_pop *p) {
     void *ptrs[] = {p->d_off[0], p->d_off[1], p->d_gpool[0], p->d_gpool[1], p->d_nbr, p->d_nn, p->d_in_e,
                     p->d_K, p->d_W, p->d_tmp, p->d_ice, p->d_coastal, p->d_cstay, p->d_cbirth, p->d_cin, p->d_carr, p->d_tact, p->d_tick, p->d_outk,
                     p->d_birth_off, p->d_bpos, p->d_rpos, p->d_tiles, p->d_tiles2, p->d_occ[0], p->d_occ[1],
-                    p->d_wave_part, p->d_scan_part, p->d_st, p->d_digest};
+                    p->d_wave_part, p->d_scan_part, p->d_st, p->d_digest, p->d_rank};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     for (int k = 0; k < 7; k++)
         if (p->d_env[k]) (void)hipFree(p->d_env[k]);
     for (auto &e : p->ev_pool) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     if (p->h_ring) (void)hipHostFree(p->h_ring);
+    if (p->h_read) (void)hipHostFree(p->h_read);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
     return 0;
@@ -1392,69 +1591,13 @@ int qhg_gpu_download_agents(qhg_pop *p, qhg_agents *a) {
     if (rc) return rc;
     const int b = p->cur();
     const int64_t n = s.n_alive[b];
-    const int64_t np = p->gwords ? s.gpool[b] : 0;
-    const AgentBuf &d = p->buf[b];
-    std::vector<int64_t> id(n), mate(n);
-    std::vector<int32_t> nbab(n), gh(n);
-    std::vector<OccCell> occ((size_t)std::max<int64_t>(0, s.n_occ[b]));
-    std::vector<uint8_t> life(n), gender(n);
-    std::vector<double> birth(n), age(n), lastb(n);
-    std::vector<uint64_t> pool;
-    hipStream_t st = p->stream;
-    if (!occ.empty())
-        HIPCHK(hipMemcpyAsync(occ.data(), p->d_occ[b], occ.size() * sizeof(OccCell), hipMemcpyDeviceToHost, st));
     if (n > 0) {
-        HIPCHK(hipMemcpyAsync(id.data(), d.id, n * 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(mate.data(), d.mate_id, n * 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(nbab.data(), d.nbabies, n * 4, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(life.data(), d.life, n, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(gender.data(), d.gender, n, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(birth.data(), d.birth, n * 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(age.data(), d.age, n * 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(lastb.data(), d.lastb, n * 8, hipMemcpyDeviceToHost, st));
-        if (p->gwords && a->genome) {
-            HIPCHK(hipMemcpyAsync(gh.data(), d.ghandle, n * 4, hipMemcpyDeviceToHost, st));
-            pool.resize((size_t)np * p->gwords);
-            if (np > 0)
-                HIPCHK(hipMemcpyAsync(pool.data(), p->d_gpool[p->gp_cur], (size_t)np * p->gwords * 8,
-                                      hipMemcpyDeviceToHost, st));
+        rc = s.max_id[b] < kRankIdLimit ? read_agents_ranked(p, s, a) : QHG_ERR_NOMEM;
+        if (rc == QHG_ERR_NOMEM) {
+            (void)hipGetLastError();   // a failed allocation's error is not the next launch's
+            rc = read_agents_sorted(p, s, a);
         }
-    }
-    HIPCHK(hipStreamSynchronize(st));
-    // every agent's cell from the occupied-cell list (cell, first slot, count)
-    std::vector<int32_t> cell(n, -1);
-    int64_t covered = 0;
-    for (const OccCell &e : occ) {
-        if (e.c < 0 || e.c >= p->ncells || (int64_t)e.s + e.n > n) return fail(QHG_ERR_STATE, "download: bad cell list");
-        for (uint32_t i = e.s; i < e.s + e.n; i++) cell[i] = e.c;
-        covered += e.n;
-    }
-    if (covered != n) return fail(QHG_ERR_STATE, "download: the cell list disagrees with the count");
-    std::vector<int64_t> order(n);
-    std::iota(order.begin(), order.end(), 0);
-    std::sort(order.begin(), order.end(), [&](int64_t x, int64_t y) { return id[x] < id[y]; });
-    std::vector<int64_t> sorted_ids(n);
-    for (int64_t k = 0; k < n; k++) sorted_ids[k] = id[order[k]];
-    for (int64_t k = 0; k < n; k++) {
-        const int64_t i = order[k];
-        if (a->id) a->id[k] = id[i];
-        if (a->cell) a->cell[k] = cell[i];
-        if (a->life) a->life[k] = life[i];
-        if (a->gender) a->gender[k] = gender[i];
-        if (a->birth_time) a->birth_time[k] = birth[i];
-        if (a->age) a->age[k] = age[i];
-        if (a->last_birth) a->last_birth[k] = lastb[i];
-        if (a->num_babies) a->num_babies[k] = nbab[i];
-        if (a->mate_id) {
-            // the partner's id while it lives, -1 once it has died
-            const int64_t m = mate[i];
-            a->mate_id[k] = (m >= 0) ? (std::binary_search(sorted_ids.begin(), sorted_ids.end(), m) ? m : -1) : m;
-        }
-        if (a->genome && p->gwords) {
-            const int64_t h = gh[i];
-            if (h < 0 || h >= np) return fail(QHG_ERR_STATE, "download: genome handle out of range");
-            std::memcpy(a->genome + (size_t)k * p->gwords, &pool[(size_t)h * p->gwords], (size_t)p->gwords * 8);
-        }
+        if (rc) return rc;
     }
     a->n = n;
     return 0;

@@ -1,0 +1,60 @@
+"""Reading agents back in id order: the live ids' bitmap at the edges of its
+words and tiles, and ids beyond it (ordered on the host instead)."""
+import numpy as np
+import pytest
+
+from qhg4_amd import abi, scenarios
+from qhg4_amd.grids import rect_grid
+
+pytestmark = pytest.mark.gpu
+
+TILE = 256 * 8 * 64   # ids per tile of the bitmap
+LIMIT = 1 << 31       # ids from here on are ordered on the host
+
+
+def _ids(kind, rng):
+    return {
+        "one": [0],
+        "one_high": [TILE],
+        "words": [0, 1, 62, 63, 64, 65, 127, 128],
+        "tiles": [TILE - 1, TILE, TILE + 1, 2 * TILE - 1, 2 * TILE, 300 * TILE + 5],
+        "dense": list(range(1, 4098)),
+        "sparse": sorted(set(rng.integers(0, 40 * TILE, 3001).tolist())),
+        "large": sorted(set(rng.integers(0, 1 << 22, 100000).tolist())),
+        "last_ranked": [3, LIMIT - 2, LIMIT - 1],
+        "past_limit": [3, LIMIT - 1, LIMIT, (1 << 40) + 7],
+    }[kind]
+
+
+@pytest.mark.parametrize("gwords", [0, 6])
+@pytest.mark.parametrize("kind", ["one", "one_high", "words", "tiles", "dense", "sparse", "large", "last_ranked",
+                                  "past_limit"])
+def test_agents_come_back_in_id_order(kind, gwords):
+    from qhg4_amd.population import GpuPopulation
+    rng = np.random.default_rng(11)
+    ids = np.array(_ids(kind, rng), dtype=np.int64)
+    n = len(ids)
+    grid = rect_grid(37, 29)
+    order = rng.permutation(n)
+    agents = {
+        "id": ids[order], "cell": rng.integers(0, grid["num_cells"], n).astype(np.int32),
+        "life": rng.choice([1, 5], n).astype(np.uint8), "gender": rng.integers(0, 2, n).astype(np.uint8),
+        "birth_time": rng.uniform(-40, 0, n), "age": rng.uniform(0, 40, n), "last_birth": rng.uniform(-9, 0, n),
+        "num_babies": rng.integers(0, 9, n).astype(np.int32), "mate_id": np.full(n, -3, dtype=np.int64),
+    }
+    actions = [(abi.ACT_GETOLD, 1)]
+    kw = {}
+    if gwords:
+        actions.append((abi.ACT_GENETICS, 2))
+        kw = dict(gen_genome_size=32 * gwords // 2, gen_num_crossover=1, gen_mutation_rate=0.0)
+        agents["genome"] = rng.integers(0, 1 << 62, n * gwords, dtype=np.int64).astype(np.uint64)
+    pop = GpuPopulation(grid, {}, scenarios.make_params(1, actions, **kw), agents, capacity=1024)
+    pop.preLoop(0.0)
+    back = np.argsort(agents["id"])
+    for _ in range(2):
+        got = pop.agents()
+        for k in abi.AGENT_FIELDS:
+            assert np.array_equal(got[k], agents[k][back]), k
+        if gwords:
+            assert np.array_equal(got["genome"], agents["genome"].reshape(n, gwords)[back])
+    pop.close()
