@@ -137,14 +137,15 @@ __global__ void __launch_bounds__(kBlock) k_eval_combine(Ctx x, const double *tm
 // altitude < 0 or ice is removed before the next step.  The buffer is cell
 // sorted, so whole cells go.  Pass 1 (one block) lists the kept occupied
 // cells of buffer b, in order, in occ_dst with dense segment starts, their
-// old starts in src_s, and the resulting counts in the other parity's
+// groups, their old starts in src_s, and the resulting counts in the other parity's
 // status; pass 2 moves the kept agents into the other buffer, which then
 // takes the current buffer's role.
 constexpr int kKillBlock = 1024;
 
 __global__ void __launch_bounds__(kKillBlock) k_env_kill(const OccCell *occ, int64_t nocc, const double *alt,
                                                          const uint8_t *ice, OccCell *occ_dst, uint32_t *src_s,
-                                                         DevStatus *st, int b) {
+                                                         GroupDesc *grp, int64_t grp_cap, uint32_t gdiv, DevStatus *st,
+                                                         int b) {
     constexpr int kWaves = kKillBlock / kWave;
     __shared__ uint32_t wkeep[kWaves], wslots[kWaves];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -181,6 +182,7 @@ __global__ void __launch_bounds__(kKillBlock) k_env_kill(const OccCell *occ, int
         if (keep) {
             const int64_t o = out + pre + below;
             occ_dst[o] = OccCell{e.c, slots + spre + incl - v, e.n, 0u};
+            group_ends(grp, grp_cap, gdiv, (uint32_t)o, slots + spre + incl - v, e.n);
             src_s[o] = e.s;
         }
         out += total;
@@ -190,6 +192,8 @@ __global__ void __launch_bounds__(kKillBlock) k_env_kill(const OccCell *occ, int
     if (threadIdx.x == 0) {
         const int nb = 1 - b;
         st->n_occ[nb] = out;
+        st->n_grp[nb] = group_close(grp, grp_cap, gdiv, (uint32_t)out, slots);
+        st->big[nb] = st->big[b];
         st->n_alive[nb] = slots;
         st->max_id[nb] = st->max_id[b];
         st->gpool[nb] = st->gpool[b];

@@ -22,11 +22,11 @@
                                        r 1 + stayer count w 4                               */
 #define QHG_B_ACT_OCC_PER_CONN  16  /* neighbour index r 4 + run slot r 4 + weight r 8     */
 #define QHG_B_ACT_OCC_W_EXTRA    8  /*   ... the extra weight of the row (conn+1 weights)   */
-#define QHG_B_ACT_LIVE_BASE     10  /* id r 8 (Philox key) + life r 1 + outcome w 1          */
-#define QHG_B_ACT_LIVE_PAIR     10  /* gender r 1 + life r 1 (pairing pass) + partner id w 8 */
-#define QHG_B_ACT_LIVE_GETOLD   16  /* birth time r 8 + age w 8                              */
-#define QHG_B_ACT_LIVE_FERT     10  /* gender r 1 + last birth r 8 + life w 1                */
-#define QHG_B_ACT_BIRTH         12  /* mother's NumBabies r/w 8 + father slot w 4            */
+#define QHG_B_ACT_LIVE_BASE     17  /* id r 8 (Philox key) + life r 1 + outcome word w 8     */
+#define QHG_B_ACT_LIVE_PAIR      5  /* gender r 1 + partner slot w 4                         */
+#define QHG_B_ACT_LIVE_GETOLD    8  /* birth time r 8                                        */
+#define QHG_B_ACT_LIVE_FERT      9  /* gender r 1 + last birth r 8                           */
+#define QHG_B_ACT_BIRTH          8  /* mother's cell and rank w 8                            */
 
 /* k_cell_scan (next counts -> segment and birth offsets).  Counted per
    occupied cell only: the scan also reads the empty cells of tiles that
@@ -41,19 +41,19 @@
 #define QHG_B_SCAN_SUMS_OCC     12  /* stayers r 4 + births r 4 + arrivals r 4              */
 
 /* k_cell_scatter (performMoves + createAgentAtIndex + makeOffspring) */
-#define QHG_B_SCAT_OCC          20  /* occupied-cell entry r 16 + next offset r 4           */
-#define QHG_B_SCAT_LIVE          1  /* outcome byte r of every agent at step start           */
-#define QHG_B_SCAT_SURVIVOR     93  /* record r 46 + w 46 (id, partner, life, gender, birth,
-                                       age, last birth, NumBabies) + outcome r 1             */
+#define QHG_B_SCAT_OCC           4  /* next offset r 4                                      */
+#define QHG_B_SCAT_LIVE          8  /* outcome word r of every agent at step start          */
+#define QHG_B_SCAT_SURVIVOR     79  /* r 33 (id, gender, birth, last birth, NumBabies,
+                                       partner slot) + w 46 (those, partner id, life, age)   */
 #define QHG_B_SCAT_SURVIVOR_GEN  8  /* genome handle r 4 + w 4                               */
-#define QHG_B_SCAT_BIRTH        54  /* newborn record w 46 + birth offset r 4 + father r 4   */
+#define QHG_B_SCAT_BIRTH        62  /* newborn record w 46 + mother's rank r 8 + position
+                                       and birth offset r 8                                  */
 #define QHG_B_SCAT_BIRTH_GEN    12  /* handle w 4 + birth record w 8                         */
 
 /* k_assort_pair (AssortativePairHamming), per live agent and per FERTILE
    agent of a cell holding both sexes; each couple's genome words are read
    through the caches, counted once per agent (a lower bound) */
-#define QHG_B_ASSORT_LIVE       22  /* life r 1 + gender r 1 + id r 8 + partner slot w 4
-                                       + mate id w 8                                         */
+#define QHG_B_ASSORT_LIVE       14  /* life r 1 + gender r 1 + id r 8 + partner slot w 4    */
 #define QHG_B_ASSORT_FERTILE     4  /* genome handle r 4, + 2 x D x 8 genome words r          */
 
 /* k_genome (Genetics::makeOffspring), per birth */

@@ -8,22 +8,23 @@
 // results do not depend on it.  A step is three launches (four with
 // Genetics), none with global atomics on agent data:
 //
-//   k_cell_act      one wave per occupied cell: RandomPair::initialize /
-//                   findMates on the cell's segment (QHG4/actions/
-//                   RandomPair.cpp:107-279), then every Action<T>::execute of
-//                   the step fused in priority order (QHG4/core/
-//                   SPopulation.cpp:554-577).  Writes each agent's outcome
-//                   (dead / stays / moves to neighbour slot d / gave birth)
-//                   and per cell the counts of stayers, movers per slot and
-//                   births.
+//   k_cell_act      one block per group of consecutive occupied cells:
+//                   RandomPair::initialize / findMates on the cells' segments
+//                   (QHG4/actions/RandomPair.cpp:107-279), then every
+//                   Action<T>::execute of the step fused in priority order
+//                   (QHG4/core/SPopulation.cpp:554-577).  Writes each agent's
+//                   outcome word (dead, or the run it lands in and its place
+//                   there; gave birth) and per cell the counts of stayers,
+//                   movers per slot and births.
 //   k_cell_scan     per cell: next count = stayers + arrivals + births; one
 //                   decoupled look-back scan gives the next segment offsets,
-//                   the birth offsets (new ids), and the absolute position of
-//                   every incoming (source cell, slot) run
-//                   (updateNumAgentsPerCell, SPopulation.cpp:509-536).
-//   k_cell_scatter  one wave per occupied source cell: stayers and movers
-//                   pushed to their next positions, newborns of the cell's
-//                   mothers appended in mother-id order (performMoves,
+//                   the birth offsets (new ids), the absolute position of
+//                   every incoming (source cell, slot) run and the next
+//                   step's groups (updateNumAgentsPerCell,
+//                   SPopulation.cpp:509-536).
+//   k_cell_scatter  one thread per agent: its record to its run's position
+//                   plus its place, a mother's newborn after the arrivals of
+//                   its cell in mother-id order (performMoves,
 //                   recycleDeadSpaceNew, createAgentAtIndex,
 //                   makePopSpecificOffspring; SPopulation.cpp:596-918).
 //   k_genome        one thread per birth: Genetics::makeOffspring
@@ -45,12 +46,17 @@
 namespace qhg {
 
 constexpr int kWave = 64;
-constexpr int kCellBlock = 64;        // per-cell kernels: one wave per block
-constexpr int kLdsCell = 256;         // cells up to this size keep their lists in LDS,
-                                      // larger ones in segment-indexed global scratch
-constexpr int kGroupSlots = 256;      // agents of one packed group of cells
-constexpr int kGroupCells = 16;       // cells of one packed group
-constexpr int kGroupCellMax = 64;     // largest cell the packed pairing takes
+constexpr int kActBlock = 256;        // k_cell_act: four waves per group of cells
+constexpr int kActWaves = kActBlock / kWave;
+constexpr int kScatterBlock = 256;    // k_cell_scatter: one thread per agent
+// Groups: the occupied cells are laid on a line, each as long as its agents
+// plus kGroupPad, and cut into pieces of some length; a group holds the
+// cells that begin in one piece.  The pad bounds the cells of a group.
+constexpr int kGroupPad = 3;
+constexpr int kGroupPieceMin = 48, kGroupPieceMax = 252;
+constexpr int kGroupCells = 64;       // cells of one group: 253 / (1 + 3), up
+constexpr int kGroupSlots = kActBlock;   // agents a block takes at once; larger cells go
+                                      // to one wave each, with global scratch lists
 constexpr int kMaxIn = 8;             // incoming neighbour slots per cell
 constexpr int kScanBlock = 256;       // k_cell_scan threads per block
 constexpr int kScanPer = 1;           // cells per k_cell_scan thread
@@ -65,18 +71,28 @@ constexpr int32_t kErrGather = 8;     // an internal count disagreed
 constexpr uint32_t kLookbackSpins = 1u << 22;
 constexpr int kParts = 3;             // per-block partial sums of k_cell_act
 
-// outcome byte of an agent in a step
-constexpr uint8_t kDecBirth = 0x80;   // registered a birth
-constexpr uint8_t kDecDead = 0x40;    // died
-constexpr uint8_t kDecDirMask = 0x07; // 0 stays, d+1 moves to neighbour slot d,
-constexpr uint8_t kDecNav = 0x07;     //   kDecNav moves along a Navigate edge
-constexpr int kNavDir = kDecNav - 1;  // the move direction of a navigating mover
+// Outcome word of an agent in a step: where it goes (an index into the table
+// of its kind and its place in that run) and what happened to it.
+constexpr uint32_t kDecDead = 0;      // died
+constexpr uint32_t kDecStay = 1;      // stays: run of cell idx (off_nxt)
+constexpr uint32_t kDecMove = 2;      // moves: run of (cell, slot) idx (rpos)
+constexpr uint32_t kDecNav = 3;       // moves along Navigate edge idx (nav.rpos)
+constexpr int kDecRankAt = 32;        // 26 bits: place in the run
+constexpr uint32_t kDecRankMask = (1u << 26) - 1u;
+constexpr int kDecKindAt = 58;
+constexpr uint64_t kDecBirth = 1ull << 60;     // registered a birth
+constexpr uint64_t kDecFertile = 1ull << 61;   // life state FERTILE (else ALIVE), where Fertility runs
+constexpr uint64_t kDecCounted = 1ull << 62;   // the birth is in NumBabies already (k_act_commit)
+constexpr uint64_t kDecAged = 1ull << 63;      // the age was set
+constexpr int kNavDir = 6;            // the move direction of a navigating mover
 
 struct DevStatus {
     int64_t n_alive[2];      // live agents at the start of a step of this parity
     int64_t n_occ[2];        // occupied cells at the start of a step of this parity
     int64_t max_id[2];
     int64_t gpool[2];        // genome pool high-water mark
+    int64_t n_grp[2];        // groups of occupied cells at the start of a step of this parity
+    int64_t big[2];          // ... and whether a cell may hold more agents than a block takes
     int64_t step;            // steps completed
     double t;
     int64_t births_last, deaths_last, moves_last;
@@ -94,6 +110,13 @@ struct OccCell {
     uint32_t pad;
 };
 
+// where a group begins: index of its first occupied cell, first slot (the
+// next entry ends it)
+struct GroupDesc {
+    uint32_t first;
+    uint32_t s;
+};
+
 struct AgentBuf {
     int64_t *id;
     int64_t *mate_id;        // partner id of this step's pairing, -3 when unpaired
@@ -104,6 +127,7 @@ struct AgentBuf {
     double *lastb;
     int32_t *nbabies;
     int32_t *ghandle;        // genome pool slot (Genetics only)
+    GroupDesc *grp;          // the groups of the occupied cells
 };
 
 // Navigate's tables on the device (n == 0: no Navigate, or no edge).  Every
@@ -121,7 +145,6 @@ struct NavDev {
     const int32_t *in_e;      // ... their indices, increasing
     uint32_t *cnt;            // n: movers per edge this step (zero outside a step)
     uint32_t *rpos;           // n: next-buffer slot of each edge's run
-    uint64_t *sel;            // per slot: edge | rank << 32 of a navigating mover
 };
 
 struct Ctx {
@@ -139,10 +162,12 @@ struct Ctx {
     const uint8_t *ice;
     const int32_t *in_e;      // ncells * in_w: incoming runs src*conn+slot, -1 padded
     int32_t in_w;             // <= kMaxIn
-    uint8_t *dec;             // per slot of the current buffer: outcome byte
-    int32_t *bfather;         // per slot: father slot of a registered birth (Genetics)
+    int64_t grp_cap;          // entries of a buffer's group list
+    uint64_t *dec;            // per slot of the current buffer: outcome word
+    uint64_t *brank;          // per mother's slot: cell | rank among the cell's births << 32
     int32_t *brec;            // per birth: mother slot, father slot (Genetics)
-    int32_t *gfu, *gmu, *gfs, *gms, *gmate;   // per-slot list scratch of large cells
+    int32_t *gmate;           // per slot: the partner's slot, -1 unpaired
+    int32_t *gfu, *gmu, *gfs, *gms;           // per-slot list scratch of large cells
     int64_t *gfid, *gmid;
     uint8_t *gflag;
     uint32_t *gprot;          // AssortativePair: kProtBudget digests (4 words each) per slot
@@ -177,31 +202,48 @@ struct StepArgs {
     uint32_t step;            // step index (Philox counter word)
     uint32_t parity;          // step & 1: which status halves are current
     double t;                 // time of the step
-    int32_t gcells;           // occupied cells per wave group (1..kGroupCells)
+    uint32_t gdiv;            // k_cell_scan cuts the next step's groups: 2^32 / piece length
+    int32_t mates;            // gmate holds the step's partners (else mate_id carries over)
+    int32_t sets_age;         // the program sets every survivor's age (t - birth)
+    int32_t sets_life;        // the program sets every survivor's life state
     int32_t dense;            // k_cell_scan reads every cell's incoming runs (many cells occupied)
 };
 
 constexpr double kPi = 3.141592653589793;   // Q_PI, QHG4/utils/qhg_consts.h:71
 
-struct Prog {
+// what the agents' part of a step reads of the program, in one piece
+struct ActConst {
+    uint64_t opword;          // the actions with an execute, in order, 4 bits each
     int32_t nops;
-    int32_t ops[QHG_MAX_ACTIONS];
-    uint64_t opword;          // ops packed 4 bits each (op q in bits 4q..4q+3)
-    int32_t load_age;         // Fertility runs before GetOld (reads the stored age)
-    int32_t has_pair;
-    int32_t need_gender, need_birth, need_lastb, need_act0, need_act1;
+    uint32_t flags;           // kAct...
     double fert_min, fert_max, fert_inter;
-    double b0, d0, theta, Kconst;
+    double b0, d0;
+    double b1, d1;            // theta - b0, theta - d0
     double rmove_p, wmove_p;
+    double Kconst;
+};
+
+constexpr uint32_t kActPair = 1u;        // RandomPair is scheduled
+constexpr uint32_t kActBirth = 2u;       // fields the program reads
+constexpr uint32_t kActLastb = 4u;
+constexpr uint32_t kActAge = 8u;         // Fertility runs before GetOld (reads the stored age)
+constexpr uint32_t kActDraw0 = 16u;      // draws 0-3, 4-7
+constexpr uint32_t kActDraw1 = 32u;
+constexpr uint32_t kActVarK = 64u;       // VerhulstVarK, Verhulst
+constexpr uint32_t kActVerh = 128u;
+
+struct Prog {
+    ActConst k;
     double oad_max, oad_unc;                // OldAgeDeath
     double atan_max, atan_slope, atan_scale;  // ATanDeath (scale from ATanDeath::preLoop)
-    int32_t gen_size, gen_cross, nbino, pad;
+    double nav_bridge_p;      // Navigate_bridge_prob
+    int32_t sets_age, sets_life;              // as StepArgs
+    int32_t gen_size, gen_cross, nbino;
     // AssortativePairHamming: mates come from k_assort_pair (x.gmate)
-    int32_t has_assort, assort_permute;
+    int32_t assort_permute;
     int32_t assort_words;     // numNucs2Blocks(numBlocks): words per strand position compared
     float assort_cutoff;
     int32_t assort_prot;      // AssortativePair: matches counted over protein digests
-    double nav_bridge_p;      // Navigate_bridge_prob
     double bino[QHG_MAX_BINO];
 };
 
@@ -218,6 +260,18 @@ __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, int k) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, k);
 }
 
+// values every lane holds alike (ballot and shuffle results), as such
+__device__ __forceinline__ int uniform_i32(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+template <typename T>
+__device__ __forceinline__ T *uniform_ptr(T *p) {
+    return (T *)(uintptr_t)uniform_i64((int64_t)(uintptr_t)p);
+}
+
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -225,15 +279,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
         v = (o > v) ? o : v;
     }
     return v;
-}
-
-// index of the group cell holding group position q; eb holds the cells'
-// first positions in lanes 0..ng-1 (increasing)
-__device__ __forceinline__ int group_cell_of(uint32_t q, uint32_t eb, int ng) {
-    int k = 0;
-    for (int kk = 1; kk < ng; kk++)
-        if (q >= readlane_u32(eb, kk)) k = kk;
-    return k;
 }
 
 // ---------------------------------------------------------------------------
@@ -394,10 +439,14 @@ struct ActItem {
 };
 
 struct CellView {             // the per-cell values every agent of the cell reads
-    uint32_t N;               // live agents at step start (getNumAgents)
-    double K;
+    double rat;               // N / K(cell), N the live agents at step start; -1 where K <= 0
+    double ratc;              // N / Verhulst_K
     int nn;
 };
+
+// LinearBirth / LinearDeath divide the cell's count by its capacity: once per
+// cell, not per agent
+__device__ __forceinline__ double vark_ratio(uint32_t N, double K) { return (K <= 0) ? -1.0 : (double)N / K; }
 
 // Every action of the program in priority order (compute only; the caller
 // loaded every field).  A dead agent stops.  Moves are only registered here
@@ -405,14 +454,17 @@ struct CellView {             // the per-cell values every agent of the cell rea
 // performMoves applies them after all actions.
 // kRare: the program may hold OldAgeDeath or ATanDeath; kNav: Navigate
 // (separate instantiations keep their code out of the common kernel)
-template <bool kRare, bool kNav = false, typename CtxT, typename ProgT>
-__device__ __forceinline__ void act_program(const CtxT &x, const ProgT &p, const StepArgs &sa, const CellView &cv,
-                                            ActItem &a, uint32_t &deaths) {
-    const double t = sa.t;
-    if (p.need_act0) draw4(x.seed, sa.step, QHG_STREAM_ACT, (uint64_t)a.id, 0, &a.u[0]);
-    if (p.need_act1) draw4(x.seed, sa.step, QHG_STREAM_ACT, (uint64_t)a.id, 1, &a.u[4]);
-    uint64_t word = p.opword;
-    for (int q = 0; q < p.nops; q++, word >>= 4) {
+// The agent's draws of the step: words 0..7 of its QHG_STREAM_ACT counter.
+__device__ __forceinline__ void act_draws(uint64_t seed, uint32_t flags, uint32_t step, ActItem &a) {
+    if (flags & kActDraw0) draw4(seed, step, QHG_STREAM_ACT, (uint64_t)a.id, 0, &a.u[0]);
+    if (flags & kActDraw1) draw4(seed, step, QHG_STREAM_ACT, (uint64_t)a.id, 1, &a.u[4]);
+}
+
+template <bool kRare, bool kNav = false, typename ProgT>
+__device__ __forceinline__ void act_program(const ProgT &p, const ActConst &k, double t, const CellView &cv, ActItem &a,
+                                            uint32_t &deaths) {
+    uint64_t word = k.opword;
+    for (int q = 0; q < k.nops; q++, word >>= 4) {
         const int op = (int)(word & 15u);
         if (op == QHG_ACT_GETOLD) {
             // GetOld::execute, QHG4/actions/GetOld.cpp:37-48
@@ -421,23 +473,18 @@ __device__ __forceinline__ void act_program(const CtxT &x, const ProgT &p, const
         } else if (op == QHG_ACT_FERTILITY) {
             // Fertility::execute, QHG4/actions/Fertility.cpp:49-74
             if (a.g == 0) {
-                a.life = (a.age > p.fert_min && a.age < p.fert_max && (t - a.lastb) > p.fert_inter)
+                a.life = (a.age > k.fert_min && a.age < k.fert_max && (t - a.lastb) > k.fert_inter)
                              ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
             } else {
-                a.life = (a.age > p.fert_min) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
+                a.life = (a.age > k.fert_min) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
             }
         } else if (op == QHG_ACT_VERHULST || op == QHG_ACT_VERHULSTVARK) {
             // LinearBirth::initialize/execute then LinearDeath (Verhulst.cpp:101-115;
             // LinearBirth.cpp:90-168; LinearDeath.cpp:92-153)
-            const double N = (double)cv.N;
-            double b, d;
-            if (op == QHG_ACT_VERHULST) {
-                b = p.b0 + (p.theta - p.b0) * (N / p.Kconst);
-                d = p.d0 + (p.theta - p.d0) * (N / p.Kconst);
-            } else {
-                b = (cv.K <= 0) ? 0.0 : p.b0 + (p.theta - p.b0) * (N / cv.K);
-                d = (cv.K <= 0) ? 1.0 : p.d0 + (p.theta - p.d0) * (N / cv.K);
-            }
+            const double rat = (op == QHG_ACT_VERHULST) ? cv.ratc : cv.rat;
+            const bool none = op == QHG_ACT_VERHULSTVARK && rat == -1.0;
+            const double b = none ? 0.0 : k.b0 + k.b1 * rat;
+            const double d = none ? 1.0 : k.d0 + k.d1 * rat;
             if (b > 0) {
                 if (a.g == 0 && a.mate >= 0) {
                     if (wrandd(a.u[QHG_ACTW_LBIRTH]) < b) a.bflag = 1;
@@ -455,7 +502,7 @@ __device__ __forceinline__ void act_program(const CtxT &x, const ProgT &p, const
             const bool rm = op == QHG_ACT_RANDOMMOVE;
             const uint32_t go = rm ? a.u[QHG_ACTW_RMOVE_GO] : a.u[QHG_ACTW_WMOVE_GO];
             const uint32_t dir = rm ? a.u[QHG_ACTW_RMOVE_DIR] : a.u[QHG_ACTW_WMOVE_DIR];
-            if (wrandd(go) < (rm ? p.rmove_p : p.wmove_p)) {
+            if (wrandd(go) < (rm ? k.rmove_p : k.wmove_p)) {
                 if (a.npend == 0) { a.pk0 = op; a.pu0 = dir; a.npend = 1; }
                 else if (a.npend == 1) { a.pk1 = op; a.pu1 = dir; a.npend = 2; }
             }
@@ -477,23 +524,22 @@ __device__ __forceinline__ void act_program(const CtxT &x, const ProgT &p, const
             const double pd = 0.5 + p.atan_scale * det_atan(p.atan_slope * (a.age - p.atan_max)) / kPi;
             if (wrandd(a.u[QHG_ACTW_ATANDEATH]) < pd) { a.life = 0; deaths++; break; }
         }
-        // RandomPair, MultiEvaluator, NPPCapacity, Genetics: no execute
     }
 }
 
 // Neighbour slot a registered move lands on, or -1 when the agent stays
-// (slot 0, a -1 hole, or ice for WeightedMove).  w: the cell's cumulative
-// weight row, nbr: its neighbour row (registers, compile-time indices only).
-template <typename CtxT>
-__device__ __forceinline__ int move_dir(const CtxT &x, int kind, uint32_t u, int nn, const double (&w)[7],
-                                        const int32_t (&nbr)[6]) {
+// (slot 0, a -1 hole, or ice for WeightedMove).  W(q): the cell's cumulative
+// weights, NB(d): its neighbours.
+template <typename WF, typename NF>
+__device__ __forceinline__ int move_dir(const uint8_t *ice, int kind, uint32_t u, int nn, int R, WF W, NF NB) {
     int idx = -1;
     if (kind == QHG_ACT_RANDOMMOVE) {
         idx = (int)(wrandd(u) * (nn + 1));
     } else {
-        double wl = w[0];
+        double w[7];
 #pragma unroll
-        for (int q = 1; q < 7; q++) if (q == nn) wl = w[q];
+        for (int q = 0; q < 7; q++) w[q] = W(q < R ? q : 0);
+        const double wl = W(nn);
         if (w[0] == wl) {
             idx = (int)wrandi(0, (uint32_t)nn + 1, 1, u);
         } else {
@@ -504,12 +550,10 @@ __device__ __forceinline__ int move_dir(const CtxT &x, int kind, uint32_t u, int
             }
         }
     }
-    if (idx <= 0) return -1;
-    int32_t nb = -1;
-#pragma unroll
-    for (int q = 0; q < 6; q++) if (q == idx - 1) nb = nbr[q];
+    if (idx <= 0 || idx >= R) return -1;
+    const int32_t nb = NB(idx - 1);
     if (nb < 0) return -1;
-    if (kind == QHG_ACT_WEIGHTEDMOVE && x.ice != nullptr && x.ice[nb]) return -1;
+    if (kind == QHG_ACT_WEIGHTEDMOVE && ice != nullptr && ice[nb]) return -1;
     return idx - 1;
 }
 
@@ -558,48 +602,34 @@ __device__ void nav_execute(const CtxT &x, const ProgT &p, const StepArgs &sa, i
 // last one winning (performMoves applies them in order,
 // QHG4/core/SPopulation.cpp:1058-1092).  Navigate takes its place in the
 // program and acts only when no move was registered before it
-// (LIFE_STATE_MOVING, Navigate.cpp:191).  w, nbr: the cell's weight and
-// neighbour rows; ne0, ne1: its Navigate edges.
-template <bool kNav, typename CtxT, typename ProgT>
+// (LIFE_STATE_MOVING, Navigate.cpp:191).  ne0, ne1: the cell's Navigate edges.
+template <bool kNav, typename CtxT, typename ProgT, typename WF, typename NF>
 __device__ __forceinline__ void resolve_moves(const CtxT &x, const ProgT &p, const StepArgs &sa, const ActItem &a,
-                                              int32_t c, int32_t ne0, int32_t ne1, int nn, const double (&w)[7],
-                                              const int32_t (&nbr)[6], int &dir, int32_t &nave, uint32_t &moves) {
-    if constexpr (!kNav) {
-        int d = move_dir(x, a.pk0, a.pu0, nn, w, nbr);
-        if (d >= 0) { dir = d; moves++; }
-        if (a.npend > 1) {
-            d = move_dir(x, a.pk1, a.pu1, nn, w, nbr);
-            if (d >= 0) { dir = d; moves++; }
-        }
-    } else {
-        // the neighbour moves' directions first (each depends on its own
-        // draw only), so the weight and neighbour rows are no longer live
-        // across Navigate's draws; then the registrations in program order,
-        // with one copy of Navigate's code, not one per place it can take
-        const int d0 = (a.npend > 0) ? move_dir(x, a.pk0, a.pu0, nn, w, nbr) : -1;
-        const int d1 = (a.npend > 1) ? move_dir(x, a.pk1, a.pu1, nn, w, nbr) : -1;
+                                              const uint8_t *ice, int32_t c, int32_t ne0, int32_t ne1, int nn, int R,
+                                              WF W, NF NB, int &dir, int32_t &nave, uint32_t &moves) {
+    // one copy of the code for every registration (a second one is rare)
 #pragma unroll 1
-        for (int q = 0; q <= a.npend; q++) {
-            if (a.navq == q + 1 && dir < 0) nav_execute(x, p, sa, a.id, c, ne0, ne1, dir, nave, moves);
-            const int d = (q == 0) ? d0 : d1;
-            if (q < a.npend && d >= 0) { dir = d; moves++; }
+    for (int q = 0; q < a.npend + (kNav ? 1 : 0); q++) {
+        if (kNav && a.navq == q + 1 && dir < 0) nav_execute(x, p, sa, a.id, c, ne0, ne1, dir, nave, moves);
+        if (!kNav || q < a.npend) {
+            const int d = move_dir(ice, q == 0 ? a.pk0 : a.pk1, q == 0 ? a.pu0 : a.pu1, nn, R, W, NB);
+            if (d >= 0) {
+                dir = d;
+                moves++;
+            }
         }
     }
 }
 
-// Places one chunk's navigating movers in their edges' runs (called by all
-// lanes).  One wave owns every edge of its cells and meets a cell's agents
-// in slot order, chunk by chunk, so the movers of an edge rank in slot
-// order: after those of earlier chunks (the edge's count so far), then in
-// lane order.  Each mover's edge and rank go to nav.sel for k_cell_scatter;
-// the edge's count (nav.cnt, read by k_cell_scan) and the target cell's
-// arrivals grow by the chunk's movers.
+// Places one wave's navigating movers in their edges' runs (called by all
+// lanes) and returns each one's place.  The edge's count (nav.cnt, read by
+// k_cell_scan) and the target cell's arrivals grow by the wave's movers.
 template <typename CtxT>
-__device__ __forceinline__ void nav_movers(const CtxT &x, bool mine, int32_t nave, uint32_t slot) {
+__device__ __forceinline__ uint32_t nav_movers(const CtxT &x, bool mine, int32_t nave) {
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt();
     uint64_t left = __ballot(mine);
-    if (!left) return;
+    if (!left) return 0u;
     // the movers sharing an edge, each edge led by its first lane: the
     // leaders then take their edges' counts in one atomic instruction (one
     // round trip for the chunk, not one per edge)
@@ -624,13 +654,13 @@ __device__ __forceinline__ void nav_movers(const CtxT &x, bool mine, int32_t nav
         x.tact[d / kCellTile] = 1u;
     }
     base = (uint32_t)__shfl((int)base, leader, 64);
-    if (mine) x.nav.sel[slot] = (uint64_t)(uint32_t)nave | ((uint64_t)(base + rank) << 32);
+    return base + rank;
 }
 
 // ---------------------------------------------------------------------------
-// k_cell_act: pairing + fused actions, one wave per occupied cell
+// k_cell_act: pairing + fused actions, one block per group of cells
 // ---------------------------------------------------------------------------
-struct PairLists {            // per-cell lists, in LDS or in global scratch
+struct PairLists {            // per-cell lists
     int32_t *fu, *mu;         // local indices of FERTILE females / males, slot order
     int64_t *fid, *mid;       // their ids
     int32_t *fs, *ms;         // id order: positions into fu/mu
@@ -640,7 +670,7 @@ struct PairLists {            // per-cell lists, in LDS or in global scratch
 
 // rank of each entry of ids[0..n) among them (ids are distinct) -> ord[rank]
 __device__ __forceinline__ void id_order(const int64_t *ids, int32_t n, int32_t *ord) {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     for (int32_t j = lane; j < n; j += kWave) {
         const int64_t my = ids[j];
         int32_t r = 0;
@@ -649,23 +679,57 @@ __device__ __forceinline__ void id_order(const int64_t *ids, int32_t n, int32_t 
     }
 }
 
-template <bool kRare, bool kAssort = false, bool kNav = false, typename CtxT, typename ProgT>
-__device__ __forceinline__ void cell_act(const CtxT &x, const ProgT &p, const StepArgs &sa, int32_t c, uint32_t s,
-                                         int32_t n, const PairLists &L, uint32_t &my_deaths, uint32_t &my_moves,
-                                         uint32_t &my_fert) {
-    const int lane = threadIdx.x;
+__device__ __forceinline__ uint64_t dec_word(const ActItem &a, uint32_t kind, uint32_t idx, uint32_t rank) {
+    return (uint64_t)idx | ((uint64_t)(rank & kDecRankMask) << kDecRankAt) | ((uint64_t)kind << kDecKindAt) |
+           (a.bflag ? kDecBirth : 0ull) | (a.life == QHG_LIFE_FERTILE ? kDecFertile : 0ull) |
+           (a.age_dirty ? kDecAged : 0ull);
+}
+
+__device__ __forceinline__ void act_item_init(ActItem &a) {
+    a.life = 0;
+    a.g = 2;
+    a.id = 0;
+    a.birth = 0;
+    a.lastb = 0;
+    a.age = 0;
+    a.mate = -1;
+    a.age_dirty = false;
+    a.bflag = 0;
+    a.npend = 0;
+    a.navq = 0;
+    a.pk0 = a.pk1 = 0;
+    a.pu0 = a.pu1 = 0;
+}
+
+// The kernel's constant arguments: kernel arguments or a batch member's
+// descriptor, both read through the constant address space.
+typedef __attribute__((address_space(4))) const Ctx ConstCtx;
+typedef __attribute__((address_space(4))) const Prog ConstProg;
+
+// A cell with more agents than a block takes, by one wave, its lists in global
+// scratch (in the cell's own slot range, so cells never overlap).
+template <bool kRare, bool kAssort, bool kNav>
+__device__ __forceinline__ void cell_act(ConstCtx &x, ConstProg &p, uint32_t step, double t, int32_t c, uint32_t s,
+                                         int32_t n, uint32_t &my_deaths, uint32_t &my_moves, uint32_t &my_fert) {
+    StepArgs sa{};
+    sa.step = step;
+    sa.t = t;
+    const PairLists L{x.gfu + s, x.gmu + s, x.gfid + s, x.gmid + s, x.gfs + s, x.gms + s, x.gmate + s, x.gflag + s};
+    const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt();
     const int R = x.conn + 1;
     const int nchunks = (n + kWave - 1) / kWave;
 
-    // large cells (rare): fields are loaded per chunk in each pass
     CellView cv;
-    cv.N = (uint32_t)n;
-    cv.K = x.K[c];
+    const ActConst pk = {p.k.opword, p.k.nops, p.k.flags, p.k.fert_min, p.k.fert_max, p.k.fert_inter, p.k.b0, p.k.d0,
+                         p.k.b1, p.k.d1, p.k.rmove_p, p.k.wmove_p, p.k.Kconst};
+    const bool has_pair = (pk.flags & kActPair) != 0;
+    cv.rat = (pk.flags & kActVarK) ? vark_ratio((uint32_t)n, x.K[c]) : 0.0;
+    cv.ratc = (pk.flags & kActVerh) ? (double)(uint32_t)n / pk.Kconst : 0.0;
     cv.nn = x.nn[c];
 
     // ---- RandomPair: FERTILE females and males of the cell
-    if (p.has_pair) {
+    if (has_pair) {
         int32_t F = 0, M = 0;
         for (int ch = 0; ch < nchunks; ch++) {
             const int32_t li = ch * kWave + lane;
@@ -738,7 +802,7 @@ __device__ __forceinline__ void cell_act(const CtxT &x, const ProgT &p, const St
         wave_sync();
     }
 
-    // ---- actions, 64 agents at a time
+    // ---- actions, 64 agents at a time; fu/fid then list the mothers
     uint32_t stay = 0, births = 0;
     uint32_t mv[6] = {0, 0, 0, 0, 0, 0};
     // the cell's Navigate edges (a population without tables, e.g. another
@@ -750,68 +814,81 @@ __device__ __forceinline__ void cell_act(const CtxT &x, const ProgT &p, const St
         const bool valid = li < n;
         const uint32_t slot = s + (uint32_t)li;
         ActItem a;
-        a.life = 0;
-        a.g = 0;
-        a.id = 0;
-        a.birth = 0;
-        a.lastb = 0;
-        a.age = 0;
-        a.mate = -1;
-        a.age_dirty = false;
-        a.bflag = 0;
-        a.npend = 0;
-        a.navq = 0;
-        a.pk0 = a.pk1 = 0;
-        a.pu0 = a.pu1 = 0;
+        act_item_init(a);
         if (valid) {
             a.life = x.cur.life[slot];
             a.id = x.cur.id[slot];
-            if (p.need_gender) a.g = x.cur.gender[slot];
-            if (p.need_birth) a.birth = x.cur.birth[slot];
-            if (p.need_lastb) a.lastb = x.cur.lastb[slot];
-            if (p.load_age) a.age = x.cur.age[slot];
+            a.g = x.cur.gender[slot];
+            if (pk.flags & kActBirth) a.birth = x.cur.birth[slot];
+            if (pk.flags & kActLastb) a.lastb = x.cur.lastb[slot];
+            if (pk.flags & kActAge) a.age = x.cur.age[slot];
         }
-        if (valid && p.has_pair) a.mate = L.mate[li];
+        if (valid && has_pair) a.mate = L.mate[li];
         if (kAssort && valid) {
             const int32_t ps = x.gmate[slot];
             a.mate = (ps >= 0) ? (int32_t)((uint32_t)ps - s) : -1;
             my_fert += (a.life == QHG_LIFE_FERTILE && a.g <= 1) ? 1u : 0u;
         }
-        const uint8_t lifeS = a.life;
         int dir = -1;
         int32_t nave = 0;
         if (valid && a.life != 0) {
-            act_program<kRare, kNav>(x, p, sa, cv, a, my_deaths);
+            act_draws(x.seed, pk.flags, step, a);
+            act_program<kRare, kNav>(p, pk, t, cv, a, my_deaths);
             if (a.npend > 0 || (kNav && a.navq)) {
-                // the cell's neighbour and weight rows, for movers only
-                int32_t nbr[6];
-                double w[7];
-#pragma unroll
-                for (int qq = 0; qq < 6; qq++) nbr[qq] = (qq < x.conn) ? x.nbr[(int64_t)c * x.conn + qq] : -1;
-#pragma unroll
-                for (int qq = 0; qq < 7; qq++) w[qq] = (qq < R) ? x.W[(int64_t)c * R + qq] : 0.0;
-                resolve_moves<kNav>(x, p, sa, a, c, cne0, cne1, cv.nn, w, nbr, dir, nave, my_moves);
+                const double *w = x.W + (int64_t)c * R;
+                const int32_t *nbr = x.nbr + (int64_t)c * x.conn;
+                resolve_moves<kNav>(x, p, sa, a, x.ice, c, cne0, cne1, cv.nn, R, [&](int q) { return w[q]; },
+                                    [&](int d) { return nbr[d]; }, dir, nave, my_moves);
             }
         }
         const bool alive = valid && a.life != 0;
-        if (kNav && x.nav.n) nav_movers(x, alive && dir == kNavDir, nave, slot);
-        if (valid) {
-            uint8_t code = (uint8_t)(dir >= 0 ? dir + 1 : 0);
-            if (!alive) code |= kDecDead;
-            if (a.bflag) code |= kDecBirth;
-            x.dec[slot] = code;
-            if (a.life != lifeS) x.cur.life[slot] = a.life;
-            if (a.age_dirty) x.cur.age[slot] = a.age;
-            if (p.has_pair) x.cur.mate_id[slot] = (a.mate >= 0) ? x.cur.id[s + a.mate] : -3;
-            if (a.bflag) {
-                x.cur.nbabies[slot] += 1;
-                if (x.gwords) x.bfather[slot] = (int32_t)(s + a.mate);
+        uint32_t kind = kDecDead, idx = 0, rank = 0;
+        const uint64_t ms = __ballot(alive && dir < 0);
+        if (alive && dir < 0) {
+            kind = kDecStay;
+            idx = (uint32_t)c;
+            rank = stay + (uint32_t)__popcll(ms & lt);
+        }
+        stay += __popcll(ms);
+#pragma unroll
+        for (int d = 0; d < 6; d++) {
+            const uint64_t mm = __ballot(alive && dir == d);
+            if (alive && dir == d) {
+                kind = kDecMove;
+                idx = (uint32_t)c * (uint32_t)x.conn + (uint32_t)d;
+                rank = mv[d] + (uint32_t)__popcll(mm & lt);
+            }
+            mv[d] += __popcll(mm);
+        }
+        if (kNav && x.nav.n) {
+            const bool sails = alive && dir == kNavDir;
+            const uint32_t r = nav_movers(x, sails, nave);
+            if (sails) {
+                kind = kDecNav;
+                idx = (uint32_t)nave;
+                rank = r;
             }
         }
-        stay += __popcll(__ballot(alive && dir < 0));
-        births += __popcll(__ballot(valid && a.bflag));
-#pragma unroll
-        for (int d = 0; d < 6; d++) mv[d] += __popcll(__ballot(alive && dir == d));
+        const uint64_t mb = __ballot(valid && a.bflag);
+        if (valid) {
+            x.dec[slot] = dec_word(a, kind, idx, rank);
+            if (has_pair) x.gmate[slot] = (a.mate >= 0) ? (int32_t)(s + (uint32_t)a.mate) : -1;
+            if (a.bflag) {
+                const uint32_t at = births + (uint32_t)__popcll(mb & lt);
+                L.fu[at] = li;
+                L.fid[at] = a.id;
+            }
+        }
+        births += __popcll(mb);
+    }
+    if (births) {
+        wave_sync();
+        for (uint32_t j = lane; j < births; j += kWave) {
+            const int64_t my = L.fid[j];
+            uint32_t r = 0;
+            for (uint32_t k = 0; k < births; k++) r += L.fid[k] < my;
+            x.brank[s + (uint32_t)L.fu[j]] = (uint64_t)(uint32_t)c | ((uint64_t)r << 32);
+        }
     }
     if (lane == 0) {
         x.cstay[c] = stay;
@@ -829,397 +906,438 @@ __device__ __forceinline__ void cell_act(const CtxT &x, const ProgT &p, const St
     wave_sync();
 }
 
+// The cells of a step that are larger than a block takes, a wave each (entry
+// i goes to wave i mod the waves; a wave looks at 64 of its entries at once).
+template <bool kRare, bool kAssort, bool kNav>
+__device__ __forceinline__ void big_cells(ConstCtx &x, ConstProg &p, uint32_t step, double t, int64_t nocc,
+                                          uint32_t &my_deaths, uint32_t &my_moves, uint32_t &my_fert) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = uniform_i64(((int64_t)blockIdx.x * kActBlock + threadIdx.x) / kWave);
+    const int64_t nwaves = (int64_t)gridDim.x * kActWaves;
+    for (int64_t base = wave; base < nocc; base += nwaves * kWave) {
+        OccCell e{0, 0, 0, 0};
+        if (base + lane * nwaves < nocc) e = x.occ_cur[base + lane * nwaves];
+        uint64_t left = __ballot(e.n > (uint32_t)kGroupSlots);
+        while (left) {
+            const int l = __ffsll((unsigned long long)left) - 1;
+            left &= left - 1ull;
+            cell_act<kRare, kAssort, kNav>(x, p, step, t, (int32_t)readlane_u32((uint32_t)e.c, l), readlane_u32(e.s, l),
+                                           (int32_t)readlane_u32(e.n, l), my_deaths, my_moves, my_fert);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
-// packed groups: several small cells in one wave, one lane per agent
+// packed groups: the cells of a group in one block, one thread per agent
 // ---------------------------------------------------------------------------
-enum { kCntF = 0, kCntM, kCntStay, kCntBirth, kCntMv, kCntN = kCntMv + 6 };
+enum { kCntF = 0, kCntM, kCntBirth, kCntStay, kCntMv, kCntN = kCntMv + 6 };
+constexpr int kGroupWords = kGroupSlots / 64;
 
 struct GroupActLds {
+    uint64_t starts[kGroupWords];                   // bit q: a cell begins at group position q
     // FERTILE lists of cell k at positions [eb_k, eb_k + n_k): females from
-    // the front (entry r at eb_k + r), males from the back (at eb_k + n_k-1-r)
-    int64_t lid[kGroupSlots];                       // ids of the list entries
-    int64_t pid[kGroupSlots];                       // partner id per agent
-    double K[kGroupCells];                          // per-cell tables
+    // the front (rank r at eb_k + r), males from the back (at eb_k + n_k-1-r)
+    int64_t lid[kGroupSlots];                       // ids, gather order; then the mothers' ids
+    double rat[kGroupCells], ratc[kGroupCells];     // per-cell tables
     double W[kGroupCells][7];
     int32_t nbr[kGroupCells][6];
-    int32_t outk[kGroupCells][6];
-    uint32_t ud[kGroupSlots];                       // choosers' draws, id rank
+    int16_t pick[kGroupSlots];                      // rank position of a chooser -> its pick among those left
     uint32_t cnt[kGroupCells][kCntN];               // per-cell counters
-    int16_t list[kGroupSlots];                      // group positions of the entries
-    int16_t srt[kGroupSlots];                       // id order: list positions
-    int16_t mate[kGroupSlots];                      // partner's group position, -1
+    int32_t c[kGroupCells];
+    uint32_t eb[kGroupCells], n[kGroupCells];       // first position, agents
+    int16_t srt[kGroupSlots];                       // id rank -> group position of the agent
+    int16_t prt[kGroupSlots];                       // id rank -> the partner's rank position, -1
     uint8_t nn[kGroupCells];
-    int32_t noff[2 * kGroupCells];                  // Navigate: first and end edge per cell
+    int32_t noff[kGroupCells], nend[kGroupCells];   // Navigate: first and end edge per cell
+    int32_t nfit;             // cells that fit the block
 };
 
-struct CellActLds {
-    int32_t fu[kLdsCell], mu[kLdsCell], fs[kLdsCell], ms[kLdsCell], mate[kLdsCell];
-    int64_t fid[kLdsCell], mid[kLdsCell];
-    uint8_t flag[kLdsCell];
-};
-
-union ActLds {
-    GroupActLds g;
-    CellActLds c;
-};
-
-// The cells of a group are consecutive occupied cells, so their segments
-// form one slot range [S0, S0+T).  Lane k < ng holds cell k's entry e and
-// eb = e.s - S0.  Each cell's lists live at its own positions [eb, eb+n).
-template <bool kRare, bool kAssort = false, bool kNav = false, typename CtxT, typename ProgT>
-__device__ __forceinline__ void group_act(const CtxT &x, const ProgT &p, const StepArgs &sa, int ng, const OccCell &e,
-                                          uint32_t eb, uint32_t S0, uint32_t T, GroupActLds &G,
-                                          uint32_t &my_deaths, uint32_t &my_moves, uint32_t &my_fert) {
-    const int lane = threadIdx.x;
-    const int R = x.conn + 1;
-    const int nchunks = (int)((T + kWave - 1) / kWave);
-
-    // one round trip: the cells' tables (staged in LDS) and the first
-    // chunk's fields
-    double tK = 0, tW0 = 0, tW1 = 0;
-    int32_t tN0 = -1, tN1 = -1, tO0 = -1, tO1 = -1;
-    uint8_t tnn = 0;
-    const int wk0 = lane / 7, wj0 = lane % 7, wk1 = (lane + 64) / 7, wj1 = (lane + 64) % 7;
-    const int nk0 = lane / 6, nj0 = lane % 6, nk1 = (lane + 64) / 6, nj1 = (lane + 64) % 6;
-    const int32_t cw0 = __shfl(e.c, wk0 < ng ? wk0 : 0, 64), cw1 = __shfl(e.c, wk1 < ng ? wk1 : 0, 64);
-    const int32_t cn0 = __shfl(e.c, nk0 < ng ? nk0 : 0, 64), cn1 = __shfl(e.c, nk1 < ng ? nk1 : 0, 64);
-    int32_t tNo = 0, tNe = 0;
-    if (lane < ng) {
-        tK = x.K[e.c];
-        tnn = x.nn[e.c];
-        if (kNav && x.nav.n != 0) {   // no tables (null pointers) when n is 0
-            tNo = x.nav.off[e.c];
-            tNe = x.nav.off[e.c + 1];
-        }
-    }
-    if (wk0 < ng && wj0 < R) tW0 = x.W[(int64_t)cw0 * R + wj0];
-    if (wk1 < ng && wj1 < R) tW1 = x.W[(int64_t)cw1 * R + wj1];
-    if (nk0 < ng && nj0 < x.conn) {
-        tN0 = x.nbr[(int64_t)cn0 * x.conn + nj0];
-        tO0 = x.outk[(int64_t)cn0 * x.conn + nj0];
-    }
-    if (nk1 < ng && nj1 < x.conn) {
-        tN1 = x.nbr[(int64_t)cn1 * x.conn + nj1];
-        tO1 = x.outk[(int64_t)cn1 * x.conn + nj1];
-    }
-    const uint32_t q0 = (uint32_t)lane;
-    const bool v0 = q0 < T;
-    const int k0 = group_cell_of(q0, eb, ng);
-    const uint32_t slot0 = S0 + q0;
-    uint8_t life0 = 0, g0 = 2;
-    int64_t id0 = 0;
-    double birth0 = 0, lastb0 = 0, age0 = 0;
-    int32_t nbab0 = 0;
-    if (v0) {
-        life0 = x.cur.life[slot0];
-        g0 = x.cur.gender[slot0];
-        id0 = x.cur.id[slot0];
-        nbab0 = x.cur.nbabies[slot0];
-        if (p.need_birth) birth0 = x.cur.birth[slot0];
-        if (p.need_lastb) lastb0 = x.cur.lastb[slot0];
-        if (p.load_age) age0 = x.cur.age[slot0];
-    }
-    // the second chunk's fields in the same round trip (groups hold up to
-    // two chunks at the usual target; later chunks load where they are used)
-    const uint32_t q1 = (uint32_t)(kWave + lane);
-    const bool v1 = q1 < T;
-    uint8_t life1 = 0, g1 = 2;
-    int64_t id1 = 0;
-    double birth1 = 0, lastb1 = 0, age1 = 0;
-    int32_t nbab1 = 0;
-    if (v1) {
-        life1 = x.cur.life[S0 + q1];
-        g1 = x.cur.gender[S0 + q1];
-        id1 = x.cur.id[S0 + q1];
-        nbab1 = x.cur.nbabies[S0 + q1];
-        if (p.need_birth) birth1 = x.cur.birth[S0 + q1];
-        if (p.need_lastb) lastb1 = x.cur.lastb[S0 + q1];
-        if (p.load_age) age1 = x.cur.age[S0 + q1];
-    }
-    // per-cell tables to LDS: their loads were issued before the fields', so
-    // waiting for them leaves the field loads in flight
-    if (lane < ng) {
-        G.K[lane] = tK;
-        G.nn[lane] = tnn;
-        if (kNav) {
-            G.noff[lane] = tNo;
-            G.noff[lane + kGroupCells] = tNe;
-        }
-#pragma unroll
-        for (int q = 0; q < kCntN; q++) G.cnt[lane][q] = 0;
-    }
-    if (wk0 < ng && wj0 < 7) G.W[wk0][wj0] = tW0;
-    if (wk1 < ng && wj1 < 7) G.W[wk1][wj1] = tW1;
-    if (nk0 < ng && nj0 < 6) { G.nbr[nk0][nj0] = tN0; G.outk[nk0][nj0] = tO0; }
-    if (nk1 < ng && nj1 < 6) { G.nbr[nk1][nj1] = tN1; G.outk[nk1][nj1] = tO1; }
-    wave_sync();
-
-    // ---- RandomPair (RandomPair.cpp:107-279), every cell of the group at once
-    if (p.has_pair) {
-        for (int ch = 0; ch < nchunks; ch++) {
-            const uint32_t q = (uint32_t)(ch * kWave + lane);
-            const bool valid = q < T;
-            const int k = (ch == 0) ? k0 : group_cell_of(q, eb, ng);
-            const uint32_t base = (uint32_t)__shfl((int)eb, k, 64);
-            const uint32_t nk = (uint32_t)__shfl((int)e.n, k, 64);
-            uint8_t l = (ch == 0) ? life0 : life1, g = (ch == 0) ? g0 : g1;
-            int64_t id = (ch == 0) ? id0 : id1;
-            if (ch > 1 && valid) {
-                l = x.cur.life[S0 + q];
-                g = x.cur.gender[S0 + q];
-                id = x.cur.id[S0 + q];
-            }
-            if (valid) {
-                G.mate[q] = -1;
-                if (l == QHG_LIFE_FERTILE && g == 0) {
-                    const uint32_t r = atomicAdd(&G.cnt[k][kCntF], 1u);
-                    G.list[base + r] = (int16_t)q;
-                    G.lid[base + r] = id;
-                } else if (l == QHG_LIFE_FERTILE && g == 1) {
-                    const uint32_t r = atomicAdd(&G.cnt[k][kCntM], 1u);
-                    G.list[base + nk - 1 - r] = (int16_t)q;
-                    G.lid[base + nk - 1 - r] = id;
-                }
-            }
-        }
-        wave_sync();
-        // id order inside each cell's lists; the choosing sex (the smaller,
-        // females on a tie) takes its pick draw now
-        for (int ch = 0; ch < nchunks; ch++) {
-            const uint32_t q = (uint32_t)(ch * kWave + lane);
-            const bool valid = q < T;
-            const int k = (ch == 0) ? k0 : group_cell_of(q, eb, ng);
-            const uint32_t base = (uint32_t)__shfl((int)eb, k, 64);
-            const uint32_t nk = (uint32_t)__shfl((int)e.n, k, 64);
-            if (!valid) continue;
-            const uint32_t Fk = G.cnt[k][kCntF], Mk = G.cnt[k][kCntM];
-            const uint32_t t = q - base;
-            if (t < Fk) {
-                const int64_t my = G.lid[q];
-                uint32_t r = 0;
-                for (uint32_t u = 0; u < Fk; u++) r += G.lid[base + u] < my;
-                G.srt[base + r] = (int16_t)q;
-                if (Fk <= Mk) G.ud[base + r] = draw(x.seed, sa.step, QHG_STREAM_PAIR, (uint64_t)my, 0);
-            } else if (nk - 1 - t < Mk) {
-                const int64_t my = G.lid[q];
-                const uint32_t top = base + nk - 1;
-                uint32_t r = 0;
-                for (uint32_t u = 0; u < Mk; u++) r += G.lid[top - u] < my;
-                G.srt[top - r] = (int16_t)q;
-                if (Mk < Fk) G.ud[base + r] = draw(x.seed, sa.step, QHG_STREAM_PAIR, (uint64_t)my, 0);
-            }
-        }
-        wave_sync();
-        // findMates (RandomPair.cpp:183-276): lane k picks for cell k, each
-        // pick the k-th (id order) still unpaired of the other sex
-        if (lane < ng) {
-            const uint32_t Fk = G.cnt[lane][kCntF], Mk = G.cnt[lane][kCntM];
-            my_fert += Fk + Mk;
-            if (Fk > 0 && Mk > 0) {
-                const bool fsel = Fk <= Mk;
-                const uint32_t nchs = fsel ? Fk : Mk, np = fsel ? Mk : Fk;
-                const uint32_t top = eb + e.n - 1;
-                uint64_t mask = (np >= 64) ? ~0ull : ((1ull << np) - 1ull);
-                uint32_t left = np;
-                for (uint32_t q = 0; q < nchs; q++) {
-                    const int kp = (int)wrandr(0, (double)left, G.ud[eb + q]);
-                    const int pos = select_bit(mask, kp);
-                    mask &= ~(1ull << pos);
-                    const int16_t la = G.srt[fsel ? eb + q : top - q];
-                    const int16_t lb = G.srt[fsel ? top - pos : eb + pos];
-                    const int16_t ja = G.list[la], jb = G.list[lb];
-                    G.mate[ja] = jb;
-                    G.mate[jb] = ja;
-                    G.pid[ja] = G.lid[lb];
-                    G.pid[jb] = G.lid[la];
-                    left--;
-                }
-            }
-        }
-    }
-    wave_sync();
-
-    // ---- actions, one lane per agent
-    for (int ch = 0; ch < nchunks; ch++) {
-        const uint32_t q = (uint32_t)(ch * kWave + lane);
-        const bool valid = q < T;
-        const uint32_t slot = S0 + q;
-        const int k = (ch == 0) ? k0 : group_cell_of(q, eb, ng);
-        const uint32_t nk = (uint32_t)__shfl((int)e.n, k, 64);
+// One group: the cells of occupied-cell entries [d0.first, d1.first), whose
+// segments form the slot range [d0.s, d1.s).
+//
+// The kernel is bound by instruction issue and by the length of its chain of
+// dependent steps, not by bytes, so the split aims at full waves and few
+// steps: 64 agents per wave wherever the cells' borders lie (a group is cut by
+// agents, not by a number of cells), every chooser's pick by its own thread,
+// one copy of every draw, partners through ranks (no sorted copies), the place
+// of every agent in its run from the counting atomics themselves, and all
+// uniform values in scalar registers from the start (read where they are
+// used, each costs a trip to the scalar cache on the chain).  With one wave
+// per group of ~4 cells, 60 % of the lanes filled and the picks one after
+// another, the kernel took 137 us at 1.39 M agents, 38.5 at 369 k and 15.5 at
+// 6 k; in this form 55, 20 and 10.
+template <bool kRare, bool kAssort, bool kNav>
+__device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t step, double t, GroupDesc d0,
+                                          GroupDesc d1, GroupActLds &G, uint32_t &my_deaths, uint32_t &my_moves,
+                                          uint32_t &my_fert) {
+    ConstCtx &x = *xp;
+    ConstProg &p = *pp;
+    StepArgs sa{};
+    sa.step = step;
+    sa.t = t;
+    ActConst pk = {p.k.opword, p.k.nops, p.k.flags, p.k.fert_min, p.k.fert_max, p.k.fert_inter, p.k.b0, p.k.d0,
+                   p.k.b1, p.k.d1, p.k.rmove_p, p.k.wmove_p, p.k.Kconst};
+    uint64_t seed = x.seed;
+    const uint8_t *ice = x.ice;
+    uint64_t *dec = x.dec;
+    int32_t *gmate = x.gmate;
+    uint32_t *cstay = x.cstay, *cbirth = x.cbirth, *cin = x.cin, *carr = x.carr, *tact = x.tact;
+    int conn = x.conn;
+    asm volatile("" : "+s"(pk.opword), "+s"(pk.nops), "+s"(pk.flags), "+s"(pk.fert_min), "+s"(pk.fert_max),
+                      "+s"(pk.fert_inter), "+s"(pk.b0), "+s"(pk.d0), "+s"(pk.b1), "+s"(pk.d1), "+s"(pk.rmove_p),
+                      "+s"(pk.wmove_p));
+    asm volatile("" : "+s"(seed), "+s"(ice), "+s"(dec), "+s"(gmate), "+s"(cstay), "+s"(cbirth), "+s"(cin), "+s"(carr),
+                      "+s"(tact), "+s"(conn));
+    const int R = conn + 1;
+    const bool has_pair = (pk.flags & kActPair) != 0;
+    uint32_t i0 = readlane_u32(d0.first, 0), S0 = readlane_u32(d0.s, 0);
+    const uint32_t i1 = readlane_u32(d1.first, 0), S1 = readlane_u32(d1.s, 0);
+    while (i0 < i1) {
+        // (a new value to the compiler in every pass: the positions and LDS
+        // addresses made from it would else be held across the loop, 60 VGPRs)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        // the agents' fields and the cells' entries in one round trip
+        const uint32_t slot = S0 + (uint32_t)tid;
         ActItem a;
-        a.life = (ch == 0) ? life0 : life1;
-        a.g = (ch == 0) ? g0 : g1;
-        a.id = (ch == 0) ? id0 : id1;
-        a.birth = (ch == 0) ? birth0 : birth1;
-        a.lastb = (ch == 0) ? lastb0 : lastb1;
-        a.age = (ch == 0) ? age0 : age1;
-        a.mate = -1;
-        a.age_dirty = false;
-        a.bflag = 0;
-        a.npend = 0;
-        a.navq = 0;
-        a.pk0 = a.pk1 = 0;
-        a.pu0 = a.pu1 = 0;
-        int32_t nbab = (ch == 0) ? nbab0 : nbab1;
-        if (ch > 1) {
-            a.life = 0;
-            if (valid) {
-                a.life = x.cur.life[slot];
-                a.id = x.cur.id[slot];
-                nbab = x.cur.nbabies[slot];
-                if (p.need_gender) a.g = x.cur.gender[slot];
-                if (p.need_birth) a.birth = x.cur.birth[slot];
-                if (p.need_lastb) a.lastb = x.cur.lastb[slot];
-                if (p.load_age) a.age = x.cur.age[slot];
+        act_item_init(a);
+        if (slot < S1) {
+            a.life = x.cur.life[slot];
+            a.g = x.cur.gender[slot];
+            a.id = x.cur.id[slot];
+            if (pk.flags & kActBirth) a.birth = x.cur.birth[slot];
+            if (pk.flags & kActLastb) a.lastb = x.cur.lastb[slot];
+            if (pk.flags & kActAge) a.age = x.cur.age[slot];
+            if (kAssort) a.mate = gmate[slot];
+        }
+        int nc = (int)(i1 - i0);
+        OccCell e{0, 0, 0, 0};
+        if (tid < nc) e = x.occ_cur[i0 + (uint32_t)tid];
+        for (int k = tid; k < nc * kCntN; k += kActBlock) (&G.cnt[0][0])[k] = 0u;
+        if (tid < kGroupWords) G.starts[tid] = 0ull;
+        if (tid == 0) G.nfit = nc;
+        G.prt[tid] = -1;
+        __syncthreads();
+        if (tid < nc) {
+            const uint32_t eb = e.s - S0;
+            if (eb < (uint32_t)kGroupSlots) {
+                // the first cell that ends past the block's agents begins the next pass
+                if (eb + e.n > (uint32_t)kGroupSlots) G.nfit = tid;
+                else atomicOr((unsigned long long *)&G.starts[eb >> 6], 1ull << (eb & 63u));
+            } else if (eb == (uint32_t)kGroupSlots) {
+                G.nfit = tid;
+            }
+            G.c[tid] = e.c;
+            G.eb[tid] = eb;
+            G.n[tid] = e.n;
+        }
+        __syncthreads();
+        nc = uniform_i32(G.nfit);
+        if (nc == 0) {   // a cell larger than the block (big_cells)
+            S0 += (uint32_t)uniform_i32((int)G.n[0]);
+            i0++;
+            __syncthreads();
+            continue;
+        }
+        // [eb, eb + n) of cell nc - 1 ends the pass
+        const uint32_t T = (uint32_t)uniform_i32((int)(G.eb[nc - 1] + G.n[nc - 1]));
+        const bool valid = (uint32_t)tid < T;
+        // the agent's cell: cells beginning at or before it
+        int k = __popcll(G.starts[tid >> 6] & (~0ull >> (63 - (tid & 63)))) - 1;
+#pragma unroll
+        for (int j = 0; j < kGroupWords - 1; j++)
+            if (j < (tid >> 6)) k += __popcll(G.starts[j]);
+        const int eb = (int)G.eb[k], nk = (int)G.n[k];
+        const int32_t c = G.c[k];
+        // the cells' tables: read now, put into LDS two barriers below, where
+        // their round trip is over
+        double tW = 0, tK = 0;
+        int32_t tN = -1, tO = -1, tE0 = 0, tE1 = 0;
+        uint8_t tnn = 0;
+        const int wk = tid / 7, wj = tid % 7, nk6 = tid / 6, nj = tid % 6;
+        if (wk < nc && wj < R) tW = x.W[(int64_t)G.c[wk] * R + wj];
+        if (nk6 < nc && nj < conn) {
+            const int64_t at = (int64_t)G.c[nk6] * conn + nj;
+            tN = x.nbr[at];
+            tO = x.outk[at];
+        }
+        const int kc = tid - kWave;   // the second wave's lanes: one cell each
+        if (kc >= 0 && kc < nc) {
+            const int32_t cc = G.c[kc];
+            if (pk.flags & kActVarK) tK = x.K[cc];
+            tnn = x.nn[cc];
+            if (kNav && x.nav.n != 0) {   // no tables (null pointers) when n is 0
+                tE0 = x.nav.off[cc];
+                tE1 = x.nav.off[cc + 1];
             }
         }
-        CellView cv;
-        cv.N = nk;
-        cv.K = G.K[k];
-        cv.nn = G.nn[k];
-        if (valid && p.has_pair) a.mate = G.mate[q];
-        if (kAssort && valid) {
-            // the partner's slot from k_assort_pair, as a group position;
-            // the FERTILE agents it considered are counted here
-            const int32_t ps = x.gmate[slot];
-            a.mate = (ps >= 0) ? (int32_t)((uint32_t)ps - S0) : -1;
-            my_fert += (a.life == QHG_LIFE_FERTILE && a.g <= 1) ? 1u : 0u;
+
+        // ---- RandomPair (RandomPair.cpp:107-279), every cell of the group at once
+        const bool isF = valid && a.life == QHG_LIFE_FERTILE && a.g == 0;
+        const bool isM = valid && a.life == QHG_LIFE_FERTILE && a.g == 1;
+        int P = -1;               // the agent's position by sex and id in its cell's run
+        int rank = 0, np = 0;     // its rank; choosers: the other sex's count
+        const int first = isF ? eb : eb + nk - 1, dirn = isF ? 1 : -1;
+        if (has_pair) {
+            if (isF || isM) {
+                const int r = (int)atomicAdd(&G.cnt[k][isF ? kCntF : kCntM], 1u);
+                G.lid[first + dirn * r] = a.id;
+                my_fert++;
+            }
+            __syncthreads();
+            // each listed agent's rank by id; the choosing sex (the smaller,
+            // females on a tie) draws its pick, the k-th of the np - rank that
+            // will be left: k = (int)wrandr(0, left, u) = left * u >> 32 (every
+            // factor is exact in a double)
+            if (isF || isM) {
+                const int Fk = (int)G.cnt[k][kCntF], Mk = (int)G.cnt[k][kCntM];
+                const int n1 = isF ? Fk : Mk;
+                for (int u = 0; u < n1; u += 4) {
+                    int64_t o[4];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) o[v] = G.lid[first + dirn * ((u + v < n1) ? u + v : 0)];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) rank += (u + v < n1 && o[v] < a.id) ? 1 : 0;
+                }
+                P = first + dirn * rank;
+                G.srt[P] = (int16_t)tid;
+                if (isF ? (Fk <= Mk) : (Mk < Fk)) {
+                    np = isF ? Mk : Fk;
+                    const uint32_t u = draw(seed, step, QHG_STREAM_PAIR, (uint64_t)a.id, 0);
+                    G.pick[P] = (int16_t)__umulhi((uint32_t)(np - rank), u);
+                }
+            }
         }
-        const uint8_t lifeS = a.life;
+        if (wk < nc) G.W[wk][wj] = tW;
+        if (nk6 < nc) G.nbr[nk6][nj] = tN;
+        if (kc >= 0 && kc < nc) {
+            G.rat[kc] = (pk.flags & kActVarK) ? vark_ratio(G.n[kc], tK) : 0.0;
+            G.ratc[kc] = (pk.flags & kActVerh) ? (double)G.n[kc] / pk.Kconst : 0.0;
+            G.nn[kc] = tnn;
+            if (kNav) {
+                G.noff[kc] = tE0;
+                G.nend[kc] = tE1;
+            }
+        }
+        if (nc * 7 > kActBlock) {   // many small cells: the rows beyond the block's threads
+            for (int q = tid + kActBlock; q < nc * 7; q += kActBlock)
+                G.W[q / 7][q % 7] = (q % 7 < R) ? x.W[(int64_t)G.c[q / 7] * R + q % 7] : 0.0;
+            for (int q = tid + kActBlock; q < nc * 6; q += kActBlock)
+                G.nbr[q / 6][q % 6] = (q % 6 < conn) ? x.nbr[(int64_t)G.c[q / 6] * conn + q % 6] : -1;
+        }
+        __syncthreads();
+        // findMates (RandomPair.cpp:183-276): choosers in id order, each
+        // taking the pick-th (id order) still unpaired of the other sex.  The
+        // place of that one among all np, by every chooser for itself: among
+        // those left before chooser j took its pick, the places from that
+        // pick on were one higher.
+        if (np > 0) {
+            int pos = G.pick[P];
+            for (int j = rank - 1; j >= 0; j -= 4) {
+                int o[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) o[v] = (j - v >= 0) ? G.pick[first + dirn * (j - v)] : 0x7FFF;
+#pragma unroll
+                for (int v = 0; v < 4; v++) pos += (pos >= o[v]) ? 1 : 0;
+            }
+            const int to = (isF ? eb + nk - 1 : eb) - dirn * pos;
+            G.prt[P] = (int16_t)to;
+            G.prt[to] = (int16_t)P;
+        }
+        act_draws(seed, pk.flags, step, a);
+        __syncthreads();
+
+        // ---- actions, one thread per agent
+        CellView cv;
+        cv.rat = G.rat[k];
+        cv.ratc = G.ratc[k];
+        cv.nn = G.nn[k];
+        if (has_pair) {
+            const int pp2 = (P >= 0) ? G.prt[P] : -1;
+            a.mate = (pp2 >= 0) ? (int32_t)(S0 + (uint32_t)G.srt[pp2]) : -1;
+        }
+        if (kAssort && valid) my_fert += (a.life == QHG_LIFE_FERTILE && a.g <= 1) ? 1u : 0u;
         int dir = -1;
         int32_t nave = 0;
-        const int32_t cc = kNav ? __shfl(e.c, k, 64) : 0;   // the agent's cell (Navigate)
         if (valid && a.life != 0) {
-            act_program<kRare, kNav>(x, p, sa, cv, a, my_deaths);
-            if (a.npend > 0 || (kNav && a.navq)) {
-                int32_t nbr[6];
-                double w[7];
-#pragma unroll
-                for (int qq = 0; qq < 6; qq++) nbr[qq] = (qq < x.conn) ? G.nbr[k][qq] : -1;
-#pragma unroll
-                for (int qq = 0; qq < 7; qq++) w[qq] = (qq < R) ? G.W[k][qq] : 0.0;
-                resolve_moves<kNav>(x, p, sa, a, cc, kNav ? G.noff[k] : 0, kNav ? G.noff[k + kGroupCells] : 0,
-                                    cv.nn, w, nbr, dir, nave, my_moves);
-            }
+            act_program<kRare, kNav>(p, pk, t, cv, a, my_deaths);
+            if (a.npend > 0 || (kNav && a.navq))
+                resolve_moves<kNav>(x, p, sa, a, ice, c, kNav ? G.noff[k] : 0, kNav ? G.nend[k] : 0, cv.nn, R,
+                                    [&](int q) { return G.W[k][q]; }, [&](int d) { return G.nbr[k][d]; }, dir, nave,
+                                    my_moves);
         }
         const bool alive = valid && a.life != 0;
-        if (kNav && x.nav.n) nav_movers(x, alive && dir == kNavDir, nave, slot);
+        uint32_t kind = kDecDead, idx = 0, place = 0;
+        if (kNav && x.nav.n) {
+            const bool sails = alive && dir == kNavDir;
+            place = nav_movers(x, sails, nave);
+            if (sails) {
+                kind = kDecNav;
+                idx = (uint32_t)nave;
+            }
+        }
+        if (alive && (!kNav || dir != kNavDir)) {
+            place = atomicAdd(&G.cnt[k][dir < 0 ? kCntStay : kCntMv + dir], 1u);
+            kind = dir < 0 ? kDecStay : kDecMove;
+            idx = dir < 0 ? (uint32_t)c : (uint32_t)c * (uint32_t)conn + (uint32_t)dir;
+        }
+        const bool gave = valid && a.bflag;
+        if (gave) G.lid[eb + (int)atomicAdd(&G.cnt[k][kCntBirth], 1u)] = a.id;
         if (valid) {
-            uint8_t code = (uint8_t)(dir >= 0 ? dir + 1 : 0);
-            if (!alive) code |= kDecDead;
-            if (a.bflag) code |= kDecBirth;
-            x.dec[slot] = code;
-            if (a.life != lifeS) x.cur.life[slot] = a.life;
-            if (a.age_dirty) x.cur.age[slot] = a.age;
-            if (p.has_pair) x.cur.mate_id[slot] = (a.mate >= 0) ? G.pid[q] : -3;
-            if (a.bflag) {
-                x.cur.nbabies[slot] = nbab + 1;
-                if (x.gwords) x.bfather[slot] = (int32_t)(S0 + a.mate);
-                atomicAdd(&G.cnt[k][kCntBirth], 1u);
-            }
-            if (alive && (!kNav || dir != kNavDir)) atomicAdd(&G.cnt[k][dir < 0 ? kCntStay : kCntMv + dir], 1u);
+            dec[slot] = dec_word(a, kind, idx, place);
+            if (has_pair) gmate[slot] = a.mate;
         }
-    }
-    wave_sync();
-    if (lane < ng) {
-        x.cstay[e.c] = G.cnt[lane][kCntStay];
-        if (G.cnt[lane][kCntBirth]) x.cbirth[e.c] = G.cnt[lane][kCntBirth];
-        if (G.cnt[lane][kCntStay] | G.cnt[lane][kCntBirth]) x.tact[e.c / kCellTile] = 1u;
-        for (int d = 0; d < x.conn; d++) {
-            const uint32_t m = G.cnt[lane][kCntMv + d];
+        __syncthreads();
+        // mothers' ranks by id in their cells, and the cells' counts
+        if (gave) {
+            const int nb = (int)G.cnt[k][kCntBirth];
+            uint32_t r = 0;
+            for (int u = 0; u < nb; u++) r += G.lid[eb + u] < a.id;
+            x.brank[slot] = (uint64_t)(uint32_t)c | ((uint64_t)r << 32);
+        }
+        if (tid < nc) {
+            const uint32_t st = G.cnt[tid][kCntStay], bi = G.cnt[tid][kCntBirth];
+            cstay[e.c] = st;
+            if (bi) cbirth[e.c] = bi;
+            if (st | bi) tact[e.c / kCellTile] = 1u;
+        }
+        for (int q = tid; q < nc * 6; q += kActBlock) {
+            const int kk = q / 6, d = q % 6;
+            const uint32_t m = G.cnt[kk][kCntMv + d];
             if (m) {
-                const int32_t dest = G.nbr[lane][d];
-                x.cin[G.outk[lane][d]] = m;
-                atomicAdd(&x.carr[dest], m);
-                x.tact[dest / kCellTile] = 1u;
+                const int32_t dest = G.nbr[kk][d];
+                cin[(q == tid) ? tO : x.outk[(int64_t)G.c[kk] * conn + d]] = m;
+                atomicAdd(&carr[dest], m);
+                tact[dest / kCellTile] = 1u;
             }
         }
+        i0 += (uint32_t)nc;
+        S0 += T;
+        if (i0 < i1) __syncthreads();   // the next pass writes the LDS read here
     }
-    wave_sync();
+}
+
+struct ActArgs {
+    Ctx x;
+    Prog p;
+    StepArgs sa;
+};
+typedef __attribute__((address_space(4))) const ActArgs ConstActArgs;
+
+// The arguments are read through the kernel's argument segment, by a pointer
+// that the compiler takes for a new one in every group: what a phase needs
+// goes to scalar registers there.  Held for the whole loop, the ~130 uniform
+// values of the two code paths do not fit: 224 of them lived in vector lanes,
+// and their reloads were a third of the vector instructions.
+__device__ __forceinline__ ConstActArgs *act_args() {
+    ConstActArgs *a = (ConstActArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return a;
+}
+
+// One word of every 64-byte line of [0, bytes), so that the lines come into the
+// scalar cache in one round trip: it is cold when a kernel starts, and each
+// line first read where it is needed costs a trip to memory of its own.
+__device__ __forceinline__ void touch_lines(const __attribute__((address_space(4))) void *at, int bytes) {
+    const __attribute__((address_space(4))) uint32_t *w = (const __attribute__((address_space(4))) uint32_t *)at;
+    uint32_t v = 0;
+#pragma unroll
+    for (int i = 0; i < bytes / 4; i += 16) v ^= w[i];
+    asm volatile("" ::"s"(v));
 }
 
 template <bool kRare, bool kAssort, bool kNav>
-__device__ __forceinline__ void cell_act_kernel(const Ctx &x, const Prog &p, const StepArgs &sa) {
-    __shared__ ActLds lds;
-    const int lane = threadIdx.x;
+__device__ __forceinline__ void cell_act_kernel() {
+    __shared__ GroupActLds lds;
+    __shared__ uint32_t part[kParts];
+    const int tid = threadIdx.x;
     uint32_t my_deaths = 0, my_moves = 0, my_fert = 0;
-    // one round trip: the status and this wave's first group of occupied
-    // cells (read ahead of the count check: every index below ncells exists)
-    const int32_t err = x.st->error;
-    const int64_t nocc = x.st->n_occ[sa.parity];
-    const int64_t gc = sa.gcells;
-    OccCell e_first{0, 0, 0, 0};
     {
-        const int64_t idx = (int64_t)blockIdx.x * gc + lane;
-        if (lane < gc && idx < x.ncells) e_first = x.occ_cur[idx];
-    }
-    // a failed step (capacity, look-back, count) freezes the population:
-    // later steps already enqueued touch nothing
-    if (err) return;
-
-    // look-back words of this step's k_cell_scan start at zero, and so do
-    // the step's death and move counts (k_cell_scan adds them up)
-    for (int32_t i = blockIdx.x * kCellBlock + lane; i < x.ntiles; i += gridDim.x * kCellBlock) {
-        x.tiles[i] = 0;
-        x.tiles2[i] = 0;
-    }
-    if (blockIdx.x == 0 && lane == 0) {
-        x.st->deaths_last = 0;
-        x.st->moves_last = 0;
-        *x.tick = 0u;
-    }
-
-    // groups of gcells consecutive occupied cells, round-robin over the
-    // waves; empty cells keep the zero counts the previous scan left
-    const int64_t ngroups = (nocc + gc - 1) / gc;
-    for (int64_t gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
-        const int64_t i0 = gi * gc;
-        const int ng = (int)((nocc - i0 < gc) ? (nocc - i0) : gc);
-        OccCell e{0, 0, 0, 0};
-        if (lane < ng) e = (gi == blockIdx.x) ? e_first : x.occ_cur[i0 + lane];
-        const uint32_t S0 = readlane_u32(e.s, 0);
-        const uint32_t T = readlane_u32(e.s, ng - 1) + readlane_u32(e.n, ng - 1) - S0;
-        const uint32_t nmax = wave_max_u32(lane < ng ? e.n : 0u);
-        if (T <= (uint32_t)kGroupSlots && nmax <= (uint32_t)kGroupCellMax) {
-            group_act<kRare, kAssort, kNav>(x, p, sa, ng, e, e.s - S0, S0, T, lds.g, my_deaths, my_moves, my_fert);
-            continue;
+        ConstActArgs &A = *act_args();
+        touch_lines(&A, (int)(offsetof(ActArgs, p) + offsetof(Prog, bino)));
+        const int64_t par = (int64_t)A.sa.parity;
+        // one round trip: the status and this block's first group (read ahead
+        // of the count check, inside the list)
+        const int32_t err = A.x.st->error;
+        const int64_t ngrp = A.x.st->n_grp[par];
+        const int64_t big = A.x.st->big[par], nocc = A.x.st->n_occ[par];
+        int64_t g = blockIdx.x;
+        const GroupDesc *grp = A.x.cur.grp;
+        const int64_t ga = (g + 1 < A.x.grp_cap) ? g : 0;
+        GroupDesc d0 = grp[ga], d1 = grp[ga + 1];
+        // a failed step (capacity, look-back, count) freezes the population:
+        // later steps already enqueued touch nothing
+        if (err) return;
+        // look-back words of this step's k_cell_scan start at zero, and so do
+        // the step's death and move counts (k_cell_scan adds them up)
+        for (int32_t i = blockIdx.x * kActBlock + tid; i < A.x.ntiles; i += gridDim.x * kActBlock) {
+            A.x.tiles[i] = 0;
+            A.x.tiles2[i] = 0;
         }
-        for (int k = 0; k < ng; k++) {
-            const int32_t c = (int32_t)readlane_u32((uint32_t)e.c, k);
-            const uint32_t s = readlane_u32(e.s, k);
-            const int32_t n = (int32_t)readlane_u32(e.n, k);
-            PairLists L;
-            if (n > kLdsCell) {
-                L = PairLists{x.gfu + s, x.gmu + s, x.gfid + s, x.gmid + s, x.gfs + s, x.gms + s, x.gmate + s,
-                              x.gflag + s};
-            } else {
-                L = PairLists{lds.c.fu, lds.c.mu, lds.c.fid, lds.c.mid, lds.c.fs, lds.c.ms, lds.c.mate,
-                              lds.c.flag};
+        if (blockIdx.x == 0 && tid == 0) {
+            A.x.st->deaths_last = 0;
+            A.x.st->moves_last = 0;
+            A.x.st->big[1 - par] = 0;   // k_cell_scan sets it
+            *A.x.tick = 0u;
+        }
+        if (tid < kParts) part[tid] = 0u;
+        for (; g < ngrp; g += gridDim.x) {
+            ConstActArgs &B = *act_args();
+            if (g != (int64_t)blockIdx.x) {
+                __syncthreads();   // the group before has read its LDS
+                d0 = B.x.cur.grp[g];
+                d1 = B.x.cur.grp[g + 1];
             }
-            cell_act<kRare, kAssort, kNav>(x, p, sa, c, s, n, L, my_deaths, my_moves, my_fert);
+            group_act<kRare, kAssort, kNav>(&B.x, &B.p, B.sa.step, B.sa.t, d0, d1, lds, my_deaths, my_moves, my_fert);
+        }
+        if (uniform_i64(big)) {
+            ConstActArgs &B = *act_args();
+            big_cells<kRare, kAssort, kNav>(B.x, B.p, B.sa.step, B.sa.t, uniform_i64(nocc), my_deaths, my_moves, my_fert);
         }
     }
+    __syncthreads();
     const uint64_t dm = wave_sum_u64(((uint64_t)my_moves << 32) | my_deaths);
     const uint32_t fe = (uint32_t)wave_sum_u64(my_fert);
-    if (lane == 0) {
-        uint32_t *wp = x.wave_part + kParts * blockIdx.x;
-        wp[0] = (uint32_t)dm;
-        wp[1] = (uint32_t)(dm >> 32);
-        wp[2] = fe;
+    if ((tid & 63) == 0) {
+        if ((uint32_t)dm) atomicAdd(&part[0], (uint32_t)dm);
+        if ((uint32_t)(dm >> 32)) atomicAdd(&part[1], (uint32_t)(dm >> 32));
+        if (fe) atomicAdd(&part[2], fe);
     }
+    __syncthreads();
+    if (tid < kParts) act_args()->x.wave_part[kParts * blockIdx.x + tid] = part[tid];
 }
 
 template <bool kRare, bool kAssort>
-__global__ void __launch_bounds__(kCellBlock) k_cell_act(Ctx x, Prog p, StepArgs sa) {
-    cell_act_kernel<kRare, kAssort, false>(x, p, sa);
+__global__ void __launch_bounds__(kActBlock) k_cell_act(ActArgs) {
+    cell_act_kernel<kRare, kAssort, false>();
 }
 
-// with Navigate: its code would take the kernel to 193 VGPRs and 2 waves per
-// SIMD; held to 3 waves (a few spilled registers)
 template <bool kRare, bool kAssort>
-__global__ void __launch_bounds__(kCellBlock) __attribute__((amdgpu_waves_per_eu(3)))
-k_cell_act_nav(Ctx x, Prog p, StepArgs sa) {
-    cell_act_kernel<kRare, kAssort, true>(x, p, sa);
+__global__ void __launch_bounds__(kActBlock) k_cell_act_nav(ActArgs) {
+    cell_act_kernel<kRare, kAssort, true>();
+}
+
+// The outcomes of a step that has acted but not committed, into the agents'
+// records, for a caller who looks at them there (the commit itself reads the
+// outcome words).  what: 1 the step's partners, 2 the outcomes.
+__global__ void __launch_bounds__(256) k_act_commit(Ctx x, StepArgs sa, int32_t what) {
+    const int64_t n = x.st->n_alive[sa.parity];
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        if (what & 1) {
+            const int32_t m = x.gmate[i];
+            x.cur.mate_id[i] = (m >= 0) ? x.cur.id[m] : -3;
+        }
+        if (what & 2) {
+            const uint64_t w = x.dec[i];
+            if (((w >> kDecKindAt) & 3u) == kDecDead) x.cur.life[i] = 0;
+            else if (sa.sets_life) x.cur.life[i] = (w & kDecFertile) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
+            if (w & kDecAged) x.cur.age[i] = sa.t - x.cur.birth[i];
+            if ((w & kDecBirth) && !(w & kDecCounted)) {
+                x.cur.nbabies[i] += 1;
+                x.dec[i] = w | kDecCounted;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1235,8 +1353,8 @@ k_cell_act_nav(Ctx x, Prog p, StepArgs sa) {
 //     females that reach it (permuted when asked), each female in turn
 //     picking at random among the unpaired males at that value.
 // The cell's draws come in the reference's order from QHG_STREAM_ASSORT.
-// Output: x.gmate[slot] = partner slot (-1 none) and mate_id; k_cell_act
-// reads gmate instead of pairing.  Scratch in the cell's own slot range
+// Output: x.gmate[slot] = partner slot (-1 none); k_cell_act reads it instead
+// of pairing.  Scratch in the cell's own slot range
 // [s, s+n): gfu/gfid, gmu/gmid (gather), gfs/gms (slots in id order),
 // gfu/gmu (then their genome handles in id order), gfid (the round's female
 // order), gflag (paired: female r at s+r, male r at s+F+r).
@@ -1286,7 +1404,6 @@ __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, in
             g = x.cur.gender[slot];
             id = x.cur.id[slot];
             x.gmate[slot] = -1;
-            x.cur.mate_id[slot] = -3;
         }
         const bool isF = valid && l == QHG_LIFE_FERTILE && g == 0;
         const bool isM = valid && l == QHG_LIFE_FERTILE && g == 1;
@@ -1418,8 +1535,6 @@ __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, in
                 pm[jm] = 1;
                 x.gmate[sf] = sm;
                 x.gmate[sm] = sf;
-                x.cur.mate_id[sf] = x.cur.id[sm];
-                x.cur.mate_id[sm] = x.cur.id[sf];
             }
             paired = true;
             wave_sync();
@@ -1436,7 +1551,6 @@ __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, in
 constexpr int kAssortMaxDist = 128;
 struct AssortLds {
     int64_t fid[kWave], mid[kWave];       // ids, gather order
-    int64_t fsid[kWave], msid[kWave];     // ids, id order
     int32_t fslot[kWave], mslot[kWave];   // slots, id order
     int32_t ord[kWave];                   // the round's female order
     uint64_t fw[kWave][4], mw[kWave][4];  // compared genome words (2 * D <= 4), id order
@@ -1469,7 +1583,6 @@ __device__ void assort_cell_lds(const CtxT &x, const Prog &p, const StepArgs &sa
         id = x.cur.id[slot];
         h = x.cur.ghandle[slot];
         x.gmate[slot] = -1;
-        x.cur.mate_id[slot] = -3;
     }
     const bool isF = valid && l == QHG_LIFE_FERTILE && g == 0;
     const bool isM = valid && l == QHG_LIFE_FERTILE && g == 1;
@@ -1491,14 +1604,12 @@ __device__ void assort_cell_lds(const CtxT &x, const Prog &p, const StepArgs &sa
         if ((isF || isM) && k < 2 * D) w[k] = gw[k];
     if (isF) {
         L.fslot[r] = (int32_t)slot;
-        L.fsid[r] = id;
 #pragma unroll
         for (int k = 0; k < 4; k++) L.fw[r][k] = w[k];
         L.pf[r] = 0;
     }
     if (isM) {
         L.mslot[r] = (int32_t)slot;
-        L.msid[r] = id;
 #pragma unroll
         for (int k = 0; k < 4; k++) L.mw[r][k] = w[k];
         L.pm[r] = 0;
@@ -1566,8 +1677,6 @@ __device__ void assort_cell_lds(const CtxT &x, const Prog &p, const StepArgs &sa
                 L.pm[jm] = 1;
                 x.gmate[sf] = sm;
                 x.gmate[sm] = sf;
-                x.cur.mate_id[sf] = L.msid[jm];
-                x.cur.mate_id[sm] = L.fsid[i];
             }
             paired = true;
             wave_sync();
@@ -1631,6 +1740,31 @@ __device__ __forceinline__ uint32_t next_tile(uint32_t *ticket, ScanLds &L) {
     const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.ticket);
     __syncthreads();
     return t;
+}
+
+// The piece of the line that place y lies in.
+__host__ __device__ __forceinline__ uint32_t group_of(uint32_t y, uint32_t gdiv) {
+    return (uint32_t)(((uint64_t)y * gdiv) >> 32);
+}
+
+// The groups that end with occupied cell number `at` (slots [o, o + n)): the
+// next cell's place on the line lies in a later piece, so it begins the next
+// group (a cell longer than a piece leaves empty groups behind it).
+__host__ __device__ __forceinline__ void group_ends(GroupDesc *grp, int64_t cap, uint32_t gdiv, uint32_t at, uint32_t o,
+                                                    uint32_t n) {
+    const uint32_t y = o + (uint32_t)kGroupPad * at, y2 = y + n + (uint32_t)kGroupPad;
+    const uint32_t g1 = group_of(y2, gdiv);
+    for (uint32_t g = group_of(y, gdiv) + 1; g <= g1 && (int64_t)g < cap; g++) grp[g] = GroupDesc{at + 1, o + n};
+}
+
+// The first entry and the one after the last group; returns the groups.
+__host__ __device__ __forceinline__ int64_t group_close(GroupDesc *grp, int64_t cap, uint32_t gdiv, uint32_t nocc,
+                                                        uint32_t total) {
+    const uint32_t y = total + (uint32_t)kGroupPad * nocc;
+    const uint32_t ng = nocc ? group_of(y - 1u, gdiv) + 1u : 0u;
+    grp[0] = GroupDesc{0u, 0u};
+    if (ng && (int64_t)ng < cap) grp[ng] = GroupDesc{nocc, total};
+    return (int64_t)ng;
 }
 
 // The inputs of one scan tile for this thread's cell: stayers, arrivals,
@@ -1811,7 +1945,11 @@ __device__ __forceinline__ void tile_write(const CtxT &x, const StepArgs &sa, ui
             x.birth_off[c] = (uint32_t)(run >> 32);
         }
         const uint32_t nn = (uint32_t)I.v;
-        if (nn != 0) x.occ_nxt[orun] = OccCell{(int32_t)c, o, nn, 0u};
+        if (nn != 0) {
+            x.occ_nxt[orun] = OccCell{(int32_t)c, o, nn, 0u};
+            group_ends(x.nxt.grp, x.grp_cap, sa.gdiv, (uint32_t)orun, o, nn);
+            if (nn > (uint32_t)kGroupSlots) x.st->big[1 - sa.parity] = 1;
+        }
     }
     if (threadIdx.x == 0) x.tact[tile] = 0u;
     if (last && threadIdx.x == kScanBlock - 1) {
@@ -1830,6 +1968,7 @@ __device__ __forceinline__ void tile_write(const CtxT &x, const StepArgs &sa, ui
         st->occupied_total += st->n_occ[p];
         st->n_alive[q] = total;
         st->n_occ[q] = (int64_t)orun;
+        st->n_grp[q] = group_close(x.nxt.grp, x.grp_cap, sa.gdiv, (uint32_t)orun, (uint32_t)total);
         st->max_id[q] = st->max_id[p] + B;
         st->gpool[q] = st->gpool[p] + (x.gwords ? B : 0);
         st->births_last = B;
@@ -1952,254 +2091,66 @@ __global__ void __launch_bounds__(kScanBlock) k_cell_scan(Ctx x, StepArgs sa) {
 }
 
 // ---------------------------------------------------------------------------
-// genetics: GeneUtils::makeMultiMask / crossOver / freeReco / mutateNucs
-// (GeneUtils.cpp:112-246, :322-360), one genome word per lane
+// k_cell_scatter: every agent's record to its place in the next buffer
 // ---------------------------------------------------------------------------
+// an agent's record as it leaves the current buffer
+struct ScatItem {
+    uint64_t w;               // outcome word
+    int64_t id, mate;
+    double birth, age, lastb;
+    int32_t gmate, nbab, gh;
+    uint8_t life, g;
+};
 
-
-
-// ---------------------------------------------------------------------------
-// k_cell_scatter: agents of one occupied source cell to the next buffer
-// ---------------------------------------------------------------------------
 template <typename CtxT>
-__device__ __forceinline__ void cell_scatter(const CtxT &x, const StepArgs &sa, int32_t c, uint32_t s, int32_t n,
-                                             int32_t *mli, int64_t *mid, int64_t max_id, int64_t gbase) {
-    const int lane = threadIdx.x;
-    const uint64_t lt = lanemask_lt();
-    const uint32_t nbase = x.off_nxt[c];
-    const uint32_t bp = x.bpos[c];
-    const uint32_t boff = x.birth_off[c];
-    uint32_t rp[6];
-#pragma unroll
-    for (int d = 0; d < 6; d++) rp[d] = (d < x.conn) ? x.rpos[(int64_t)c * x.conn + d] : 0u;
-    uint32_t nstay = 0, nmoth = 0;
-    uint32_t nrun[6] = {0, 0, 0, 0, 0, 0};
-    for (int32_t b = 0; b < n; b += kWave) {
-        const int32_t li = b + lane;
-        const bool valid = li < n;
-        const uint32_t from = s + (uint32_t)li;
-        uint8_t code = kDecDead;
-        int64_t id = 0, mate = 0;
-        uint8_t life = 0, g = 0;
-        double birth = 0, age = 0, lastb = 0;
-        int32_t nbab = 0, gh = 0;
-        if (valid) {
-            code = x.dec[from];
-            id = x.cur.id[from];
-            mate = x.cur.mate_id[from];
-            life = x.cur.life[from];
-            g = x.cur.gender[from];
-            birth = x.cur.birth[from];
-            age = x.cur.age[from];
-            lastb = x.cur.lastb[from];
-            nbab = x.cur.nbabies[from];
-            if (x.gwords) gh = x.cur.ghandle[from];
-        }
-        const bool alive = valid && !(code & kDecDead);
-        const uint32_t dir = code & kDecDirMask;
-        int64_t to = -1;
-        const uint64_t ms = __ballot(alive && dir == 0);
-        if (alive && dir == 0) to = (int64_t)nbase + nstay + __popcll(ms & lt);
-        nstay += __popcll(ms);
-#pragma unroll
-        for (int d = 0; d < 6; d++) {
-            const bool mine = alive && dir == (uint32_t)(d + 1);
-            const uint64_t mm = __ballot(mine);
-            if (mine) to = (int64_t)rp[d] + nrun[d] + __popcll(mm & lt);
-            nrun[d] += __popcll(mm);
-        }
-        if (alive && dir == kDecNav) {
-            // a Navigate edge's run: its slot and the rank k_cell_act gave it
-            const uint64_t ns = x.nav.sel[from];
-            to = (int64_t)x.nav.rpos[(uint32_t)ns] + (uint32_t)(ns >> 32);
-        }
-        if (to >= 0) {
-            x.nxt.id[to] = id;
-            x.nxt.mate_id[to] = mate;
-            x.nxt.life[to] = life;
-            x.nxt.gender[to] = g;
-            x.nxt.birth[to] = birth;
-            x.nxt.age[to] = age;
-            x.nxt.lastb[to] = lastb;
-            x.nxt.nbabies[to] = nbab;
-            if (x.gwords) x.nxt.ghandle[to] = gh;
-        }
-        const bool isb = valid && (code & kDecBirth);
-        const uint64_t mb = __ballot(isb);
-        if (isb) {
-            const uint32_t at = nmoth + __popcll(mb & lt);
-            mli[at] = li;
-            mid[at] = id;
-        }
-        nmoth += __popcll(mb);
-    }
-    if (nmoth == 0) return;
-    wave_sync();
-    // newborns in mother-id order: createAgentAtIndex + makePopSpecificOffspring
-    // (SPopulation.cpp:880-918); new ids rank births by (cell, mother id)
-    for (uint32_t j = lane; j < nmoth; j += kWave) {
-        const int64_t my = mid[j];
-        uint32_t r = 0;
-        for (uint32_t k = 0; k < nmoth; k++) r += mid[k] < my;
-        const int64_t to = (int64_t)bp + r;
-        const int64_t rg = (int64_t)boff + r;
-        const int64_t nid = max_id + 1 + rg;
-        x.nxt.id[to] = nid;
-        x.nxt.mate_id[to] = -3;
-        x.nxt.birth[to] = sa.t;
-        x.nxt.age[to] = 0.0;
-        x.nxt.lastb[to] = 0.0;
-        x.nxt.nbabies[to] = 0;
-        const uint32_t u = draw(x.seed, sa.step, QHG_STREAM_NEWBORN, (uint64_t)nid, 0);
-        const uint8_t gg = (uint8_t)(2 * wrandd(u));
-        x.nxt.gender[to] = gg;
-        x.nxt.life[to] = (gg == 0) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
-        if (x.gwords) {
-            const uint32_t mslot = s + (uint32_t)mli[j];
-            x.nxt.ghandle[to] = (int32_t)(gbase + rg);
-            x.brec[2 * rg] = (int32_t)mslot;
-            x.brec[2 * rg + 1] = x.bfather[mslot];
-        }
-    }
-    wave_sync();
+__device__ __forceinline__ void scatter_load(const CtxT &x, const StepArgs &sa, int64_t i, ScatItem &a) {
+    a.w = x.dec[i];
+    a.gmate = -1;
+    a.mate = -3;
+    a.life = 0;
+    a.age = 0;
+    a.gh = 0;
+    if (sa.mates) a.gmate = x.gmate[i];
+    else a.mate = x.cur.mate_id[i];
+    a.id = x.cur.id[i];
+    a.birth = x.cur.birth[i];
+    a.lastb = x.cur.lastb[i];
+    a.g = x.cur.gender[i];
+    a.nbab = x.cur.nbabies[i];
+    if (!sa.sets_age) a.age = x.cur.age[i];
+    if (!sa.sets_life) a.life = x.cur.life[i];
+    if (x.gwords) a.gh = x.cur.ghandle[i];
 }
 
-enum { kScStay = 0, kScMv = 1, kScMoth = 7, kScN = 8 };
-
-struct GroupScatLds {
-    int64_t mid[kGroupSlots];                 // ids of the mothers, per cell region
-    uint32_t cnt[kGroupCells][kScN];          // per-cell running counts
-    int16_t mj[kGroupSlots];                  // group positions of the mothers
-};
-
-struct CellScatLds {
-    int32_t mli[kLdsCell];
-    int64_t mid[kLdsCell];
-};
-
-union ScatLds {
-    GroupScatLds g;
-    CellScatLds c;
-};
-
-// all cells of a group (see group_act): stayers and movers ranked per cell
-// and run by masked ballots, running counts across chunks in LDS
+// One agent, and its newborn: createAgentAtIndex + makePopSpecificOffspring
+// (SPopulation.cpp:880-918); new ids rank births by (cell, mother id).
 template <typename CtxT>
-__device__ __forceinline__ void group_scatter(const CtxT &x, const StepArgs &sa, int ng, const OccCell &e,
-                                              uint32_t eb, uint32_t S0, uint32_t T, GroupScatLds &G,
+__device__ __forceinline__ void scatter_agent(const CtxT &x, const StepArgs &sa, int64_t i, const ScatItem &a,
                                               int64_t max_id, int64_t gbase) {
-    const int lane = threadIdx.x;
-    const uint64_t lt = lanemask_lt();
-    const int nchunks = (int)((T + kWave - 1) / kWave);
-    // the cells' newborn positions and birth ranks, read now so the newborn
-    // pass below needs no round trip of its own (values of cells without
-    // births are stale and unused)
-    uint32_t cb_pos = 0, cb_off = 0;
-    if (lane < ng) {
-#pragma unroll
-        for (int q = 0; q < kScN; q++) G.cnt[lane][q] = 0;
-        cb_pos = x.bpos[e.c];
-        cb_off = x.birth_off[e.c];
+    const uint32_t kind = (uint32_t)(a.w >> kDecKindAt) & 3u;
+    const bool birth = (a.w & kDecBirth) != 0;
+    uint64_t br = 0;
+    if (birth) br = x.brank[i];
+    if (kind != kDecDead) {
+        const uint32_t *table = (kind == kDecStay) ? x.off_nxt : (kind == kDecMove) ? x.rpos : x.nav.rpos;
+        const uint32_t at = table[(uint32_t)a.w];
+        int64_t mate = a.mate;
+        if (sa.mates && a.gmate >= 0) mate = x.cur.id[a.gmate];
+        const int64_t to = (int64_t)at + ((uint32_t)(a.w >> kDecRankAt) & kDecRankMask);
+        x.nxt.id[to] = a.id;
+        x.nxt.birth[to] = a.birth;
+        x.nxt.age[to] = sa.sets_age ? sa.t - a.birth : a.age;
+        x.nxt.lastb[to] = a.lastb;
+        x.nxt.nbabies[to] = a.nbab + ((birth && !(a.w & kDecCounted)) ? 1 : 0);
+        x.nxt.gender[to] = a.g;
+        x.nxt.life[to] = !sa.sets_life ? a.life : (a.w & kDecFertile) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
+        if (x.gwords) x.nxt.ghandle[to] = a.gh;
+        x.nxt.mate_id[to] = mate;
     }
-    wave_sync();
-    for (int ch = 0; ch < nchunks; ch++) {
-        const uint32_t q = (uint32_t)(ch * kWave + lane);
-        const bool valid = q < T;
-        const uint32_t from = S0 + q;
-        const int k = group_cell_of(q, eb, ng);
-        const int32_t c = __shfl(e.c, k, 64);
-        const uint32_t base = (uint32_t)__shfl((int)eb, k, 64);
-        const uint32_t nk = (uint32_t)__shfl((int)e.n, k, 64);
-        uint8_t code = kDecDead;
-        int64_t id = 0, mate = 0;
-        uint8_t life = 0, g = 0;
-        double birth = 0, age = 0, lastb = 0;
-        int32_t nbab = 0, gh = 0;
-        uint32_t nbase = 0;
-        uint32_t rp[6] = {0, 0, 0, 0, 0, 0};
-        if (valid) {
-            code = x.dec[from];
-            id = x.cur.id[from];
-            mate = x.cur.mate_id[from];
-            life = x.cur.life[from];
-            g = x.cur.gender[from];
-            birth = x.cur.birth[from];
-            age = x.cur.age[from];
-            lastb = x.cur.lastb[from];
-            nbab = x.cur.nbabies[from];
-            if (x.gwords) gh = x.cur.ghandle[from];
-            nbase = x.off_nxt[c];
-#pragma unroll
-            for (int d = 0; d < 6; d++)
-                if (d < x.conn) rp[d] = x.rpos[(int64_t)c * x.conn + d];
-        }
-        // lanes of this lane's cell inside the chunk
-        const int lo = (int)base - ch * kWave;
-        const int hi = (int)(base + nk) - ch * kWave;
-        const uint64_t cm = (valid ? ((hi >= 64) ? ~0ull : ((1ull << hi) - 1ull)) : 0ull) &
-                            ~((lo <= 0) ? 0ull : ((1ull << lo) - 1ull));
-        const bool last_of_cell = valid && ((int)lane == ((hi >= 64) ? 63 : hi - 1));
-        const bool alive = valid && !(code & kDecDead);
-        const uint32_t dir = code & kDecDirMask;
-        int64_t to = -1;
-        const uint64_t ms = __ballot(alive && dir == 0);
-        const uint32_t c_stay = valid ? G.cnt[k][kScStay] : 0u;
-        if (alive && dir == 0) to = (int64_t)nbase + c_stay + __popcll(ms & lt & cm);
-        uint32_t add[7];
-        add[0] = __popcll(ms & cm);
-#pragma unroll
-        for (int d = 0; d < 6; d++) {
-            const bool mine = alive && dir == (uint32_t)(d + 1);
-            const uint64_t mm = __ballot(mine);
-            if (mine) to = (int64_t)rp[d] + G.cnt[k][kScMv + d] + __popcll(mm & lt & cm);
-            add[1 + d] = __popcll(mm & cm);
-        }
-        if (alive && dir == kDecNav) {
-            const uint64_t ns = x.nav.sel[from];
-            to = (int64_t)x.nav.rpos[(uint32_t)ns] + (uint32_t)(ns >> 32);
-        }
-        if (to >= 0) {
-            x.nxt.id[to] = id;
-            x.nxt.mate_id[to] = mate;
-            x.nxt.life[to] = life;
-            x.nxt.gender[to] = g;
-            x.nxt.birth[to] = birth;
-            x.nxt.age[to] = age;
-            x.nxt.lastb[to] = lastb;
-            x.nxt.nbabies[to] = nbab;
-            if (x.gwords) x.nxt.ghandle[to] = gh;
-        }
-        if (valid && (code & kDecBirth)) {
-            const uint32_t r = atomicAdd(&G.cnt[k][kScMoth], 1u);
-            G.mj[base + r] = (int16_t)q;
-            G.mid[base + r] = id;
-        }
-        wave_sync();
-        if (last_of_cell) {
-#pragma unroll
-            for (int d = 0; d < 7; d++) G.cnt[k][kScStay + d] += add[d];
-        }
-        wave_sync();
-    }
-    // newborns in mother-id order per cell: createAgentAtIndex +
-    // makePopSpecificOffspring (SPopulation.cpp:880-918); new ids rank births
-    // by (cell, mother id)
-    for (int ch = 0; ch < nchunks; ch++) {
-        const uint32_t q = (uint32_t)(ch * kWave + lane);
-        const bool valid = q < T;
-        const int k = group_cell_of(q, eb, ng);
-        const uint32_t base = (uint32_t)__shfl((int)eb, k, 64);
-        const uint32_t kpos = (uint32_t)__shfl((int)cb_pos, k, 64);
-        const uint32_t koff = (uint32_t)__shfl((int)cb_off, k, 64);
-        if (!valid) continue;
-        const uint32_t nm = G.cnt[k][kScMoth];
-        const uint32_t t = q - base;
-        if (t >= nm) continue;
-        const int64_t my = G.mid[q];
-        uint32_t r = 0;
-        for (uint32_t u = 0; u < nm; u++) r += G.mid[base + u] < my;
-        const int64_t to = (int64_t)kpos + r;
-        const int64_t rg = (int64_t)koff + r;
+    if (birth) {
+        const uint32_t c = (uint32_t)br, r = (uint32_t)(br >> 32);
+        const int64_t to = (int64_t)x.bpos[c] + r;
+        const int64_t rg = (int64_t)x.birth_off[c] + r;
         const int64_t nid = max_id + 1 + rg;
         x.nxt.id[to] = nid;
         x.nxt.mate_id[to] = -3;
@@ -2212,35 +2163,36 @@ __device__ __forceinline__ void group_scatter(const CtxT &x, const StepArgs &sa,
         x.nxt.gender[to] = gg;
         x.nxt.life[to] = (gg == 0) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
         if (x.gwords) {
-            const uint32_t mslot = S0 + (uint32_t)G.mj[q];
             x.nxt.ghandle[to] = (int32_t)(gbase + rg);
-            x.brec[2 * rg] = (int32_t)mslot;
-            x.brec[2 * rg + 1] = x.bfather[mslot];
+            x.brec[2 * rg] = (int32_t)i;
+            x.brec[2 * rg + 1] = a.gmate;
         }
     }
-    wave_sync();
 }
 
-__global__ void __launch_bounds__(kCellBlock) k_cell_scatter(Ctx x, StepArgs sa) {
-    __shared__ ScatLds lds;
-    const int lane = threadIdx.x;
+// A record's place is its run's first slot plus its place in the run, both
+// ready, so agents need nothing of each other: full waves over the slots,
+// whatever the cells, two dependent round trips (record, run) and the
+// writes.  By cells, with every agent's place from ballots, the kernel took
+// 55 us at 1.39 M agents, 18.4 at 369 k and 6.4 at 6 k; so 41, 12.7 and 5.
+// (Non-temporal stores: 95 and 26; a line is written in pieces, by several
+// waves, and must stay in the cache until it is whole.)
+__global__ void __launch_bounds__(kScatterBlock) k_cell_scatter(Ctx x, StepArgs sa) {
+    const int tid = threadIdx.x, lane = tid & 63;
     const int pr = (int)sa.parity;
-    const int64_t G = gridDim.x - 1;
-    const int64_t b0 = (int64_t)blockIdx.x - 1;
-    // one round trip: the status and this wave's first group (read ahead of
-    // the count check: every index below ncells exists)
+    const int64_t stride = (int64_t)(gridDim.x - 1) * kScatterBlock;
+    int64_t i = ((int64_t)blockIdx.x - 1) * kScatterBlock + tid;
+    // one round trip: the status and this thread's first record (read ahead
+    // of the count check, inside the buffers)
     const int32_t err = x.st->error;
     const int64_t max_id = x.st->max_id[pr];
     const int64_t gbase = x.st->gpool[pr];
-    const int64_t nocc = x.st->n_occ[pr];
-    const int64_t gc = sa.gcells;
-    OccCell e_first{0, 0, 0, 0};
-    {
-        const int64_t idx = b0 * gc + lane;
-        if (b0 >= 0 && lane < gc && idx < x.ncells) e_first = x.occ_cur[idx];
-    }
+    const int64_t n = x.st->n_alive[pr];
+    ScatItem a;
+    if (i >= 0 && i < x.cap) scatter_load(x, sa, i, a);
     if (err) return;
     if (blockIdx.x == 0) {
+        if (tid >= kWave) return;
         // the step's deaths, moves and FERTILE counts (k_cell_scan's per-wave
         // sums) go into the status and the host's snapshot; the status words
         // and the sums load in the same round trip, one word per lane
@@ -2284,29 +2236,16 @@ __global__ void __launch_bounds__(kCellBlock) k_cell_scatter(Ctx x, StepArgs sa)
         }
         return;
     }
-    const int64_t ngroups = (nocc + gc - 1) / gc;
-    for (int64_t gi = b0; gi < ngroups; gi += G) {
-        const int64_t i0 = gi * gc;
-        const int ng = (int)((nocc - i0 < gc) ? (nocc - i0) : gc);
-        OccCell e{0, 0, 0, 0};
-        if (lane < ng) e = (gi == b0) ? e_first : x.occ_cur[i0 + lane];
-        const uint32_t S0 = readlane_u32(e.s, 0);
-        const uint32_t T = readlane_u32(e.s, ng - 1) + readlane_u32(e.n, ng - 1) - S0;
-        if (T <= (uint32_t)kGroupSlots) {
-            group_scatter(x, sa, ng, e, e.s - S0, S0, T, lds.g, max_id, gbase);
-            continue;
-        }
-        for (int k = 0; k < ng; k++) {
-            const int32_t c = (int32_t)readlane_u32((uint32_t)e.c, k);
-            const uint32_t s = readlane_u32(e.s, k);
-            const int32_t n = (int32_t)readlane_u32(e.n, k);
-            // mothers of a large cell go to the cell's own range of global scratch
-            int32_t *mli = (n > kLdsCell) ? x.gfu + s : lds.c.mli;
-            int64_t *mid = (n > kLdsCell) ? x.gfid + s : lds.c.mid;
-            cell_scatter(x, sa, c, s, n, mli, mid, max_id, gbase);
-        }
+    for (bool first = true; i < n; i += stride, first = false) {
+        if (!first) scatter_load(x, sa, i, a);
+        scatter_agent(x, sa, i, a, max_id, gbase);
     }
 }
+
+// ---------------------------------------------------------------------------
+// genetics: GeneUtils::makeMultiMask / crossOver / freeReco / mutateNucs
+// (GeneUtils.cpp:112-246, :322-360), one genome word per lane
+// ---------------------------------------------------------------------------
 
 // bits lo..hi (inclusive, lo <= hi <= 63)
 __device__ __forceinline__ uint64_t bit_range(int lo, int hi) {
@@ -2478,22 +2417,9 @@ struct BatchArgs {
     uint64_t *tiles;          // per tile of every member: agents | births totals
     uint64_t *tiles2;         //   ... and occupied-cell totals (k_batch_scan_sums)
     int64_t *bctr;            // BC_COUNT copies of the batch step index
-    double group_agents;      // target agents per wave group
+    uint32_t gdiv;            // as StepArgs
     int32_t genome;           // k_batch_genome runs in this step
-    int32_t pad;
 };
-
-// values every lane holds alike (ballot and shuffle results), as such
-__device__ __forceinline__ int uniform_i32(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-template <typename T>
-__device__ __forceinline__ T *uniform_ptr(T *p) {
-    return (T *)(uintptr_t)uniform_i64((int64_t)(uintptr_t)p);
-}
 
 __device__ __forceinline__ int64_t batch_step_in(const BatchArgs &B, int k, int next) {
     const int64_t b = uniform_i64(B.bctr[k]);
@@ -2512,22 +2438,10 @@ __host__ __device__ __forceinline__ int32_t scan_dense(int64_t occ, int64_t ncel
     return ((occ << shift) >= ncells) ? 1 : 0;
 }
 
-// cells per wave group: about `target` agents per group from the mean
-// occupancy (results do not depend on it)
-__host__ __device__ __forceinline__ int32_t group_cells(double target, int64_t alive, int64_t occ) {
-    const double o = (double)(occ > 0 ? occ : 1);
-    double mean = (double)alive / o;
-    mean = mean > 1.0 ? mean : 1.0;
-    const double g = floor(target / mean);
-    return (int32_t)(g < 1.0 ? 1.0 : (g > (double)kGroupCells ? (double)kGroupCells : g));
-}
-
 // The descriptor table is written by the host before a launch and by no
 // kernel: read through the constant address space, its fields go to scalar
 // registers (and stay there across the kernels' own stores).
 typedef __attribute__((address_space(4))) const PopDesc ConstPopDesc;
-typedef __attribute__((address_space(4))) const Ctx ConstCtx;
-typedef __attribute__((address_space(4))) const Prog ConstProg;
 
 __device__ __forceinline__ ConstPopDesc &pop_desc(const BatchArgs &B, int r) {
     return ((ConstPopDesc *)B.pops)[r];
@@ -2535,25 +2449,27 @@ __device__ __forceinline__ ConstPopDesc &pop_desc(const BatchArgs &B, int r) {
 
 // A member's step arguments: step and time advance by one per batch step
 // from where the member joined (fixed for the whole batch step, whatever the
-// kernels write into its status); the group size follows its occupancy.
+// kernels write into its status).
 template <typename Desc>
-__device__ __forceinline__ StepArgs pop_step_args(const Desc &d, int64_t bstep, double group_agents) {
+__device__ __forceinline__ StepArgs pop_step_args(const Desc &d, int64_t bstep, uint32_t gdiv) {
     StepArgs a{};
     const int64_t step = d.step0 + (bstep - d.join);
     a.step = (uint32_t)step;
     a.parity = (uint32_t)(step & 1);
     a.t = d.t0 + (double)(bstep - d.join);
     const DevStatus *st = d.ctx[0].st;
-    a.gcells = group_cells(group_agents, st->n_alive[a.parity], st->n_occ[a.parity]);
+    a.gdiv = gdiv;
+    a.mates = (d.prog.k.flags & kActPair) ? 1 : 0;   // assortative populations do not run in batches
+    a.sets_age = d.prog.sets_age;
+    a.sets_life = d.prog.sets_life;
     a.dense = scan_dense(st->n_occ[a.parity], d.ctx[0].ncells, 1);
     return a;
 }
 
 // the same for a member every lane of the wave works on (its values as such)
 template <typename Desc>
-__device__ __forceinline__ StepArgs pop_step_args_uniform(const Desc &d, int64_t bstep, double group_agents) {
-    StepArgs a = pop_step_args(d, bstep, group_agents);
-    a.gcells = uniform_i32(a.gcells);
+__device__ __forceinline__ StepArgs pop_step_args_uniform(const Desc &d, int64_t bstep, uint32_t gdiv) {
+    StepArgs a = pop_step_args(d, bstep, gdiv);
     a.dense = uniform_i32(a.dense);
     return a;
 }
@@ -2589,82 +2505,91 @@ __device__ __forceinline__ int64_t lane_value(const int64_t (&v)[4], int r) {
     return uniform_i64(out);
 }
 
-// per-member group counts of the current step
-__device__ __forceinline__ void batch_groups(const BatchArgs &B, int64_t bstep, int64_t (&cnt)[4]) {
+// Per-member counts of the current step: its groups, or (slots != 0) its
+// agents in runs of that many.  big: bit k, whether lane + 64 k's member may
+// hold a cell larger than a block takes.
+__device__ __forceinline__ void batch_items(const BatchArgs &B, int64_t bstep, int slots, int64_t (&cnt)[4],
+                                            uint32_t &big) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int r = lane + 64 * k;
         cnt[k] = 0;
+        if (k == 0) big = 0;
         if (r < B.npops) {
-            const DevStatus *st = pop_desc(B, r).ctx[0].st;
+            ConstPopDesc &d = pop_desc(B, r);
+            const DevStatus *st = d.ctx[0].st;
             if (!st->error) {
-                const StepArgs a = pop_step_args(pop_desc(B, r), bstep, B.group_agents);
-                const int64_t nocc = st->n_occ[a.parity];
-                cnt[k] = (nocc + a.gcells - 1) / a.gcells;
+                const int par = (int)((d.step0 + (bstep - d.join)) & 1);
+                cnt[k] = slots ? (st->n_alive[par] + slots - 1) / slots : st->n_grp[par];
+                if (!slots && st->big[par]) big |= 1u << k;
             }
         }
     }
 }
 
 template <bool kRare, bool kNav = false>
-__global__ void __launch_bounds__(kCellBlock) k_batch_act(BatchArgs B) {
-    __shared__ ActLds lds;
-    const int lane = threadIdx.x;
+__global__ void __launch_bounds__(kActBlock) k_batch_act(BatchArgs B) {
+    __shared__ GroupActLds lds;
+    __shared__ uint32_t part[kParts];
+    const int tid = threadIdx.x;
     const int64_t bstep = batch_step_in(B, BC_ACT, BC_SCAN);
     int64_t cnt[4], base[4];
-    batch_groups(B, bstep, cnt);
+    uint32_t big;
+    batch_items(B, bstep, 0, cnt, big);
     const int64_t total = pop_prefix(cnt, base);
-    // a contiguous run of groups per block, so a block stays with one member
-    // for long stretches and adds its counts to that member once per stretch
-    const int64_t per = (total + gridDim.x - 1) / gridDim.x;
-    const int64_t g0 = (int64_t)blockIdx.x * per;
-    const int64_t g1 = (g0 + per < total) ? g0 + per : total;
-    // one stretch per member: its context is fixed for the inner loop
-    for (int64_t g = g0; g < g1;) {
-        const int r = pop_of(base, B.npops, g);
-        const int64_t rbase = lane_value(base, r);
-        const int64_t rend0 = rbase + lane_value(cnt, r);
-        const int64_t rend = rend0 < g1 ? rend0 : g1;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.group_agents);
-        ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[sa.parity]);
-        ConstProg &pg = *uniform_ptr(&pop_desc(B, r).prog);
-        const int64_t nocc = uniform_i64(x.st->n_occ[sa.parity]);
-        const int64_t gc = sa.gcells;
-        uint32_t deaths = 0, moves = 0, fert = 0;
-        for (; g < rend; g++) {
-            const int64_t i0 = (g - rbase) * gc;
-            const int ng = (int)((nocc - i0 < gc) ? (nocc - i0) : gc);
-            OccCell e{0, 0, 0, 0};
-            if (lane < ng) e = x.occ_cur[i0 + lane];
-            const uint32_t S0 = readlane_u32(e.s, 0);
-            const uint32_t T = readlane_u32(e.s, ng - 1) + readlane_u32(e.n, ng - 1) - S0;
-            const uint32_t nmax = wave_max_u32(lane < ng ? e.n : 0u);
-            if (T <= (uint32_t)kGroupSlots && nmax <= (uint32_t)kGroupCellMax) {
-                group_act<kRare, false, kNav>(x, pg, sa, ng, e, e.s - S0, S0, T, lds.g, deaths, moves, fert);
-                continue;
-            }
-            for (int k = 0; k < ng; k++) {
-                const int32_t c = (int32_t)readlane_u32((uint32_t)e.c, k);
-                const uint32_t s = readlane_u32(e.s, k);
-                const int32_t n = (int32_t)readlane_u32(e.n, k);
-                PairLists L;
-                if (n > kLdsCell) {
-                    L = PairLists{x.gfu + s, x.gmu + s, x.gfid + s, x.gmid + s, x.gfs + s, x.gms + s,
-                                  x.gmate + s, x.gflag + s};
-                } else {
-                    L = PairLists{lds.c.fu, lds.c.mu, lds.c.fid, lds.c.mid, lds.c.fs, lds.c.ms, lds.c.mate,
-                                  lds.c.flag};
-                }
-                cell_act<kRare, false, kNav>(x, pg, sa, c, s, n, L, deaths, moves, fert);
-            }
+    if (tid < kParts) part[tid] = 0u;
+    if (blockIdx.x == 0)
+        for (int r = tid; r < B.npops; r += kActBlock) {
+            ConstPopDesc &d = pop_desc(B, r);
+            d.ctx[0].st->big[1 - ((d.step0 + (bstep - d.join)) & 1)] = 0;   // k_batch_scan sets it
         }
+    for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
+        const int r = pop_of(base, B.npops, g);
+        const int64_t gl = g - lane_value(base, r);
+        ConstPopDesc *dp = uniform_ptr(&pop_desc(B, r));
+        asm volatile("" : "+s"(dp));   // as act_args: a new pointer for every group
+        const StepArgs sa = pop_step_args_uniform(*dp, bstep, B.gdiv);
+        ConstCtx &x = dp->ctx[sa.parity];
+        const GroupDesc d0 = x.cur.grp[gl], d1 = x.cur.grp[gl + 1];
+        uint32_t deaths = 0, moves = 0, fert = 0;
+        group_act<kRare, false, kNav>(&x, &dp->prog, sa.step, sa.t, d0, d1, lds, deaths, moves, fert);
         const uint64_t dm = wave_sum_u64(((uint64_t)moves << 32) | deaths);
         const uint32_t fe = (uint32_t)wave_sum_u64(fert);
-        if (lane == 0) {
-            atomicAdd((unsigned long long *)&x.st->acc_deaths, (unsigned long long)(uint32_t)dm);
-            atomicAdd((unsigned long long *)&x.st->acc_moves, (unsigned long long)(dm >> 32));
-            atomicAdd((unsigned long long *)&x.st->fertile_total, (unsigned long long)fe);
+        if ((tid & 63) == 0) {
+            if ((uint32_t)dm) atomicAdd(&part[0], (uint32_t)dm);
+            if ((uint32_t)(dm >> 32)) atomicAdd(&part[1], (uint32_t)(dm >> 32));
+            if (fe) atomicAdd(&part[2], fe);
+        }
+        __syncthreads();   // and the group's LDS has been read
+        if (tid < kParts) {
+            unsigned long long *to = (unsigned long long *)(tid == 0   ? &x.st->acc_deaths
+                                                            : tid == 1 ? &x.st->acc_moves
+                                                                       : &x.st->fertile_total);
+            if (part[tid]) atomicAdd(to, (unsigned long long)part[tid]);
+            part[tid] = 0u;
+        }
+    }
+#pragma unroll 1
+    for (int k = 0; k < 4; k++) {
+        uint64_t left = __ballot((big >> k) & 1u);
+        while (left) {
+            const int r = 64 * k + __ffsll((unsigned long long)left) - 1;
+            left &= left - 1ull;
+            ConstPopDesc *dp = uniform_ptr(&pop_desc(B, r));
+            asm volatile("" : "+s"(dp));
+            const StepArgs sa = pop_step_args_uniform(*dp, bstep, B.gdiv);
+            ConstCtx &x = dp->ctx[sa.parity];
+            uint32_t deaths = 0, moves = 0, fert = 0;
+            big_cells<kRare, false, kNav>(x, dp->prog, sa.step, sa.t, uniform_i64(x.st->n_occ[sa.parity]), deaths, moves,
+                                          fert);
+            const uint64_t dm = wave_sum_u64(((uint64_t)moves << 32) | deaths);
+            const uint64_t fe = wave_sum_u64(fert);
+            if ((tid & 63) == 0 && (dm | fe)) {
+                atomicAdd((unsigned long long *)&x.st->acc_deaths, (unsigned long long)(uint32_t)dm);
+                atomicAdd((unsigned long long *)&x.st->acc_moves, (unsigned long long)(dm >> 32));
+                atomicAdd((unsigned long long *)&x.st->fertile_total, (unsigned long long)fe);
+            }
         }
     }
 }
@@ -2689,7 +2614,7 @@ __global__ void __launch_bounds__(kScanBlock) k_batch_scan_sums(BatchArgs B) {
         const int64_t lt = t - lane_value(tb, r);
         const DevStatus *st = pop_desc(B, r).ctx[0].st;
         if (st->error) continue;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.group_agents);
+        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.gdiv);
         const ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[sa.parity]);
         uint64_t tot = 0, otot = 0;
         if (!tile_idle(x, (uint32_t)lt)) {
@@ -2726,7 +2651,7 @@ __global__ void __launch_bounds__(kScanBlock) k_batch_scan(BatchArgs B) {
         const int64_t lt = t - first;
         const DevStatus *st = pop_desc(B, r).ctx[0].st;
         if (st->error) continue;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.group_agents);
+        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.gdiv);
         const ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[sa.parity]);
         if (tile_idle(x, (uint32_t)lt)) continue;
         if (threadIdx.x < 64) {
@@ -2753,11 +2678,11 @@ __global__ void __launch_bounds__(kScanBlock) k_batch_scan(BatchArgs B) {
     }
 }
 
-__global__ void __launch_bounds__(kCellBlock) k_batch_scatter(BatchArgs B) {
-    __shared__ ScatLds lds;
-    const int lane = threadIdx.x;
+__global__ void __launch_bounds__(kScatterBlock) k_batch_scatter(BatchArgs B) {
+    const int tid = threadIdx.x, lane = tid & 63;
     const int64_t bstep = batch_step_in(B, BC_SCATTER, BC_GENOME);
     if (blockIdx.x == 0) {
+        if (tid >= kWave) return;
         // close every member's step and copy its status into host memory,
         // one lane per member
         for (int r = lane; r < B.npops; r += kWave) {
@@ -2792,46 +2717,22 @@ __global__ void __launch_bounds__(kCellBlock) k_batch_scatter(BatchArgs B) {
         }
         return;
     }
-    // the same group numbering as k_batch_act
+    // the members' slots in runs of a block
     int64_t cnt[4], base[4];
-    batch_groups(B, bstep, cnt);
+    uint32_t big;
+    batch_items(B, bstep, kScatterBlock, cnt, big);
     const int64_t total = pop_prefix(cnt, base);
-    const int64_t G = gridDim.x - 1;
-    const int64_t per = (total + G - 1) / G;
-    const int64_t g0 = (int64_t)(blockIdx.x - 1) * per;
-    const int64_t g1 = (g0 + per < total) ? g0 + per : total;
-    // one stretch per member: its context is fixed for the inner loop
-    for (int64_t g = g0; g < g1;) {
+    for (int64_t g = (int64_t)blockIdx.x - 1; g < total; g += gridDim.x - 1) {
         const int r = pop_of(base, B.npops, g);
-        const int64_t rbase = lane_value(base, r);
-        const int64_t rend0 = rbase + lane_value(cnt, r);
-        const int64_t rend = rend0 < g1 ? rend0 : g1;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.group_agents);
-        ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[sa.parity]);
+        const int64_t i = (g - lane_value(base, r)) * kScatterBlock + tid;
+        ConstPopDesc *dp = uniform_ptr(&pop_desc(B, r));
+        const StepArgs sa = pop_step_args_uniform(*dp, bstep, B.gdiv);
+        ConstCtx &x = dp->ctx[sa.parity];
         const DevStatus *st = x.st;
-        const int64_t nocc = uniform_i64(st->n_occ[sa.parity]);
-        const int64_t max_id = uniform_i64(st->max_id[sa.parity]);
-        const int64_t gbase = uniform_i64(st->gpool[sa.parity]);
-        const int64_t gc = sa.gcells;
-        for (; g < rend; g++) {
-            const int64_t i0 = (g - rbase) * gc;
-            const int ng = (int)((nocc - i0 < gc) ? (nocc - i0) : gc);
-            OccCell e{0, 0, 0, 0};
-            if (lane < ng) e = x.occ_cur[i0 + lane];
-            const uint32_t S0 = readlane_u32(e.s, 0);
-            const uint32_t T = readlane_u32(e.s, ng - 1) + readlane_u32(e.n, ng - 1) - S0;
-            if (T <= (uint32_t)kGroupSlots) {
-                group_scatter(x, sa, ng, e, e.s - S0, S0, T, lds.g, max_id, gbase);
-                continue;
-            }
-            for (int k = 0; k < ng; k++) {
-                const int32_t c = (int32_t)readlane_u32((uint32_t)e.c, k);
-                const uint32_t s = readlane_u32(e.s, k);
-                const int32_t n = (int32_t)readlane_u32(e.n, k);
-                int32_t *mli = (n > kLdsCell) ? x.gfu + s : lds.c.mli;
-                int64_t *mid = (n > kLdsCell) ? x.gfid + s : lds.c.mid;
-                cell_scatter(x, sa, c, s, n, mli, mid, max_id, gbase);
-            }
+        if (i < st->n_alive[sa.parity]) {
+            ScatItem a;
+            scatter_load(x, sa, i, a);
+            scatter_agent(x, sa, i, a, st->max_id[sa.parity], st->gpool[sa.parity]);
         }
     }
 }
@@ -2858,7 +2759,7 @@ __global__ void __launch_bounds__(kWave) k_batch_genome(BatchArgs B) {
         const int r = pop_of(base, B.npops, g);
         const int64_t gl = g - lane_value(base, r);
         const DevStatus *st = pop_desc(B, r).ctx[0].st;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.group_agents);
+        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.gdiv);
         const int par = (int)sa.parity;
         ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[par]);
         ConstProg &pg = *uniform_ptr(&pop_desc(B, r).prog);

@@ -57,20 +57,38 @@ const char *kKernelNames[KB_COUNT] = {"k_cell_act", "k_cell_scan",     "k_cell_s
 
 constexpr int kRing = kStatusRing;
 #ifndef QHG_GROUP_AGENTS
-#define QHG_GROUP_AGENTS 64.0     // target agents per wave group
+#define QHG_GROUP_AGENTS 64.0     // target agents per wave
 #endif
 #ifndef QHG_CELL_GRID_PER_CU
-#define QHG_CELL_GRID_PER_CU 16   // k_cell_act / k_cell_scatter blocks per compute unit
+#define QHG_CELL_GRID_PER_CU 16   // k_cell_act / k_cell_scatter blocks per compute unit, at most
 #endif
 
+// Length of the pieces that groups are cut by (pads included), from the mean
+// agents per occupied cell: a group's agents, the last cell's overhang with
+// them, should fit one block (a group that does not takes a second pass).
+// Shorter pieces leave waves idle: with pieces of 252, 189 and 125 the act
+// kernel takes 59, 73 and 101 us at 1.39 M agents (15 per cell).
+uint32_t group_div(double group_agents, int64_t alive, int64_t occ) {
+    const double m = std::max(1.0, (double)alive / (double)std::max<int64_t>(1, occ));
+    double w = (kGroupSlots - 1.3 * m) * (m + kGroupPad) / m;
+    w = std::min({w, kActWaves * group_agents - kGroupPad, (double)kGroupPieceMax});
+    w = std::max(w, (double)kGroupPieceMin);
+    return (uint32_t)(4294967296.0 / std::floor(w));
+}
+
+// entries of a buffer's group list at the shortest pieces
+int64_t group_entries(int64_t cap, int64_t ncells) {
+    return (cap + (int64_t)kGroupPad * std::min(ncells, cap)) / kGroupPieceMin + 3;
+}
+
 void free_agentbuf(AgentBuf &a) {
-    void *ptrs[] = {a.id, a.mate_id, a.life, a.gender, a.birth, a.age, a.lastb, a.nbabies, a.ghandle};
+    void *ptrs[] = {a.id, a.mate_id, a.life, a.gender, a.birth, a.age, a.lastb, a.nbabies, a.ghandle, a.grp};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     a = AgentBuf{};
 }
 
-int alloc_agentbuf(AgentBuf &a, int64_t cap, bool genomes) {
+int alloc_agentbuf(AgentBuf &a, int64_t cap, int64_t ncells, bool genomes) {
     a = AgentBuf{};
     const size_t n = (size_t)cap;
     HIPCHK(hipMalloc(&a.id, n * 8));
@@ -82,6 +100,7 @@ int alloc_agentbuf(AgentBuf &a, int64_t cap, bool genomes) {
     HIPCHK(hipMalloc(&a.lastb, n * 8));
     HIPCHK(hipMalloc(&a.nbabies, n * 4));
     if (genomes) HIPCHK(hipMalloc(&a.ghandle, n * 4));
+    HIPCHK(hipMalloc(&a.grp, (size_t)group_entries(cap, ncells) * sizeof(GroupDesc)));
     return 0;
 }
 
@@ -94,7 +113,9 @@ struct qhg_pop {
     hipStream_t stream = nullptr;
     int device = 0;
     int num_cu = 256;
-    int act_grid = 1, scatter_grid = 1, scan_grid = 1, ntiles = 1;
+    int max_grid = 1;         // blocks of k_cell_act and k_cell_scatter, at most
+    int act_grid = 1;         // blocks of the current step's k_cell_act
+    int scan_grid = 1, ntiles = 1;
     // launch shapes (results do not depend on them)
     double group_agents = QHG_GROUP_AGENTS;
     int blocks_per_cu = QHG_CELL_GRID_PER_CU;
@@ -105,8 +126,9 @@ struct qhg_pop {
     uint32_t *d_off[2] = {nullptr, nullptr};
     OccCell *d_occ[2] = {nullptr, nullptr};   // occupied-cell lists per buffer
     // per-slot step scratch (cap entries)
-    uint8_t *d_dec = nullptr, *d_gflag = nullptr;
-    int32_t *d_bfather = nullptr, *d_brec = nullptr;
+    uint64_t *d_dec = nullptr;
+    uint8_t *d_gflag = nullptr;
+    int32_t *d_brec = nullptr;
     int32_t *d_gfu = nullptr, *d_gmu = nullptr, *d_gfs = nullptr, *d_gms = nullptr, *d_gmate = nullptr;
     int64_t *d_gfid = nullptr, *d_gmid = nullptr;
     uint32_t *d_gprot = nullptr;   // AssortativePair: kProtBudget digests per slot
@@ -153,7 +175,6 @@ struct qhg_pop {
     int32_t *d_nav_in_off = nullptr, *d_nav_in_e = nullptr;
     double *d_nav_stay = nullptr, *d_nav_cum = nullptr;
     uint32_t *d_nav_cnt = nullptr, *d_nav_rpos = nullptr;
-    uint64_t *d_nav_sel = nullptr;   // per slot (slot scratch)
 
     Prog prog{};
     bool has_pair = false, has_me = false, has_cap = false, has_assort = false;
@@ -163,6 +184,7 @@ struct qhg_pop {
     bool me_done = false;
     bool acted = false;       // k_cell_act launched for the current step
     bool initialized = false; // initialize phase done for the current step
+    bool looked = false;      // the current step's outcomes were written into the records (k_act_commit)
     double t_next = 0.0;      // time of the next step
 
     // asynchronous status readback ring
@@ -212,8 +234,9 @@ struct qhg_pop {
         x.ice = d_ice;
         x.in_e = d_in_e;
         x.in_w = in_w;
+        x.grp_cap = group_entries(cap, ncells);
         x.dec = d_dec;
-        x.bfather = d_bfather;
+        x.brank = reinterpret_cast<uint64_t *>(d_gmid);   // the lists of k_cell_act are done when it is written
         x.brec = d_brec;
         x.gfu = d_gfu;
         x.gmu = d_gmu;
@@ -259,7 +282,6 @@ struct qhg_pop {
         x.nav.in_e = d_nav_in_e;
         x.nav.cnt = d_nav_cnt;
         x.nav.rpos = d_nav_rpos;
-        x.nav.sel = d_nav_sel;
         return x;
     }
 
@@ -268,10 +290,11 @@ struct qhg_pop {
         a.step = (uint32_t)steps_enqueued;
         a.parity = (uint32_t)cur();
         a.t = t_next;
-        // cells per wave group from the newest known mean occupancy: about
-        // one wave of agents per group (results do not depend on it)
         const int kb = (int)(known_step & 1);
-        a.gcells = group_cells(group_agents, known.n_alive[kb], known.n_occ[kb]);
+        a.gdiv = group_div(group_agents, known.n_alive[kb], known.n_occ[kb]);
+        a.mates = (has_pair || has_assort) ? 1 : 0;
+        a.sets_age = prog.sets_age;
+        a.sets_life = prog.sets_life;
         a.dense = scan_dense(known.n_occ[kb], ncells, 3);
         return a;
     }
@@ -282,17 +305,21 @@ namespace {
 constexpr int kMaxBlocksPerCu = 32;
 
 void set_shape(qhg_pop *p) {
-    p->act_grid = (int)std::max<int64_t>(1, std::min<int64_t>(p->ncells, (int64_t)p->num_cu * p->blocks_per_cu));
-    p->scatter_grid = p->act_grid;
+    p->max_grid = std::max(1, p->num_cu * p->blocks_per_cu);
+}
+
+// blocks for `items` pieces of work as of the newest known status, with some
+// room for the growth since (the kernels stride over what there is)
+int grid_items(const qhg_pop *p, int64_t items) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>(items + items / 8 + 4, p->max_grid));
 }
 
 // device memory held by a population: agent buffers and slot scratch (cap
 // slots), genome pools, per-cell tables, fixed-size scratch
 int64_t device_bytes(const qhg_pop *p) {
     const int64_t g = p->gwords ? 1 : 0;
-    const int64_t per_slot = 2 * (46 + 4 * g) + 38 + 12 * g + (p->has_prot ? 16 * kProtBudget + 4 : 0) +
-                             (p->has_nav ? 8 : 0);
-    int64_t b = p->cap * per_slot;
+    const int64_t per_slot = 2 * (46 + 4 * g) + 45 + 8 * g + (p->has_prot ? 16 * kProtBudget + 4 : 0);
+    int64_t b = p->cap * per_slot + 2 * group_entries(p->cap, p->ncells) * (int64_t)sizeof(GroupDesc);
     for (int k = 0; k < 2; k++)
         if (p->d_gpool[k]) b += p->gcap * p->gwords * 8;
     const int64_t nc = p->ncells, cn = p->conn;
@@ -421,24 +448,24 @@ int collect_timing(qhg_pop *p) {
 }
 
 void free_slot_scratch(qhg_pop *p) {
-    void *ptrs[] = {p->d_dec, p->d_gflag, p->d_bfather, p->d_brec, p->d_gfu, p->d_gmu, p->d_gfs, p->d_gms,
-                    p->d_gmate, p->d_gfid, p->d_gmid, p->d_gprot, p->d_gnprot, p->d_nav_sel};
+    void *ptrs[] = {p->d_dec, p->d_gflag, p->d_brec, p->d_gfu, p->d_gmu, p->d_gfs, p->d_gms,
+                    p->d_gmate, p->d_gfid, p->d_gmid, p->d_gprot, p->d_gnprot};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
-    p->d_nav_sel = nullptr;
-    p->d_dec = p->d_gflag = nullptr;
-    p->d_bfather = p->d_brec = p->d_gfu = p->d_gmu = p->d_gfs = p->d_gms = p->d_gmate = nullptr;
+    p->d_dec = nullptr;
+    p->d_gflag = nullptr;
+    p->d_brec = p->d_gfu = p->d_gmu = p->d_gfs = p->d_gms = p->d_gmate = nullptr;
     p->d_gfid = p->d_gmid = nullptr;
     p->d_gprot = nullptr;
     p->d_gnprot = nullptr;
 }
 
-// per-slot scratch: outcome bytes, birth records, and the list scratch of
+// per-slot scratch: outcome words, birth records, and the list scratch of
 // cells too large for LDS (indexed by segment slot, so cells never overlap)
 int alloc_slot_scratch(qhg_pop *p, int64_t cap) {
     free_slot_scratch(p);
     const size_t n = (size_t)cap;
-    HIPCHK(hipMalloc(&p->d_dec, n));
+    HIPCHK(hipMalloc(&p->d_dec, n * 8));
     HIPCHK(hipMalloc(&p->d_gflag, n));
     HIPCHK(hipMalloc(&p->d_gfu, n * 4));
     HIPCHK(hipMalloc(&p->d_gmu, n * 4));
@@ -447,15 +474,11 @@ int alloc_slot_scratch(qhg_pop *p, int64_t cap) {
     HIPCHK(hipMalloc(&p->d_gmate, n * 4));
     HIPCHK(hipMalloc(&p->d_gfid, n * 8));
     HIPCHK(hipMalloc(&p->d_gmid, n * 8));
-    if (p->gwords) {
-        HIPCHK(hipMalloc(&p->d_bfather, n * 4));
-        HIPCHK(hipMalloc(&p->d_brec, n * 8));
-    }
+    if (p->gwords) HIPCHK(hipMalloc(&p->d_brec, n * 8));
     if (p->has_prot) {
         HIPCHK(hipMalloc(&p->d_gprot, n * 16 * kProtBudget));
         HIPCHK(hipMalloc(&p->d_gnprot, n * 4));
     }
-    if (p->has_nav) HIPCHK(hipMalloc(&p->d_nav_sel, n * 8));
     return 0;
 }
 
@@ -486,26 +509,40 @@ int build_prog(qhg_pop *p) {
     });
     Prog &g = p->prog;
     g = Prog{};
-    g.nops = P.num_actions;
+    ActConst &k = g.k;
     bool seen_getold = false;
     for (int q = 0; q < P.num_actions; q++) {
-        const int k = P.action_kind[idx[q]];
-        if (k < QHG_ACT_GETOLD || k > QHG_ACT_LAST) return fail(QHG_ERR_ARG, "unknown action kind");
-        g.ops[q] = k;
-        g.opword |= (uint64_t)k << (4 * q);
+        const int kind = P.action_kind[idx[q]];
+        if (kind < QHG_ACT_GETOLD || kind > QHG_ACT_LAST) return fail(QHG_ERR_ARG, "unknown action kind");
         // actions that set the age before Fertility reads it
-        if (k == QHG_ACT_GETOLD || k == QHG_ACT_OLDAGEDEATH || k == QHG_ACT_ATANDEATH) seen_getold = true;
-        if (k == QHG_ACT_FERTILITY && !seen_getold) g.load_age = 1;
+        if (kind == QHG_ACT_GETOLD || kind == QHG_ACT_OLDAGEDEATH || kind == QHG_ACT_ATANDEATH) seen_getold = true;
+        switch (kind) {
+        case QHG_ACT_GETOLD: k.flags |= kActBirth; g.sets_age = 1; break;
+        case QHG_ACT_FERTILITY:
+            k.flags |= kActLastb | (seen_getold ? 0u : kActAge);
+            g.sets_life = 1;
+            break;
+        case QHG_ACT_VERHULST: k.flags |= kActDraw0 | kActVerh; break;
+        case QHG_ACT_VERHULSTVARK: k.flags |= kActDraw0 | kActVarK; break;
+        case QHG_ACT_RANDOMMOVE: k.flags |= kActDraw1; break;
+        case QHG_ACT_WEIGHTEDMOVE: k.flags |= kActDraw0; break;
+        case QHG_ACT_OLDAGEDEATH:
+        case QHG_ACT_ATANDEATH: k.flags |= kActBirth | kActDraw1; g.sets_age = 1; break;
+        case QHG_ACT_NAVIGATE: break;
+        default: continue;   // RandomPair, the assortative pairings, MultiEvaluator, NPPCapacity, Genetics: no execute
+        }
+        k.opword |= (uint64_t)kind << (4 * k.nops++);
     }
-    g.fert_min = P.fert_min_age;
-    g.fert_max = P.fert_max_age;
-    g.fert_inter = P.fert_interbirth;
-    g.b0 = P.verh_b0;
-    g.d0 = P.verh_d0;
-    g.theta = P.verh_theta;
-    g.Kconst = P.verh_K;
-    g.rmove_p = P.rmove_prob;
-    g.wmove_p = P.wmove_prob;
+    k.fert_min = P.fert_min_age;
+    k.fert_max = P.fert_max_age;
+    k.fert_inter = P.fert_interbirth;
+    k.b0 = P.verh_b0;
+    k.d0 = P.verh_d0;
+    k.b1 = P.verh_theta - P.verh_b0;
+    k.d1 = P.verh_theta - P.verh_d0;
+    k.Kconst = P.verh_K;
+    k.rmove_p = P.rmove_prob;
+    k.wmove_p = P.wmove_prob;
     g.oad_max = P.oad_max_age;
     g.oad_unc = P.oad_uncertainty;
     g.atan_max = P.atan_max_age;
@@ -531,28 +568,13 @@ int build_prog(qhg_pop *p) {
         g.assort_cutoff = (float)P.assort_cutoff;
         g.assort_permute = P.assort_permute != 0;
         g.assort_prot = p->has_prot ? 1 : 0;
-        g.has_assort = 1;
-        g.need_gender = 1;   // k_cell_act counts the FERTILE agents by sex
     }
     p->has_me = has_kind(P, QHG_ACT_MULTIEVAL);
     p->has_cap = has_kind(P, QHG_ACT_NPPCAP);
     p->has_nav = has_kind(P, QHG_ACT_NAVIGATE);
     p->has_rare = has_kind(P, QHG_ACT_OLDAGEDEATH) || has_kind(P, QHG_ACT_ATANDEATH);
     g.nav_bridge_p = P.nav_bridge_prob;
-    g.has_pair = p->has_pair;
-    for (int q = 0; q < g.nops; q++) {
-        switch (g.ops[q]) {
-        case QHG_ACT_GETOLD: g.need_birth = 1; break;
-        case QHG_ACT_FERTILITY: g.need_gender = 1; g.need_lastb = 1; break;
-        case QHG_ACT_VERHULST:
-        case QHG_ACT_VERHULSTVARK: g.need_gender = 1; g.need_act0 = 1; break;
-        case QHG_ACT_RANDOMMOVE: g.need_act1 = 1; break;
-        case QHG_ACT_WEIGHTEDMOVE: g.need_act0 = 1; break;
-        case QHG_ACT_OLDAGEDEATH:
-        case QHG_ACT_ATANDEATH: g.need_birth = 1; g.need_act1 = 1; break;
-        default: break;
-        }
-    }
+    if (p->has_pair) k.flags |= kActPair;
     if (has_kind(P, QHG_ACT_GENETICS)) {
         if (P.gen_genome_size <= 0 || P.gen_genome_size > 64 * 32) return fail(QHG_ERR_ARG, "Genetics_genome_size out of range");
         if (P.gen_num_crossover < -1 || P.gen_num_crossover > kMaxCross) return fail(QHG_ERR_ARG, "Genetics_num_crossover out of range");
@@ -935,6 +957,18 @@ int read_agents_sorted(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
     return 0;
 }
 
+// A caller may read the agents inside a step (partners paired, outcomes
+// decided, nothing committed): write what is decided so far into their records.
+int look_inside(qhg_pop *p) {
+    const int what = ((p->acted && p->has_pair) || ((p->acted || p->initialized) && p->has_assort) ? 1 : 0) |
+                     (p->acted ? 2 : 0);
+    if (!what || (p->looked && p->acted)) return 0;
+    hipLaunchKernelGGL(k_act_commit, dim3(p->num_cu * 4), dim3(256), 0, p->stream, p->ctx(), p->step_args(), what);
+    HIPCHK(hipGetLastError());
+    p->looked = p->acted;
+    return 0;
+}
+
 // Genome pool compaction in stream order: the genomes of the current
 // buffer's agents move to handles 0..n-1 of the other pool (reallocated to
 // new_gcap first when that differs).
@@ -973,12 +1007,14 @@ int grow_agents(qhg_pop *p, int64_t new_cap, int64_t n) {
     const int b = p->cur();
     AgentBuf nb[2];
     for (int k = 0; k < 2; k++) {
-        int rc = alloc_agentbuf(nb[k], new_cap, p->gwords != 0);
+        int rc = alloc_agentbuf(nb[k], new_cap, p->ncells, p->gwords != 0);
         if (rc) { free_agentbuf(nb[0]); free_agentbuf(nb[1]); return rc; }
     }
     const AgentBuf &o = p->buf[b];
     hipStream_t s = p->stream;
     const size_t m = (size_t)n;
+    HIPCHK(hipMemcpyAsync(nb[b].grp, o.grp, (size_t)group_entries(p->cap, p->ncells) * sizeof(GroupDesc),
+                          hipMemcpyDeviceToDevice, s));
     if (m > 0) {
         HIPCHK(hipMemcpyAsync(nb[b].id, o.id, m * 8, hipMemcpyDeviceToDevice, s));
         HIPCHK(hipMemcpyAsync(nb[b].mate_id, o.mate_id, m * 8, hipMemcpyDeviceToDevice, s));
@@ -1165,7 +1201,8 @@ int phase_initialize(qhg_pop *p) {
     }
     if (p->has_assort) {
         // AssortativePairHam::initialize pairs in the initialize phase
-        rc = launch_bs(p, KB_ASSORT, k_assort_pair, p->act_grid, kWave, p->ctx(), p->prog, p->step_args());
+        const int grid = (int)std::min<int64_t>(p->ncells, (int64_t)p->max_grid);
+        rc = launch_bs(p, KB_ASSORT, k_assort_pair, grid, kWave, p->ctx(), p->prog, p->step_args());
         if (rc) return rc;
     }
     p->initialized = true;
@@ -1183,9 +1220,11 @@ int phase_act(qhg_pop *p) {
                                           : (p->has_assort ? k_cell_act_nav<false, true> : k_cell_act_nav<false, false>))
               : p->has_rare ? (p->has_assort ? k_cell_act<true, true> : k_cell_act<true, false>)
                             : (p->has_assort ? k_cell_act<false, true> : k_cell_act<false, false>);
-    int rc = launch_bs(p, KB_ACT, kern, p->act_grid, kCellBlock, p->ctx(), p->prog, p->step_args());
+    p->act_grid = grid_items(p, p->known.n_grp[p->known_step & 1]);
+    int rc = launch_bs(p, KB_ACT, kern, p->act_grid, kActBlock, ActArgs{p->ctx(), p->prog, p->step_args()});
     if (rc) return rc;
     p->acted = true;
+    p->looked = false;
     return 0;
 }
 
@@ -1200,8 +1239,9 @@ int phase_finalize(qhg_pop *p) {
     int rc = (p->scan_grid >= p->ntiles) ? launch_bs(p, KB_SCAN, k_cell_scan<true>, p->scan_grid, kScanBlock, x, sa)
                                          : launch_bs(p, KB_SCAN, k_cell_scan<false>, p->scan_grid, kScanBlock, x, sa);
     if (rc) return rc;
-    // one more block than the groups use: the step's bookkeeping
-    rc = launch_bs(p, KB_SCATTER, k_cell_scatter, p->scatter_grid + 1, kCellBlock, x, sa);
+    // one more block than the agents use: the step's bookkeeping
+    const int64_t runs = (p->known.n_alive[p->known_step & 1] + kScatterBlock - 1) / kScatterBlock;
+    rc = launch_bs(p, KB_SCATTER, k_cell_scatter, grid_items(p, runs) + 1, kScatterBlock, x, sa);
     if (rc) return rc;
     if (p->gwords) {
         rc = launch_bs(p, KB_GENOME, k_genome, p->num_cu * 16, kWave, x, p->prog, sa);
@@ -1303,8 +1343,8 @@ int qhg_gpu_create(const qhg_grid_desc *grid, const qhg_env_desc *env, const qhg
     capacity = (capacity + 255) / 256 * 256;
 #define CK(x) do { int r_ = (x); if (r_) return cleanup_fail(r_); } while (0)
     p->cap = capacity;
-    CK(alloc_agentbuf(p->buf[0], capacity, p->gwords != 0));
-    CK(alloc_agentbuf(p->buf[1], capacity, p->gwords != 0));
+    CK(alloc_agentbuf(p->buf[0], capacity, p->ncells, p->gwords != 0));
+    CK(alloc_agentbuf(p->buf[1], capacity, p->ncells, p->gwords != 0));
     CK(alloc_slot_scratch(p, capacity));
     if (p->gwords) {
         p->gcap = capacity;
@@ -1428,9 +1468,9 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
         while (nc < 2 * n + 1024) nc *= 2;
         free_agentbuf(p->buf[0]);
         free_agentbuf(p->buf[1]);
-        int rc = alloc_agentbuf(p->buf[0], nc, p->gwords != 0);
+        int rc = alloc_agentbuf(p->buf[0], nc, p->ncells, p->gwords != 0);
         if (rc) return rc;
-        rc = alloc_agentbuf(p->buf[1], nc, p->gwords != 0);
+        rc = alloc_agentbuf(p->buf[1], nc, p->ncells, p->gwords != 0);
         if (rc) return rc;
         rc = alloc_slot_scratch(p, nc);
         if (rc) return rc;
@@ -1474,6 +1514,11 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
         if (off[(size_t)c + 1] > 0) occ.push_back(OccCell{c, off[c], off[(size_t)c + 1], 0u});
         off[(size_t)c + 1] += off[c];
     }
+    const uint32_t gdiv = group_div(p->group_agents, n, (int64_t)occ.size());
+    const int64_t grp_cap = group_entries(p->cap, p->ncells);
+    std::vector<GroupDesc> grp((size_t)grp_cap, GroupDesc{0u, 0u});
+    for (size_t k = 0; k < occ.size(); k++) group_ends(grp.data(), grp_cap, gdiv, (uint32_t)k, occ[k].s, occ[k].n);
+    const int64_t ngrp = group_close(grp.data(), grp_cap, gdiv, (uint32_t)occ.size(), (uint32_t)n);
     const int b = p->cur();
     const size_t ncz = (size_t)p->ncells;
     HIPCHK(hipMemsetAsync(p->d_cstay, 0, (ncz + 2) * 4, p->stream));
@@ -1487,6 +1532,7 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
     const AgentBuf &d = p->buf[b];
     hipStream_t s = p->stream;
     HIPCHK(hipMemcpyAsync(p->d_off[b], off.data(), off.size() * 4, hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(d.grp, grp.data(), (size_t)(ngrp + 1) * sizeof(GroupDesc), hipMemcpyHostToDevice, s));
     if (n > 0) {
         HIPCHK(hipMemcpyAsync(d.id, id.data(), n * 8, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(d.mate_id, mate.data(), n * 8, hipMemcpyHostToDevice, s));
@@ -1509,6 +1555,9 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
     st.n_occ[b] = (int64_t)occ.size();
     st.max_id[b] = max_id;
     st.gpool[b] = p->gwords ? n : 0;
+    st.n_grp[b] = ngrp;
+    st.big[b] = 0;
+    for (const OccCell &e : occ) st.big[b] |= e.n > (uint32_t)kGroupSlots ? 1 : 0;
     st.step = p->steps_enqueued;
     st.error = 0;
     HIPCHK(hipMemcpyAsync(p->d_st, &st, sizeof(st), hipMemcpyHostToDevice, s));
@@ -1543,6 +1592,8 @@ int qhg_gpu_set_clock(qhg_pop *p, int64_t step, double t, int64_t max_id) {
         std::swap(st.n_occ[0], st.n_occ[1]);
         std::swap(st.max_id[0], st.max_id[1]);
         std::swap(st.gpool[0], st.gpool[1]);
+        std::swap(st.n_grp[0], st.n_grp[1]);
+        std::swap(st.big[0], st.big[1]);
     }
     st.max_id[nb] = std::max(st.max_id[nb], max_id);
     st.step = step;
@@ -1591,6 +1642,8 @@ int qhg_gpu_download_agents(qhg_pop *p, qhg_agents *a) {
     if (rc) return rc;
     const int b = p->cur();
     const int64_t n = s.n_alive[b];
+    rc = look_inside(p);
+    if (rc) return rc;
     if (n > 0) {
         rc = s.max_id[b] < kRankIdLimit ? read_agents_ranked(p, s, a) : QHG_ERR_NOMEM;
         if (rc == QHG_ERR_NOMEM) {
@@ -1609,6 +1662,8 @@ int qhg_gpu_state_digest(qhg_pop *p, uint64_t out[3]) {
     int rc = read_status_sync(p, &s);
     if (rc) return rc;
     const int b = p->cur();
+    rc = look_inside(p);
+    if (rc) return rc;
     if (!p->d_digest) HIPCHK(hipMalloc(&p->d_digest, 2 * sizeof(unsigned long long)));
     HIPCHK(hipMemsetAsync(p->d_digest, 0, 2 * sizeof(unsigned long long), p->stream));
     const int64_t nocc = s.n_occ[b];
@@ -1729,6 +1784,7 @@ int qhg_gpu_env_event(qhg_pop *p, const qhg_env_desc *env, int32_t events) {
             uint32_t *src_s = reinterpret_cast<uint32_t *>(p->d_tmp);
             rc = launch_bs(p, KB_CAPACITY, k_env_kill, 1, kKillBlock, (const OccCell *)p->d_occ[b], st.n_occ[b],
                            (const double *)p->d_env[0], (const uint8_t *)p->d_ice, p->d_occ[1 - b], src_s,
+                           p->buf[1 - b].grp, group_entries(p->cap, p->ncells), p->step_args().gdiv,
                            p->d_st, b);
             if (rc) return rc;
             rc = launch(p, KB_CAPACITY, k_env_move, grid_for(st.n_occ[b] * kWave, 4096), p->buf[b], p->buf[1 - b],
@@ -1745,6 +1801,8 @@ int qhg_gpu_env_event(qhg_pop *p, const qhg_env_desc *env, int32_t events) {
             std::swap(st.n_occ[0], st.n_occ[1]);
             std::swap(st.max_id[0], st.max_id[1]);
             std::swap(st.gpool[0], st.gpool[1]);
+            std::swap(st.n_grp[0], st.n_grp[1]);
+            std::swap(st.big[0], st.big[1]);
             HIPCHK(hipMemcpyAsync(p->d_st, &st, sizeof(st), hipMemcpyHostToDevice, p->stream));
             HIPCHK(hipStreamSynchronize(p->stream));
             p->known = st;
@@ -2026,6 +2084,7 @@ struct qhg_batch {
     int device = 0;
     int num_cu = 256;
     int scan_grid = 1, genome_grid = 1;
+    int act_per_cu[3] = {1, 1, 1};   // blocks of the act kernels (plain, age deaths, Navigate) a CU holds
     std::vector<qhg_pop *> pops;
     std::vector<int64_t> gens, step0, join;
     std::vector<double> t0;
@@ -2041,6 +2100,7 @@ struct qhg_batch {
     int64_t *d_bctr = nullptr;     // the kernels' copies of the batch step index
     // launch shapes (results do not depend on them)
     double group_agents = QHG_GROUP_AGENTS;
+    uint32_t gdiv = 0;             // the members' group cuts, as of the last table
     int blocks_per_cu = QHG_CELL_GRID_PER_CU;
     // one step captured as a graph, replayed while the launch set is unchanged
     bool use_graph = false;
@@ -2087,28 +2147,35 @@ BatchArgs batch_args(const qhg_batch *b) {
     A.tiles = b->d_tiles;
     A.tiles2 = b->d_tiles2;
     A.bctr = b->d_bctr;
-    A.group_agents = b->group_agents;
+    A.gdiv = b->gdiv;
     A.genome = b->any_genetics ? 1 : 0;
     return A;
 }
 
-int batch_act_grid(const qhg_batch *b) { return b->num_cu * b->blocks_per_cu; }
+// every block works out the members' shares before its first group, so no more
+// blocks than are resident at once (256 CUs x 16 blocks against 3: 101 us
+// against 56 for 24 members of 931 k agents)
+int batch_act_grid(const qhg_batch *b) {
+    const int k = b->any_nav ? 2 : b->any_death ? 1 : 0;
+    return b->num_cu * std::min(b->blocks_per_cu, b->act_per_cu[k]);
+}
 
 // the kernels of one batch step, in order
 int batch_launch_step(qhg_batch *b) {
     const BatchArgs A = batch_args(b);
     const int ag = batch_act_grid(b);
-    int rc = b->any_nav     ? blaunch(b, BK_ACT, k_batch_act<true, true>, ag, kCellBlock, A)
-             : b->any_death ? blaunch(b, BK_ACT, k_batch_act<true>, ag, kCellBlock, A)
-                            : blaunch(b, BK_ACT, k_batch_act<false>, ag, kCellBlock, A);
+    const int cg = b->num_cu * b->blocks_per_cu;
+    int rc = b->any_nav     ? blaunch(b, BK_ACT, k_batch_act<true, true>, ag, kActBlock, A)
+             : b->any_death ? blaunch(b, BK_ACT, k_batch_act<true>, ag, kActBlock, A)
+                            : blaunch(b, BK_ACT, k_batch_act<false>, ag, kActBlock, A);
     if (rc) return rc;
     const int sg = std::max(1, std::min(b->scan_grid, b->total_tiles));
     rc = blaunch(b, BK_SCAN_SUMS, k_batch_scan_sums, sg, kScanBlock, A);
     if (rc) return rc;
     rc = blaunch(b, BK_SCAN, k_batch_scan, sg, kScanBlock, A);
     if (rc) return rc;
-    // one more block than the groups use: the members' bookkeeping
-    rc = blaunch(b, BK_SCATTER, k_batch_scatter, ag + 1, kCellBlock, A);
+    // one more block than the agents use: the members' bookkeeping
+    rc = blaunch(b, BK_SCATTER, k_batch_scatter, cg + 1, kScatterBlock, A);
     if (rc) return rc;
     if (b->any_genetics) return blaunch(b, BK_GENOME, k_batch_genome, b->genome_grid, kWave, A);
     return 0;
@@ -2192,8 +2259,11 @@ int batch_upload_table(qhg_batch *b) {
     b->any_genetics = false;
     b->any_death = false;
     b->any_nav = false;
+    int64_t alive = 0, occ = 0;
     for (size_t i = 0; i < n; i++) {
         qhg_pop *p = b->pops[i];
+        alive += p->known.n_alive[p->known_step & 1];
+        occ += p->known.n_occ[p->known_step & 1];
         for (int par = 0; par < 2; par++) {
             desc[i].ctx[par] = p->ctx_for(par);
             desc[i].ctx[par].tiles = b->d_tiles + tile_base[i];
@@ -2211,6 +2281,7 @@ int batch_upload_table(qhg_batch *b) {
     if (n) HIPCHK(hipMemcpy(b->d_desc, desc.data(), n * sizeof(PopDesc), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(b->d_tile_base, tile_base.data(), (n + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
     b->total_tiles = tile_base[n];
+    b->gdiv = group_div(b->group_agents, alive, occ);
     b->dirty = false;
     b->table_version++;
     return 0;
@@ -2242,6 +2313,12 @@ int qhg_batch_create(qhg_batch **out) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_scan, kScanBlock, 0) != hipSuccess || per_cu < 1)
         per_cu = 1;
     b->scan_grid = per_cu * b->num_cu;
+    void (*const act[3])(BatchArgs) = {k_batch_act<false>, k_batch_act<true>, k_batch_act<true, true>};
+    for (int k = 0; k < 3; k++) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, act[k], kActBlock, 0) == hipSuccess && n > 1)
+            b->act_per_cu[k] = n;
+    }
     b->genome_grid = b->num_cu * 16;
     *out = b;
     return 0;

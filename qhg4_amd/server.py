@@ -33,9 +33,9 @@ from .ensemble import capacity_for, summary
 from .population import GpuBatch, GpuPopulation
 
 # device bytes of a population without genetics: agent buffers (two of 46 B
-# per slot) and slot scratch (38 B); per-cell tables at most 340 B per cell
+# per slot), slot scratch (45 B) and group lists (1 B); per-cell tables at most 340 B per cell
 # (the population reports its exact figure once it exists)
-PER_SLOT_BYTES = 130
+PER_SLOT_BYTES = 138
 PER_CELL_BYTES = 340
 FIXED_BYTES = 1 << 20
 MAX_MEMBERS = 256

@@ -1,0 +1,131 @@
+"""The step's grouping of cells at its edges: cells of around 64, 128 and 256
+agents (a wave, half a block, a block, larger than a block), groups of many
+small cells (table rows beyond the block's threads), groups that do not fit a
+block, a mix of all; against the oracle, bit for bit.  And a look at the agents
+inside a step, which must not change what the step commits."""
+import numpy as np
+import pytest
+
+from qhg4_amd import abi, scenarios
+from qhg4_amd.grids import rect_grid
+from qhg4_amd.population import GpuBatch, GpuPopulation
+from oracle.oracle import Oracle
+from tests.helpers import assert_same_state, tut_verhulst
+
+pytestmark = pytest.mark.gpu
+
+
+def _counts(kind, ncells, rng):
+    n = np.zeros(ncells, dtype=np.int64)
+    if kind == "edges":
+        sizes = [1, 2, 62, 63, 64, 65, 66, 126, 127, 128, 129, 130, 254, 255, 256, 257, 258, 511, 513]
+        at = rng.choice(ncells, len(sizes), replace=False)
+        n[at] = sizes
+    elif kind == "ones":          # the most cells a group can hold
+        n[:] = 1
+    elif kind == "sixes":         # groups of 28 cells
+        n[:] = 6
+    elif kind == "fours":         # groups of 36 cells: weight rows past the block's threads, neighbour rows not
+        n[:] = 4
+    elif kind == "threes":        # groups of 42 cells: both
+        n[:] = 3
+    elif kind == "hundreds":      # two or three cells per group, some groups past a block
+        n[rng.choice(ncells, 40, replace=False)] = rng.integers(90, 125, 40)
+    elif kind == "mixed":
+        n[:] = rng.choice([0, 0, 1, 2, 5, 30, 70], ncells)
+        n[rng.choice(ncells, 6, replace=False)] = [150, 200, 256, 257, 300, 400]
+    elif kind == "alone":
+        n[7] = 1
+    return n
+
+
+def _scenario(kind, model, seed):
+    rng = np.random.default_rng(seed)
+    if model == "lattice":
+        sc = tut_verhulst(scenarios.c1(seed=seed, width=23, height=19, n_agents=10))
+        sc["params"].verh_K = 400.0
+    else:
+        sc = scenarios.c2(seed=seed, level=3, n_agents=10, patch_cells=5, genetics=model == "genetics")
+        sc["params"].npp_k_max = 600.0
+    ncells = sc["grid"]["num_cells"]
+    n = _counts(kind, ncells, rng)
+    cell = np.repeat(np.arange(ncells), n).astype(np.int32)
+    m = len(cell)
+    age = rng.uniform(0, 40, m)
+    sc["agents"] = {
+        "id": rng.permutation(np.arange(1, 3 * m + 1, dtype=np.int64))[:m], "cell": cell,
+        "life": np.full(m, abi.QHG_LIFE_FERTILE, dtype=np.uint8), "gender": (rng.random(m) < 0.5).astype(np.uint8),
+        "birth_time": -age, "age": age, "last_birth": np.full(m, -5.0), "mate_id": np.full(m, -3, dtype=np.int64),
+        "num_babies": np.zeros(m, dtype=np.int32)}
+    if model == "genetics":
+        sc["agents"]["genome"] = scenarios.initial_genomes(rng, m, 256)
+    return sc
+
+
+KINDS = ["edges", "ones", "fours", "threes", "sixes", "hundreds", "mixed", "alone"]
+
+
+@pytest.mark.parametrize("model", ["lattice", "ooa", "genetics"])
+@pytest.mark.parametrize("kind", KINDS)
+def test_groups_match_the_oracle(kind, model):
+    sc = _scenario(kind, model, 41)
+    gpu, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    gpu.preLoop()
+    ora.pre_loop()
+    for k in range(8):
+        gpu.run(1)
+        ora.run(1)
+        assert_same_state(gpu.agents(), ora.agents(), "%s %s step %d" % (kind, model, k))
+        gs, os_ = gpu.stats(), ora.stats()
+        for f in ("num_alive", "births_last", "deaths_last", "moves_last"):
+            assert gs[f] == os_[f], (f, gs[f], os_[f])
+    gpu.close()
+
+
+@pytest.mark.parametrize("group_agents", [1.0, 20.0, 64.0, 4096.0])
+def test_group_sizes_do_not_change_results(group_agents):
+    sc = _scenario("mixed", "ooa", 43)
+    pop, bat, ora = GpuPopulation.from_scenario(sc), GpuPopulation.from_scenario(sc), Oracle(sc)
+    pop.set_tuning(group_agents, 1)
+    ora.pre_loop()
+    b = GpuBatch()
+    for p in (pop, bat):
+        p.preLoop()
+    b.add(bat)
+    b.set_tuning(group_agents, 1)
+    for k in range(3):
+        pop.run(3)
+        b.run(3)
+        ora.run(3)
+        assert_same_state(pop.agents(), ora.agents(), "alone %d" % k)
+        assert_same_state(bat.agents(), ora.agents(), "batch %d" % k)
+    b.close()
+
+
+@pytest.mark.parametrize("model", ["lattice", "genetics"])
+def test_a_look_inside_a_step_changes_nothing(model):
+    sc = _scenario("mixed", model, 47)
+    gpu, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    gpu.preLoop()
+    ora.pre_loop()
+    for k in range(4):
+        before = gpu.agents()
+        gpu.initializeStep(float(k))
+        gpu.doActions(0, float(k))
+        for _ in range(2):
+            inside = gpu.agents()
+            assert np.array_equal(inside["id"], before["id"])
+            assert np.array_equal(inside["birth_time"], before["birth_time"])
+            alive = inside["life"] != 0
+            assert np.array_equal(inside["age"][alive], (k - inside["birth_time"])[alive])
+            gave = inside["num_babies"] - before["num_babies"]
+            assert set(gave) <= {0, 1} and np.all(inside["gender"][gave == 1] == 0)
+            paired = np.flatnonzero(inside["mate_id"] >= 0)
+            at = np.searchsorted(inside["id"], inside["mate_id"][paired])
+            assert np.array_equal(inside["mate_id"][at], inside["id"][paired])
+            assert np.array_equal(inside["cell"][at], inside["cell"][paired])
+        gpu.state_digest()
+        gpu.finalizeStep()
+        ora.step()
+        assert_same_state(gpu.agents(), ora.agents(), "%s step %d" % (model, k))
+    gpu.close()
