@@ -58,7 +58,7 @@ constexpr int kGroupCells = 64;       // cells of one group: 253 / (1 + 3), up
 constexpr int kGroupSlots = kActBlock;   // agents a block takes at once; larger cells go
                                       // to one wave each, with global scratch lists
 constexpr int kMaxIn = 8;             // incoming neighbour slots per cell
-constexpr int kScanBlock = 256;       // k_cell_scan threads per block
+constexpr int kScanBlock = 512;       // k_cell_scan threads per block
 constexpr int kScanPer = 1;           // cells per k_cell_scan thread
 constexpr int kCellTile = kScanBlock * kScanPer;   // cells per look-back tile
 constexpr int kMaxCross = 32;         // device limit on Genetics_num_crossover
@@ -66,9 +66,8 @@ constexpr int kStatusRing = 8;        // host-mapped status snapshots
 constexpr int kStatusSealEvery = 4;   // steps whose snapshot k_cell_scatter seals for the host
 
 constexpr int32_t kErrCapacity = 1;   // the next population does not fit
-constexpr int32_t kErrLookback = 4;   // a look-back wait exceeded its spin limit
 constexpr int32_t kErrGather = 8;     // an internal count disagreed
-constexpr uint32_t kLookbackSpins = 1u << 22;
+constexpr uint32_t kLookbackSpins = 128;   // waits on a tile before its sums are taken over
 constexpr int kParts = 3;             // per-block partial sums of k_cell_act
 
 // Outcome word of an agent in a step: where it goes (an index into the table
@@ -184,7 +183,6 @@ struct Ctx {
     uint64_t *tiles;          // look-back words of k_cell_scan: agents | births,
     uint64_t *tiles2;         //   and occupied cells
     int32_t ntiles;
-    uint32_t *tick;           // k_cell_scan's tile tickets (zeroed by k_cell_act)
     int32_t nact_blocks;      // grid of k_cell_act
     uint32_t *wave_part;      // kParts per k_cell_act block: deaths, moves, fertile
     uint64_t *scan_part;      // 3 per k_cell_scan wave: the sums of its slice of wave_part
@@ -351,12 +349,14 @@ __device__ __forceinline__ uint64_t tile_read(uint64_t *w) {
 // read as inclusive zeros), so up to 64 * kLookWin predecessors resolve in
 // one read once their aggregates are out.  A predecessor counts only when
 // both of its words carry the same flag (the publisher writes them one after
-// the other).  Every wait is bounded: past the spin limit the step is
-// flagged as failed.
+// the other).  A tile that stays silent (its block may not have started, with
+// other streams' kernels on the device) is summed here, by take(tile, s1, s2),
+// and its aggregate published for it, so no wait depends on which blocks run.
 constexpr int kLookWin = 4;
 
-__device__ void lookback2(uint64_t *t1, uint64_t *t2, uint32_t tile, uint64_t agg1, uint64_t agg2, int32_t *err,
-                          uint64_t &ex1, uint64_t &ex2) {
+template <typename TakeF>
+__device__ __forceinline__ void lookback2(uint64_t *t1, uint64_t *t2, uint32_t tile, uint64_t agg1, uint64_t agg2,
+                                          TakeF take, uint64_t &ex1, uint64_t &ex2) {
     const int lane = threadIdx.x & 63;
     ex1 = 0;
     ex2 = 0;
@@ -382,7 +382,8 @@ __device__ void lookback2(uint64_t *t1, uint64_t *t2, uint32_t tile, uint64_t ag
             w2[m] = (j >= 0) ? tile_read(&t2[j]) : kFlagInc;
         }
         uint64_t s1 = 0, s2 = 0;
-        bool wait = false, done = false;
+        bool done = false;
+        int64_t silent = -1;
 #pragma unroll
         for (int m = 0; m < kLookWin; m++) {
             const uint64_t f1 = w1[m] & ~kValMask, f2 = w2[m] & ~kValMask;
@@ -392,7 +393,7 @@ __device__ void lookback2(uint64_t *t1, uint64_t *t2, uint32_t tile, uint64_t ag
             const int first = inc ? (__ffsll((unsigned long long)inc) - 1) : 64;
             const uint64_t need = (first >= 63) ? ~0ull : ((2ull << first) - 1ull);
             if (nready & need) {
-                wait = true;
+                silent = top - 64 * m - (__ffsll((unsigned long long)(nready & need)) - 1);
                 break;
             }
             s1 += wave_sum_u64(lane <= first ? (w1[m] & kValMask) : 0ull);
@@ -402,18 +403,31 @@ __device__ void lookback2(uint64_t *t1, uint64_t *t2, uint32_t tile, uint64_t ag
                 break;
             }
         }
-        if (wait) {
+        if (silent >= 0) {
             if (++spins < kLookbackSpins) {
                 __builtin_amdgcn_s_sleep(1);
                 continue;
             }
-            if (lane == 0) atomicOr(err, kErrLookback);
-            break;
+            // take the tile's sums, and publish them if it is still silent: its
+            // block puts its inputs back to zero only after it has published
+            spins = 0;
+            uint64_t a1, a2;
+            take((uint32_t)silent, a1, a2);
+            if (lane == 0 && tile_read(&t1[silent]) == 0 && tile_read(&t2[silent]) == 0) {
+                uint64_t zero = 0;
+                __hip_atomic_compare_exchange_strong(&t1[silent], &zero, kFlagAgg | a1, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                zero = 0;
+                __hip_atomic_compare_exchange_strong(&t2[silent], &zero, kFlagAgg | a2, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            continue;
         }
         ex1 += s1;
         ex2 += s2;
         if (done) break;
         top -= 64 * kLookWin;
+        spins = 0;
     }
     if (lane == 0) {
         tile_publish(&t1[tile], kFlagInc | (ex1 + agg1));
@@ -1278,7 +1292,6 @@ __device__ __forceinline__ void cell_act_kernel() {
             A.x.st->deaths_last = 0;
             A.x.st->moves_last = 0;
             A.x.st->big[1 - par] = 0;   // k_cell_scan sets it
-            *A.x.tick = 0u;
         }
         if (tid < kParts) part[tid] = 0u;
         for (; g < ngrp; g += gridDim.x) {
@@ -1708,12 +1721,18 @@ __global__ void __launch_bounds__(kWave) k_assort_pair(Ctx x, Prog p, StepArgs s
 // k_cell_scan: next per-cell counts and birth counts, scanned together
 // (low 32 bits agents, high bits births), and the occupied cells of the next
 // step, with a decoupled look-back over tiles of kCellTile cells, one cell
-// per thread.  Blocks take tiles by ticket; the grid fits on the device.
-// Also writes the absolute next-buffer position of every incoming run and
-// of each cell's newborns.  The block of the last tile closes the step's
-// bookkeeping in the other status half.
+// per thread, block b taking tiles b, b + grid, ...  Also writes the absolute
+// next-buffer position of every incoming run and of each cell's newborns.
+// The block of the last tile closes the step's bookkeeping in the other
+// status half.
 // The scan is latency-bound (one wave per SIMD at most): every thread's
 // loads go out in one round trip, and the code on that path is kept short.
+// Tiles were handed out by an atomic ticket at first, for progress with few
+// blocks resident; at ~20 ns each on one address, the tickets alone took 13 of
+// 25 us at 641 tiles (1.39 M agents), 3.5 of 11.3 at 161 (369 k); now 16 and
+// 8.6.  Tiles of 512 cells rather than 256: half the words to look back over
+// (15.8 against 17.4 us at 1.39 M agents, the same below; 1,024: 14.2, but 9.9
+// against 8.6 at 369 k).
 // ---------------------------------------------------------------------------
 constexpr int kStageWords = kCellTile * kMaxIn;       // a tile's incoming-run words
 constexpr int kStagePer = kStageWords / kScanBlock;   // ... per thread
@@ -1722,25 +1741,11 @@ static_assert(kScanPer == 1, "one cell per scan thread");
 struct ScanLds {
     uint64_t w[kScanBlock / 64], w2[kScanBlock / 64];
     uint64_t excl, excl2;
-    uint32_t ticket;
     // dense steps: the tile's incoming-run counts and source slots, loaded
     // coalesced (cell-major, in_w words per cell)
     uint32_t cm[kStageWords];
     int32_t ie[kStageWords];
 };
-
-// The next tile for this block.  Tiles are handed out in increasing order by
-// an atomic counter, so every tile a block waits on in the look-back has
-// been taken by a block that is already running: the scan makes progress
-// however few of its blocks are resident (other streams' kernels may hold
-// compute units meanwhile).
-__device__ __forceinline__ uint32_t next_tile(uint32_t *ticket, ScanLds &L) {
-    if (threadIdx.x == 0) L.ticket = atomicAdd(ticket, 1u);
-    __syncthreads();
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.ticket);
-    __syncthreads();
-    return t;
-}
 
 // The piece of the line that place y lies in.
 __host__ __device__ __forceinline__ uint32_t group_of(uint32_t y, uint32_t gdiv) {
@@ -1995,32 +2000,44 @@ __device__ __forceinline__ void scan_tile(const CtxT &x, const StepArgs &sa, uin
         }
         return;
     }
-    tile_clear(x, tile, I);
     const TileSums S = tile_sums(I, L);
     if (threadIdx.x < 64) {
         uint64_t ex, ex2;
-        lookback2(x.tiles, x.tiles2, tile, S.tot, S.otot, &x.st->error, ex, ex2);
+        const auto take = [&](uint32_t t, uint64_t &a1, uint64_t &a2) {
+            a1 = a2 = 0;
+            for (int64_t c = (int64_t)t * kCellTile + (threadIdx.x & 63), q = 0; q < kCellTile / kWave; q++, c += kWave) {
+                if (c >= x.ncells) break;
+                const uint32_t st = x.cstay[c], bi = x.cbirth[c], ar = x.carr[c];
+                a1 += (uint64_t)(st + ar + bi) | ((uint64_t)bi << 32);
+                a2 += (st + ar + bi) ? 1u : 0u;
+            }
+            a1 = wave_sum_u64(a1);
+            a2 = wave_sum_u64(a2);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the inputs are read before the words again
+        };
+        lookback2(x.tiles, x.tiles2, tile, S.tot, S.otot, take, ex, ex2);
+        // the tile's words are out before its inputs go back to zero
+        __builtin_amdgcn_s_waitcnt(0);
         if (threadIdx.x == 0) { L.excl = ex; L.excl2 = ex2; }
     }
     __syncthreads();
+    tile_clear(x, tile, I);
     tile_write(x, sa, tile, I, L, L.excl + S.pre, L.excl2 + S.opre);
     if (more) __syncthreads();
 }
 
-// kOneRound: the grid has a block per tile, so the first round of tickets
-// hands out every tile and no block asks again (straight-line code; the
-// host launches the looping form otherwise).
+// kOneRound: the grid has a block per tile (straight-line code; the host
+// launches the looping form otherwise).
 template <bool kOneRound>
 __global__ void __launch_bounds__(kScanBlock) k_cell_scan(Ctx x, StepArgs sa) {
     __shared__ ScanLds lds;
     const int lane = threadIdx.x & 63;
     const uint32_t nt = (uint32_t)x.ntiles;
     // One round trip for: the status, this thread's first slice of the
-    // k_cell_act partials (deaths, moves, FERTILE counts), the inputs of tile
-    // blockIdx.x (the ticket this block most likely draws) with its activity
-    // flag, and, issued last, the first ticket: waiting for the ticket waits
-    // for them all.  The partials' wave sums are stored at the end for
-    // k_cell_scatter's bookkeeping block (plain stores: no contended atomics).
+    // k_cell_act partials (deaths, moves, FERTILE counts) and the inputs of
+    // the block's first tile with its activity flag.  The partials' wave sums
+    // are stored at the end for k_cell_scatter's bookkeeping block (plain
+    // stores: no contended atomics).
     const int32_t err = x.st->error;
     const int32_t j0 = blockIdx.x * kScanBlock + threadIdx.x;
     const int32_t jstride = gridDim.x * kScanBlock;
@@ -2029,48 +2046,24 @@ __global__ void __launch_bounds__(kScanBlock) k_cell_scan(Ctx x, StepArgs sa) {
     const uint32_t p0 = x.wave_part[kParts * jc + 0];
     const uint32_t p1 = x.wave_part[kParts * jc + 1];
     const uint32_t p2 = x.wave_part[kParts * jc + 2];
-    const uint32_t spec = (blockIdx.x < nt) ? blockIdx.x : nt - 1;
-    const uint32_t ta = x.tact[spec];
+    const uint32_t first = blockIdx.x;   // the grid has at most a block per tile
+    const uint32_t ta = x.tact[first];
     TileIn I;
-    tile_load(x, sa, spec, true, I);
-    uint32_t tk = 0;
-    if (threadIdx.x == 0) tk = atomicAdd(x.tick, 1u);
+    tile_load(x, sa, first, true, I);
     tile_ready(I);
-    tile_stage(I, lds);
-    if (threadIdx.x == 0) lds.ticket = tk;
-    __syncthreads();
-    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.ticket);
     if (err) return;
     const auto active = [&](uint32_t t, uint32_t flag) -> uint32_t {
         return ((int64_t)t * kCellTile + kCellTile >= x.ncells || flag != 0u) ? 1u : 0u;
     };
-    if (kOneRound) {
-        if (first < nt) {
-            uint32_t act = active(spec, ta);
-            if (first != spec) {
-                // not the tile loaded ahead: load this one now
-                __syncthreads();   // the LDS staging may still be read
-                act = active(first, x.tact[first]);
-                tile_load(x, sa, first, true, I);
-                tile_ready(I);
-                tile_stage(I, lds);
-            }
-            scan_tile(x, sa, first, act, I, lds, false);
-        }
-    } else {
-        uint32_t tile = spec;
-        for (uint32_t t = first; t < nt; t = next_tile(x.tick, lds)) {
-            uint32_t act = active(tile, ta);
-            if (t != tile) {
-                __syncthreads();   // the LDS staging may still be read
-                tile = t;
-                act = active(tile, x.tact[tile]);
-                tile_load(x, sa, tile, true, I);
-                tile_ready(I);
-                tile_stage(I, lds);
-            }
+    tile_stage(I, lds);
+    scan_tile(x, sa, first, active(first, ta), I, lds, !kOneRound);
+    if (!kOneRound) {
+        for (uint32_t t = first + gridDim.x; t < nt; t += gridDim.x) {
+            const uint32_t act = active(t, x.tact[t]);
+            tile_load(x, sa, t, true, I);
+            tile_ready(I);
+            tile_stage(I, lds);
             scan_tile(x, sa, t, act, I, lds, true);
-            tile = nt;   // later tiles are loaded on demand
         }
     }
     uint64_t D = pok ? p0 : 0u, Mv = pok ? p1 : 0u, Fe = pok ? p2 : 0u;

@@ -147,7 +147,6 @@ struct qhg_pop {
     double *d_env[7] = {};   // alt lon lat water npp temp rain
     uint32_t *d_cstay = nullptr, *d_cbirth = nullptr, *d_cin = nullptr, *d_carr = nullptr, *d_birth_off = nullptr;
     uint32_t *d_tact = nullptr;   // per scan tile
-    uint32_t *d_tick = nullptr;   // the scan's tile tickets
     int32_t *d_outk = nullptr;
     uint32_t *d_bpos = nullptr, *d_rpos = nullptr;
     uint64_t *d_tiles = nullptr, *d_tiles2 = nullptr;
@@ -253,7 +252,6 @@ struct qhg_pop {
         x.cin = d_cin;
         x.carr = d_carr;
         x.tact = d_tact;
-        x.tick = d_tick;
         x.outk = d_outk;
         x.birth_off = d_birth_off;
         x.bpos = d_bpos;
@@ -1360,7 +1358,6 @@ int qhg_gpu_create(const qhg_grid_desc *grid, const qhg_env_desc *env, const qhg
         hipMalloc(&p->d_off[1], (nc + 1) * 4) != hipSuccess || hipMalloc(&p->d_cstay, (nc + 2) * 4) != hipSuccess ||
         hipMalloc(&p->d_cbirth, (nc + 2) * 4) != hipSuccess || hipMalloc(&p->d_cin, nc * p->in_w * 4) != hipSuccess ||
         hipMalloc(&p->d_carr, (nc + 2) * 4) != hipSuccess || hipMalloc(&p->d_tact, (size_t)p->ntiles * 4) != hipSuccess ||
-        hipMalloc(&p->d_tick, 4) != hipSuccess ||
         hipMalloc(&p->d_birth_off, (nc + 1) * 4) != hipSuccess || hipMalloc(&p->d_bpos, nc * 4) != hipSuccess ||
         hipMalloc(&p->d_rpos, nc * p->conn * 4) != hipSuccess ||
         hipMalloc(&p->d_tiles, (size_t)p->ntiles * 8) != hipSuccess ||
@@ -1383,7 +1380,6 @@ int qhg_gpu_create(const qhg_grid_desc *grid, const qhg_env_desc *env, const qhg
     (void)hipMemsetAsync(p->d_cin, 0, nc * p->in_w * 4, p->stream);
     (void)hipMemsetAsync(p->d_carr, 0, (nc + 2) * 4, p->stream);
     (void)hipMemsetAsync(p->d_tact, 0, (size_t)p->ntiles * 4, p->stream);
-    (void)hipMemsetAsync(p->d_tick, 0, 4, p->stream);
     (void)hipMemsetAsync(p->d_st, 0, sizeof(DevStatus), p->stream);
     if (env) {
         const double *src[7] = {env->altitude, env->longitude, env->latitude, env->water,
@@ -1419,7 +1415,7 @@ int qhg_gpu_destroy(qhg_pop *p) {
     free_slot_scratch(p);
     free_nav_tables(p);
     void *ptrs[] = {p->d_off[0], p->d_off[1], p->d_gpool[0], p->d_gpool[1], p->d_nbr, p->d_nn, p->d_in_e,
-                    p->d_K, p->d_W, p->d_tmp, p->d_ice, p->d_coastal, p->d_cstay, p->d_cbirth, p->d_cin, p->d_carr, p->d_tact, p->d_tick, p->d_outk,
+                    p->d_K, p->d_W, p->d_tmp, p->d_ice, p->d_coastal, p->d_cstay, p->d_cbirth, p->d_cin, p->d_carr, p->d_tact, p->d_outk,
                     p->d_birth_off, p->d_bpos, p->d_rpos, p->d_tiles, p->d_tiles2, p->d_occ[0], p->d_occ[1],
                     p->d_wave_part, p->d_scan_part, p->d_st, p->d_digest, p->d_rank};
     for (void *q : ptrs)

@@ -129,3 +129,29 @@ def test_a_look_inside_a_step_changes_nothing(model):
         ora.step()
         assert_same_state(gpu.agents(), ora.agents(), "%s step %d" % (model, k))
     gpu.close()
+
+
+@pytest.mark.parametrize("width,height", [(1, 1), (511, 1), (512, 1), (513, 1), (32, 32), (41, 25), (600, 300)])
+def test_scan_tiles_match_the_oracle(width, height):
+    """Grids of a tile less one cell, a tile, one more, several; agents in
+    every 7th cell and in the last one."""
+    sc = tut_verhulst(scenarios.c1(seed=9, width=width, height=height, n_agents=10))
+    ncells = width * height
+    rng = np.random.default_rng(9)
+    cell = np.unique(np.concatenate([np.arange(0, ncells, 7), [ncells - 1]])).repeat(5).astype(np.int32)
+    m = len(cell)
+    age = rng.uniform(0, 40, m)
+    sc["agents"] = {
+        "id": np.arange(1, m + 1, dtype=np.int64), "cell": cell,
+        "life": np.full(m, abi.QHG_LIFE_FERTILE, dtype=np.uint8), "gender": (rng.random(m) < 0.5).astype(np.uint8),
+        "birth_time": -age, "age": age, "last_birth": np.zeros(m), "mate_id": np.full(m, -3, dtype=np.int64),
+        "num_babies": np.zeros(m, dtype=np.int32)}
+    gpu, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    gpu.preLoop()
+    ora.pre_loop()
+    for k in range(4):
+        gpu.run(3)
+        ora.run(3)
+        assert_same_state(gpu.agents(), ora.agents(), "step %d" % (3 * k + 3))
+        assert np.array_equal(gpu.getNumAgentsArray(), ora.cell_counts())
+    gpu.close()
