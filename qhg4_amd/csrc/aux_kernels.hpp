@@ -194,6 +194,7 @@ __global__ void __launch_bounds__(kKillBlock) k_env_kill(const OccCell *occ, int
         st->n_occ[nb] = out;
         st->n_grp[nb] = group_close(grp, grp_cap, gdiv, (uint32_t)out, slots);
         st->big[nb] = st->big[b];
+        st->mid[nb] = st->mid[b];
         st->n_alive[nb] = slots;
         st->max_id[nb] = st->max_id[b];
         st->gpool[nb] = st->gpool[b];

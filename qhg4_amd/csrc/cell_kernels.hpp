@@ -57,6 +57,7 @@ constexpr int kGroupPieceMin = 48, kGroupPieceMax = 252;
 constexpr int kGroupCells = 64;       // cells of one group: 253 / (1 + 3), up
 constexpr int kGroupSlots = kActBlock;   // agents a block takes at once; larger cells go
                                       // to one wave each, with global scratch lists
+constexpr int kAssortCell = 128;      // largest cell a block of k_assort_pair takes
 constexpr int kMaxIn = 8;             // incoming neighbour slots per cell
 constexpr int kScanBlock = 512;       // k_cell_scan threads per block
 constexpr int kScanPer = 1;           // cells per k_cell_scan thread
@@ -91,7 +92,8 @@ struct DevStatus {
     int64_t max_id[2];
     int64_t gpool[2];        // genome pool high-water mark
     int64_t n_grp[2];        // groups of occupied cells at the start of a step of this parity
-    int64_t big[2];          // ... and whether a cell may hold more agents than a block takes
+    int64_t big[2];          // ... and whether a cell may hold more agents than a block of
+    int64_t mid[2];          // k_cell_act takes, or of k_assort_pair
     int64_t step;            // steps completed
     double t;
     int64_t births_last, deaths_last, moves_last;
@@ -239,6 +241,7 @@ struct Prog {
     int32_t gen_size, gen_cross, nbino;
     // AssortativePairHamming: mates come from k_assort_pair (x.gmate)
     int32_t assort_permute;
+    int32_t assort_dmax;      // largest distance whose match counts (-1: none)
     int32_t assort_words;     // numNucs2Blocks(numBlocks): words per strand position compared
     float assort_cutoff;
     int32_t assort_prot;      // AssortativePair: matches counted over protein digests
@@ -947,8 +950,56 @@ __device__ __forceinline__ void big_cells(ConstCtx &x, ConstProg &p, uint32_t st
 enum { kCntF = 0, kCntM, kCntBirth, kCntStay, kCntMv, kCntN = kCntMv + 6 };
 constexpr int kGroupWords = kGroupSlots / 64;
 
-struct GroupActLds {
+// The cells of a group in one block, one thread per agent.
+struct GroupCells {
     uint64_t starts[kGroupWords];                   // bit q: a cell begins at group position q
+    int32_t c[kGroupCells];
+    uint32_t eb[kGroupCells], n[kGroupCells];       // first position, agents
+    int32_t nfit;                                   // cells that fit the block
+};
+
+__device__ __forceinline__ void group_clear(GroupCells &G, int tid, int nc) {
+    if (tid < kGroupWords) G.starts[tid] = 0ull;
+    if (tid == 0) G.nfit = nc;
+}
+
+// cell number tid of the group (after group_clear and a barrier)
+template <int kMaxCell>
+__device__ __forceinline__ void group_cell(GroupCells &G, int tid, const OccCell &e, uint32_t S0) {
+    const uint32_t eb = e.s - S0;
+    // the first cell that ends past the block's agents, or is too large for it,
+    // begins the next pass
+    if (eb + e.n > (uint32_t)kGroupSlots || e.n > (uint32_t)kMaxCell) atomicMin(&G.nfit, tid);
+    else atomicOr((unsigned long long *)&G.starts[eb >> 6], 1ull << (eb & 63u));
+    G.c[tid] = e.c;
+    G.eb[tid] = eb;
+    G.n[tid] = e.n;
+}
+
+// the cell of group position tid: cells beginning at or before it
+__device__ __forceinline__ int group_cell_of(const GroupCells &G, int tid) {
+    int k = __popcll(G.starts[tid >> 6] & (~0ull >> (63 - (tid & 63)))) - 1;
+#pragma unroll
+    for (int j = 0; j < kGroupWords - 1; j++)
+        if (j < (tid >> 6)) k += __popcll(G.starts[j]);
+    return k;
+}
+
+// entries below id among the n at first, first + dirn, ...
+__device__ __forceinline__ int group_id_rank(const int64_t *lid, int first, int dirn, int n, int64_t id) {
+    int rank = 0;
+    for (int u = 0; u < n; u += 4) {
+        int64_t o[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) o[v] = lid[first + dirn * ((u + v < n) ? u + v : 0)];
+#pragma unroll
+        for (int v = 0; v < 4; v++) rank += (u + v < n && o[v] < id) ? 1 : 0;
+    }
+    return rank;
+}
+
+struct GroupActLds {
+    GroupCells gc;
     // FERTILE lists of cell k at positions [eb_k, eb_k + n_k): females from
     // the front (rank r at eb_k + r), males from the back (at eb_k + n_k-1-r)
     int64_t lid[kGroupSlots];                       // ids, gather order; then the mothers' ids
@@ -957,13 +1008,10 @@ struct GroupActLds {
     int32_t nbr[kGroupCells][6];
     int16_t pick[kGroupSlots];                      // rank position of a chooser -> its pick among those left
     uint32_t cnt[kGroupCells][kCntN];               // per-cell counters
-    int32_t c[kGroupCells];
-    uint32_t eb[kGroupCells], n[kGroupCells];       // first position, agents
     int16_t srt[kGroupSlots];                       // id rank -> group position of the agent
     int16_t prt[kGroupSlots];                       // id rank -> the partner's rank position, -1
     uint8_t nn[kGroupCells];
     int32_t noff[kGroupCells], nend[kGroupCells];   // Navigate: first and end edge per cell
-    int32_t nfit;             // cells that fit the block
 };
 
 // One group: the cells of occupied-cell entries [d0.first, d1.first), whose
@@ -1028,56 +1076,39 @@ __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t 
         OccCell e{0, 0, 0, 0};
         if (tid < nc) e = x.occ_cur[i0 + (uint32_t)tid];
         for (int k = tid; k < nc * kCntN; k += kActBlock) (&G.cnt[0][0])[k] = 0u;
-        if (tid < kGroupWords) G.starts[tid] = 0ull;
-        if (tid == 0) G.nfit = nc;
+        group_clear(G.gc, tid, nc);
         G.prt[tid] = -1;
         __syncthreads();
-        if (tid < nc) {
-            const uint32_t eb = e.s - S0;
-            if (eb < (uint32_t)kGroupSlots) {
-                // the first cell that ends past the block's agents begins the next pass
-                if (eb + e.n > (uint32_t)kGroupSlots) G.nfit = tid;
-                else atomicOr((unsigned long long *)&G.starts[eb >> 6], 1ull << (eb & 63u));
-            } else if (eb == (uint32_t)kGroupSlots) {
-                G.nfit = tid;
-            }
-            G.c[tid] = e.c;
-            G.eb[tid] = eb;
-            G.n[tid] = e.n;
-        }
+        if (tid < nc) group_cell<kGroupSlots>(G.gc, tid, e, S0);
         __syncthreads();
-        nc = uniform_i32(G.nfit);
+        nc = uniform_i32(G.gc.nfit);
         if (nc == 0) {   // a cell larger than the block (big_cells)
-            S0 += (uint32_t)uniform_i32((int)G.n[0]);
+            S0 += (uint32_t)uniform_i32((int)G.gc.n[0]);
             i0++;
             __syncthreads();
             continue;
         }
         // [eb, eb + n) of cell nc - 1 ends the pass
-        const uint32_t T = (uint32_t)uniform_i32((int)(G.eb[nc - 1] + G.n[nc - 1]));
+        const uint32_t T = (uint32_t)uniform_i32((int)(G.gc.eb[nc - 1] + G.gc.n[nc - 1]));
         const bool valid = (uint32_t)tid < T;
-        // the agent's cell: cells beginning at or before it
-        int k = __popcll(G.starts[tid >> 6] & (~0ull >> (63 - (tid & 63)))) - 1;
-#pragma unroll
-        for (int j = 0; j < kGroupWords - 1; j++)
-            if (j < (tid >> 6)) k += __popcll(G.starts[j]);
-        const int eb = (int)G.eb[k], nk = (int)G.n[k];
-        const int32_t c = G.c[k];
+        const int k = group_cell_of(G.gc, tid);
+        const int eb = (int)G.gc.eb[k], nk = (int)G.gc.n[k];
+        const int32_t c = G.gc.c[k];
         // the cells' tables: read now, put into LDS two barriers below, where
         // their round trip is over
         double tW = 0, tK = 0;
         int32_t tN = -1, tO = -1, tE0 = 0, tE1 = 0;
         uint8_t tnn = 0;
         const int wk = tid / 7, wj = tid % 7, nk6 = tid / 6, nj = tid % 6;
-        if (wk < nc && wj < R) tW = x.W[(int64_t)G.c[wk] * R + wj];
+        if (wk < nc && wj < R) tW = x.W[(int64_t)G.gc.c[wk] * R + wj];
         if (nk6 < nc && nj < conn) {
-            const int64_t at = (int64_t)G.c[nk6] * conn + nj;
+            const int64_t at = (int64_t)G.gc.c[nk6] * conn + nj;
             tN = x.nbr[at];
             tO = x.outk[at];
         }
         const int kc = tid - kWave;   // the second wave's lanes: one cell each
         if (kc >= 0 && kc < nc) {
-            const int32_t cc = G.c[kc];
+            const int32_t cc = G.gc.c[kc];
             if (pk.flags & kActVarK) tK = x.K[cc];
             tnn = x.nn[cc];
             if (kNav && x.nav.n != 0) {   // no tables (null pointers) when n is 0
@@ -1106,13 +1137,7 @@ __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t 
             if (isF || isM) {
                 const int Fk = (int)G.cnt[k][kCntF], Mk = (int)G.cnt[k][kCntM];
                 const int n1 = isF ? Fk : Mk;
-                for (int u = 0; u < n1; u += 4) {
-                    int64_t o[4];
-#pragma unroll
-                    for (int v = 0; v < 4; v++) o[v] = G.lid[first + dirn * ((u + v < n1) ? u + v : 0)];
-#pragma unroll
-                    for (int v = 0; v < 4; v++) rank += (u + v < n1 && o[v] < a.id) ? 1 : 0;
-                }
+                rank = group_id_rank(G.lid, first, dirn, n1, a.id);
                 P = first + dirn * rank;
                 G.srt[P] = (int16_t)tid;
                 if (isF ? (Fk <= Mk) : (Mk < Fk)) {
@@ -1125,8 +1150,8 @@ __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t 
         if (wk < nc) G.W[wk][wj] = tW;
         if (nk6 < nc) G.nbr[nk6][nj] = tN;
         if (kc >= 0 && kc < nc) {
-            G.rat[kc] = (pk.flags & kActVarK) ? vark_ratio(G.n[kc], tK) : 0.0;
-            G.ratc[kc] = (pk.flags & kActVerh) ? (double)G.n[kc] / pk.Kconst : 0.0;
+            G.rat[kc] = (pk.flags & kActVarK) ? vark_ratio(G.gc.n[kc], tK) : 0.0;
+            G.ratc[kc] = (pk.flags & kActVerh) ? (double)G.gc.n[kc] / pk.Kconst : 0.0;
             G.nn[kc] = tnn;
             if (kNav) {
                 G.noff[kc] = tE0;
@@ -1135,9 +1160,9 @@ __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t 
         }
         if (nc * 7 > kActBlock) {   // many small cells: the rows beyond the block's threads
             for (int q = tid + kActBlock; q < nc * 7; q += kActBlock)
-                G.W[q / 7][q % 7] = (q % 7 < R) ? x.W[(int64_t)G.c[q / 7] * R + q % 7] : 0.0;
+                G.W[q / 7][q % 7] = (q % 7 < R) ? x.W[(int64_t)G.gc.c[q / 7] * R + q % 7] : 0.0;
             for (int q = tid + kActBlock; q < nc * 6; q += kActBlock)
-                G.nbr[q / 6][q % 6] = (q % 6 < conn) ? x.nbr[(int64_t)G.c[q / 6] * conn + q % 6] : -1;
+                G.nbr[q / 6][q % 6] = (q % 6 < conn) ? x.nbr[(int64_t)G.gc.c[q / 6] * conn + q % 6] : -1;
         }
         __syncthreads();
         // findMates (RandomPair.cpp:183-276): choosers in id order, each
@@ -1220,7 +1245,7 @@ __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t 
             const uint32_t m = G.cnt[kk][kCntMv + d];
             if (m) {
                 const int32_t dest = G.nbr[kk][d];
-                cin[(q == tid) ? tO : x.outk[(int64_t)G.c[kk] * conn + d]] = m;
+                cin[(q == tid) ? tO : x.outk[(int64_t)G.gc.c[kk] * conn + d]] = m;
                 atomicAdd(&carr[dest], m);
                 tact[dest / kCellTile] = 1u;
             }
@@ -1291,7 +1316,7 @@ __device__ __forceinline__ void cell_act_kernel() {
         if (blockIdx.x == 0 && tid == 0) {
             A.x.st->deaths_last = 0;
             A.x.st->moves_last = 0;
-            A.x.st->big[1 - par] = 0;   // k_cell_scan sets it
+            A.x.st->big[1 - par] = A.x.st->mid[1 - par] = 0;   // k_cell_scan sets them
         }
         if (tid < kParts) part[tid] = 0u;
         for (; g < ngrp; g += gridDim.x) {
@@ -1355,22 +1380,29 @@ __global__ void __launch_bounds__(256) k_act_commit(Ctx x, StepArgs sa, int32_t 
 
 // ---------------------------------------------------------------------------
 // k_assort_pair: AssortativePairHamming (AssortativePairHam.cpp:93-238 with
-// RankTable.cpp:119-278), one wave per occupied cell, before k_cell_act.
-//   - the cell's FERTILE females and males, each in id order;
-//   - the match of female i and male j, 1 - calcDist(i, j, numBlocks) /
-//     genomeSize as a float (GeneUtils.cpp:414-444), read from the genomes
-//     when needed rather than held in a table: a couple's value in the
-//     reference's table is that match while both are unpaired and it is at
-//     or above the cutoff, else 0;
+// RankTable.cpp:119-278) and AssortativePair (AssortativePair.cpp:94-271), one
+// block per group of cells, before k_cell_act.
+//   - the cells' FERTILE females and males, each in id order;
+//   - the match of female i and male j of a cell: 1 - calcDist(i, j,
+//     numBlocks) / genomeSize as a float (GeneUtils.cpp:414-444), or the
+//     number of equal protein digests; a couple counts while both are
+//     unpaired and its match is above 0 and at or above the cutoff;
 //   - rounds of RankTable::pairHighestRankers: the largest value, the
 //     females that reach it (permuted when asked), each female in turn
 //     picking at random among the unpaired males at that value.
 // The cell's draws come in the reference's order from QHG_STREAM_ASSORT.
 // Output: x.gmate[slot] = partner slot (-1 none); k_cell_act reads it instead
-// of pairing.  Scratch in the cell's own slot range
-// [s, s+n): gfu/gfid, gmu/gmid (gather), gfs/gms (slots in id order),
-// gfu/gmu (then their genome handles in id order), gfid (the round's female
-// order), gflag (paired: female r at s+r, male r at s+F+r).
+// of pairing.
+//
+// The rounds compare matches only, so the table holds their order as a byte:
+// dmax + 1 - distance (dmax the largest distance whose match counts: the match
+// falls with the distance), or the number of equal digests (256, all of
+// two full lists, as 255, which no lists give); 0 does not count.  The
+// rounds are serial within a cell and short, so 16 lanes take a cell and a
+// block its ~14 cells at once; a wave per cell left most lanes idle and took
+// 55 us at 369 k agents against 25.6 here (7 blocks per CU; 29.5 at 5), the
+// protein matches, recomputed from global memory in every round, 913 us at
+// 80 k agents against 51 and k_proteins' 28.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int bitcount2(uint64_t v) {   // GeneUtils::bitcount2
     return __popcll((v | (v >> 1)) & 0x5555555555555555ull);
@@ -1389,21 +1421,27 @@ __device__ __forceinline__ uint32_t assort_draw(uint64_t seed, uint32_t step, in
     return draw(seed, step, QHG_STREAM_ASSORT, (uint64_t)(uint32_t)c | ((uint64_t)(j >> 16) << 32), j & 0xffffu);
 }
 
-template <typename CtxT>
-__device__ __forceinline__ float assort_match(const CtxT &x, const Prog &p, int32_t hf, int32_t hm) {
-    const uint64_t *a = x.gpool + (int64_t)hf * x.gwords;
-    const uint64_t *b = x.gpool + (int64_t)hm * x.gwords;
-    const int D = p.assort_words;
+__device__ __forceinline__ int assort_dist(const uint64_t *a, const uint64_t *b, int D) {
     int c1 = 0, c2 = 0;
     for (int k = 0; k < 2 * D; k++) c1 += bitcount2(a[k] ^ b[k]);
     for (int k = 0; k < D; k++) c2 += bitcount2(a[k + D] ^ b[k]) + bitcount2(a[k] ^ b[k + D]);
-    const int d = (c1 < c2) ? c1 : c2;
-    return (float)(1.0 - (1.0 * d) / (double)p.gen_size);
+    return (c1 < c2) ? c1 : c2;
 }
 
 template <typename CtxT>
+__device__ __forceinline__ float assort_match(const CtxT &x, const Prog &p, int32_t hf, int32_t hm) {
+    const int d = assort_dist(x.gpool + (int64_t)hf * x.gwords, x.gpool + (int64_t)hm * x.gwords, p.assort_words);
+    return (float)(1.0 - (1.0 * d) / (double)p.gen_size);
+}
+
+// A cell too large for a block, by one wave: lists in the cell's
+// range of global scratch, matches recomputed when needed.  Scratch [s, s+n):
+// gfu/gfid, gmu/gmid (gather), gfs/gms (slots in id order), gfu/gmu (then
+// their genome handles in id order), gfid (the round's female order), gflag
+// (paired: female r at s+r, male r at s+F+r).
+template <typename CtxT>
 __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, int32_t c, uint32_t s, int32_t n) {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt();
     int32_t F = 0, M = 0;
     for (int32_t b = 0; b < n; b += kWave) {
@@ -1449,17 +1487,10 @@ __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, in
     const int32_t *hf = x.gfu + s, *hm = x.gmu + s;
     uint8_t *pf = x.gflag + s, *pm = x.gflag + s + F;
     if (p.assort_prot) {
-        // AssortativePair: every listed agent's protein digests into its
-        // slot's share of the pool (translateGenomeHash)
         for (int32_t j = lane; j < F + M; j += kWave) {
             const int32_t sl = (j < F) ? x.gfs[s + j] : x.gms[s + (j - F)];
-            const int32_t h = (j < F) ? hf[j] : hm[j - F];
-            const int32_t np = protein_digests(x.gpool + (int64_t)h * x.gwords, x.gwords, p.gen_size,
-                                               x.gprot + (int64_t)sl * (4 * kProtBudget));
-            x.gnprot[sl] = np;
-            if (np > kProtBudget) atomicOr(&x.st->error, kErrProteins);
+            if (x.gnprot[sl] > kProtBudget) atomicOr(&x.st->error, kErrProteins);
         }
-        wave_sync();
     }
     // the match of female i and male j (id order)
     const auto match = [&](int32_t i, int32_t j) -> float {
@@ -1556,164 +1587,355 @@ __device__ void assort_cell(const CtxT &x, const Prog &p, const StepArgs &sa, in
     }
 }
 
-// A cell of at most one wave of agents, everything in LDS: the sorted
-// lists, the compared genome words and the whole distance table (F + M <=
-// 64, so F * M <= 1024), read from HBM once.  A couple's match is the
-// block's table value of its distance (d <= 2 * D * 32 = 128), the same
-// float as 1 - d / genomeSize.  Same rounds and draws as assort_cell.
-constexpr int kAssortMaxDist = 128;
-struct AssortLds {
-    int64_t fid[kWave], mid[kWave];       // ids, gather order
-    int32_t fslot[kWave], mslot[kWave];   // slots, id order
-    int32_t ord[kWave];                   // the round's female order
-    uint64_t fw[kWave][4], mw[kWave][4];  // compared genome words (2 * D <= 4), id order
-    float val[kAssortMaxDist + 1];        // match of each distance
-    uint32_t rmax[kWave];                 // a round's largest value per female (float bits)
-    uint8_t T[kWave * kWave / 4];         // distance of female i and male j at i * M + j
-    uint8_t pf[kWave], pm[kWave];         // paired
+constexpr int kProtPool = 1024;   // digests that a k_assort_pair block keeps in LDS
+struct Digest {
+    uint64_t lo, hi;
 };
 
-__device__ __forceinline__ int assort_dist_w(const uint64_t *a, const uint64_t *b, int D) {
-    int c1 = 0, c2 = 0;
-    for (int k = 0; k < 2 * D; k++) c1 += bitcount2(a[k] ^ b[k]);
-    for (int k = 0; k < D; k++) c2 += bitcount2(a[k + D] ^ b[k]) + bitcount2(a[k] ^ b[k + D]);
-    return (c1 < c2) ? c1 : c2;
+template <bool kProt>
+struct AssortLds {
+    GroupCells gc;
+    uint32_t cnt[kGroupCells][2];         // FERTILE females, males
+    uint32_t toff[kGroupCells];           // a cell's part of T
+    int64_t lid[kGroupSlots];             // ids, gather order (positions as in GroupActLds)
+    // by id rank: compared genome words (2 * D <= 4), or the agent's number of
+    // proteins and where its digests begin in the pool (-1: they do not fit)
+    uint64_t w[kProt ? 1 : kGroupSlots][4];
+    Digest pool[kProt ? kProtPool : 1];
+    int16_t np[kProt ? kGroupSlots : 1], poff[kProt ? kGroupSlots : 1];
+    uint32_t npool;
+    int16_t srt[kGroupSlots];             // id rank -> group position of the agent
+    int16_t prt[kGroupSlots];             // id rank -> the partner's rank position, -1
+    uint8_t ord[kGroupSlots];             // a round's females, from the cell's first position
+    uint8_t rmax[kGroupSlots];            // a round's largest value per female
+    // value of female i and male j of a cell at toff + i * Mp + j, Mp: M rounded
+    // up to 4 (rows are read by words; the padding is 0)
+    uint32_t T[(kGroupSlots / kAssortCell * (kAssortCell * kAssortCell / 4) + 3 * kGroupSlots) / 4];
+};
+
+constexpr int kSub = 16;   // lanes per cell in the rounds
+
+__device__ __forceinline__ int select16(uint32_t v, int k) {
+    int pos = 0, c = __popc(v & 0xFFu);
+    if (k >= c) { k -= c; v >>= 8; pos = 8; }
+    c = __popc(v & 0xFu);
+    if (k >= c) { k -= c; v >>= 4; pos += 4; }
+    c = __popc(v & 0x3u);
+    if (k >= c) { k -= c; v >>= 2; pos += 2; }
+    return pos + ((k >= (int)(v & 1u)) ? 1 : 0);
 }
 
-template <typename CtxT>
-__device__ void assort_cell_lds(const CtxT &x, const Prog &p, const StepArgs &sa, int32_t c, uint32_t s, int32_t n,
-                                AssortLds &L) {
-    const int lane = threadIdx.x;
-    const uint64_t lt = lanemask_lt();
-    const bool valid = lane < n;
-    const uint32_t slot = s + (uint32_t)lane;
-    uint8_t l = 0, g = 2;
-    int64_t id = 0;
-    int32_t h = 0;
-    if (valid) {
-        l = x.cur.life[slot];
-        g = x.cur.gender[slot];
-        id = x.cur.id[slot];
-        h = x.cur.ghandle[slot];
-        x.gmate[slot] = -1;
-    }
-    const bool isF = valid && l == QHG_LIFE_FERTILE && g == 0;
-    const bool isM = valid && l == QHG_LIFE_FERTILE && g == 1;
-    const uint64_t mF = __ballot(isF), mM = __ballot(isM);
-    const int F = __popcll(mF), M = __popcll(mM);
+// The table and the rounds of group cell k, by the 16 lanes (l) of a quarter
+// wave.  Every branch on the way is the same for the 16.
+template <bool kProt>
+__device__ __forceinline__ void assort_rounds(const Ctx &x, const Prog &p, const StepArgs &sa, AssortLds<kProt> &L, int k,
+                                              int l, uint32_t S0) {
+    const int F = (int)L.cnt[k][0], M = (int)L.cnt[k][1];
     if (F == 0 || M == 0) return;
-    if (isF) L.fid[__popcll(mF & lt)] = id;
-    if (isM) L.mid[__popcll(mM & lt)] = id;
-    wave_sync();
-    // id order (ids are distinct), then the compared genome words
-    int r = 0;
-    if (isF) for (int k = 0; k < F; k++) r += L.fid[k] < id;
-    if (isM) for (int k = 0; k < M; k++) r += L.mid[k] < id;
-    const int D = p.assort_words;
-    const uint64_t *gw = x.gpool + (int64_t)h * x.gwords;
-    uint64_t w[4] = {0, 0, 0, 0};   // constant indices only: stays in registers
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        if ((isF || isM) && k < 2 * D) w[k] = gw[k];
-    if (isF) {
-        L.fslot[r] = (int32_t)slot;
-#pragma unroll
-        for (int k = 0; k < 4; k++) L.fw[r][k] = w[k];
-        L.pf[r] = 0;
+    const int sh = (threadIdx.x & 63) & ~(kSub - 1);
+    const uint32_t lt = (1u << l) - 1u;
+    const auto votes = [&](bool v) -> uint32_t { return (uint32_t)(__ballot(v) >> sh) & 0xFFFFu; };
+    const int f0 = (int)L.gc.eb[k], m0 = f0 + (int)L.gc.n[k] - 1;   // female i at f0 + i, male j at m0 - j
+    const int32_t c = L.gc.c[k];
+    const int Mp = (M + 3) & ~3, Mw = Mp / 4;
+    uint32_t *Tw = L.T + L.toff[k] / 4;
+    uint8_t *T = reinterpret_cast<uint8_t *>(Tw);
+    const float inv = 1.0f / (float)Mp;
+    if (kProt) {
+        for (int i = l; i < F + M; i += kSub)
+            if (L.np[i < F ? f0 + i : m0 - (i - F)] > kProtBudget) atomicOr(&x.st->error, kErrProteins);
     }
-    if (isM) {
-        L.mslot[r] = (int32_t)slot;
-#pragma unroll
-        for (int k = 0; k < 4; k++) L.mw[r][k] = w[k];
-        L.pm[r] = 0;
-    }
-    wave_sync();
-    for (int t = lane; t < F * M; t += kWave) {
-        const int i = t / M, j = t - i * M;
-        L.T[t] = (uint8_t)assort_dist_w(L.fw[i], L.mw[j], D);
-    }
-    wave_sync();
-    const float cut = p.assort_cutoff;
-    // the cell's draws, computed 64 at a time and taken in order
-    uint32_t dj = 0, ubase = 0;
-    uint32_t U = assort_draw(x.seed, sa.step, c, (uint32_t)lane);
-    auto next_u = [&]() -> uint32_t {
-        if (dj - ubase >= (uint32_t)kWave) {
-            ubase = dj;
-            U = assort_draw(x.seed, sa.step, c, ubase + (uint32_t)lane);
+    for (int t = l; t < F * Mp; t += kSub) {
+        const int i = (int)(((float)t + 0.5f) * inv), j = t - i * Mp;
+        int v = 0;
+        if (j >= M) {
+        } else if (kProt) {
+            const int nf = min((int)L.np[f0 + i], kProtBudget), nm = min((int)L.np[m0 - j], kProtBudget);
+            const int of = L.poff[f0 + i], om = L.poff[m0 - j];
+            if (of >= 0 && om >= 0) {
+                for (int q = 0; q < nf; q++) {
+                    const Digest df = L.pool[of + q];
+                    for (int r = 0; r < nm; r++) {
+                        const Digest dm = L.pool[om + r];
+                        v += (df.lo == dm.lo && df.hi == dm.hi) ? 1 : 0;
+                    }
+                }
+            } else {
+                const int64_t sf = (int64_t)S0 + L.srt[f0 + i], sm = (int64_t)S0 + L.srt[m0 - j];
+                v = protein_matches(x.gprot + sf * (4 * kProtBudget), nf, x.gprot + sm * (4 * kProtBudget), nm);
+            }
+            v = ((float)v >= p.assort_cutoff) ? (v < 255 ? v : 255) : 0;
+        } else {
+            const int d = assort_dist(L.w[f0 + i], L.w[m0 - j], p.assort_words);
+            v = (d <= p.assort_dmax) ? p.assort_dmax + 1 - d : 0;
         }
-        return readlane_u32(U, (int)(dj++ - ubase));
+        T[t] = (uint8_t)v;
+    }
+    wave_sync();
+    // the cell's draws, computed 16 at a time and taken in order
+    uint32_t dj = 0, ubase = 0;
+    uint32_t U = assort_draw(x.seed, sa.step, c, (uint32_t)l);
+    const auto next_u = [&]() -> uint32_t {
+        if (dj - ubase >= (uint32_t)kSub) {
+            ubase = dj;
+            U = assort_draw(x.seed, sa.step, c, ubase + (uint32_t)l);
+        }
+        return (uint32_t)__shfl((int)U, sh + (int)(dj++ - ubase), 64);
     };
     for (int round = 0; round < F; round++) {
-        // each unpaired female's largest value at or above the cutoff among
-        // the unpaired males (0 when none; positive floats order as their bits)
-        if (lane < F) L.rmax[lane] = 0u;
+        // each female's largest value (rows and columns of the paired are 0)
+        int top = 0;
+        for (int i = l; i < F; i += kSub) {
+            uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
+            for (int j = 0; j < Mw; j++) {
+                const uint32_t v = Tw[i * Mw + j];
+                r0 = max(r0, v & 255u);
+                r1 = max(r1, (v >> 8) & 255u);
+                r2 = max(r2, (v >> 16) & 255u);
+                r3 = max(r3, v >> 24);
+            }
+            const int rm = (int)max(max(r0, r1), max(r2, r3));
+            L.rmax[f0 + i] = (uint8_t)rm;
+            top = rm > top ? rm : top;
+        }
+#pragma unroll
+        for (int d = kSub / 2; d >= 1; d >>= 1) {
+            const int o = __shfl_xor(top, d, 64);
+            top = o > top ? o : top;
+        }
+        if (top == 0) break;
         wave_sync();
-        for (int t = lane; t < F * M; t += kWave) {
-            const int i = t / M, j = t - i * M;
-            if (L.pf[i] || L.pm[j]) continue;
-            const float v = L.val[L.T[t]];
-            if (v >= cut && v > 0.f) atomicMax(&L.rmax[i], __float_as_uint(v));
+        // females reaching it, in id order
+        int np = 0;
+        for (int b = 0; b < F; b += kSub) {
+            const bool reach = b + l < F && L.rmax[f0 + b + l] == top;
+            const uint32_t mk = votes(reach);
+            if (reach) L.ord[f0 + np + __popc(mk & lt)] = (uint8_t)(b + l);
+            np += __popc(mk);
         }
         wave_sync();
-        const float rm = (lane < F) ? __uint_as_float(L.rmax[lane]) : 0.f;
-        const float vmax = wave_max_f32(rm);
-        if (!(vmax > 0.f)) break;
-        // females reaching it, in id order; lane q holds the round's entry q
-        const bool reach = lane < F && rm >= vmax;
-        const uint64_t mk = __ballot(reach);
-        const uint32_t np = (uint32_t)__popcll(mk);
-        if (reach) L.ord[__popcll(mk & lt)] = lane;
-        wave_sync();
-        int32_t ord = ((uint32_t)lane < np) ? L.ord[lane] : 0;
         if (p.assort_permute && np > 2) {
             // for i = np-1 down to 2: swap entry i with entry wrandi(0, i)
-            for (uint32_t i = np - 1; i > 1; i--) {
-                const uint32_t k = wrandi(0, i, 1, next_u());
-                const int32_t vk = (int32_t)readlane_u32((uint32_t)ord, (int)k);
-                const int32_t vi = (int32_t)readlane_u32((uint32_t)ord, (int)i);
-                ord = (lane == (int)k) ? vi : ((lane == (int)i) ? vk : ord);
+            for (int i = np - 1; i > 1; i--) {
+                const int q = (int)__umulhi((uint32_t)i, next_u());   // wrandi(0, i), exact in a double
+                if (l == 0) {
+                    const uint8_t vq = L.ord[f0 + q], vi = L.ord[f0 + i];
+                    L.ord[f0 + q] = vi;
+                    L.ord[f0 + i] = vq;
+                }
             }
-        }
-        // each female in turn: a random unpaired male at vmax
-        bool paired = false;
-        for (uint32_t q = 0; q < np; q++) {
-            const int i = (int)readlane_u32((uint32_t)ord, (int)q);
-            const bool ok = lane < M && !L.pm[lane] && L.val[L.T[i * M + lane]] >= vmax;
-            const uint64_t cm = __ballot(ok);
-            const uint32_t cnt = (uint32_t)__popcll(cm);
-            if (cnt == 0) continue;
-            const int jm = select_bit(cm, (int)wrandi(0, cnt, 1, next_u()));
-            if (lane == 0) {
-                const int32_t sf = L.fslot[i], sm = L.mslot[jm];
-                L.pf[i] = 1;
-                L.pm[jm] = 1;
-                x.gmate[sf] = sm;
-                x.gmate[sm] = sf;
-            }
-            paired = true;
             wave_sync();
         }
-        if (!paired) break;   // makeAllPairings stops at a round without pairs
+        // each female in turn: a random unpaired male at that value
+        for (int q = 0; q < np; q++) {
+            const int i = L.ord[f0 + q];
+            int cnt = 0;
+            uint32_t mk = 0;
+            for (int b = 0; b < M; b += kSub) {
+                mk = votes(b + l < M && T[i * Mp + b + l] == top);
+                cnt += __popc(mk);
+            }
+            if (cnt == 0) continue;
+            int sel = (int)__umulhi((uint32_t)cnt, next_u());
+            int jm = 0;
+            if (M <= kSub) {
+                jm = select16(mk, sel);
+            } else {
+                for (int b = 0; b < M; b += kSub) {
+                    mk = votes(b + l < M && T[i * Mp + b + l] == top);
+                    if (sel < __popc(mk)) {
+                        jm = b + select16(mk, sel);
+                        break;
+                    }
+                    sel -= __popc(mk);
+                }
+            }
+            for (int j = l; j < Mw; j += kSub) Tw[i * Mw + j] = 0;
+            for (int r = l; r < F; r += kSub) T[r * Mp + jm] = 0;
+            if (l == 0) {
+                L.prt[f0 + i] = (int16_t)(m0 - jm);
+                L.prt[m0 - jm] = (int16_t)(f0 + i);
+            }
+            wave_sync();
+        }
+        // (the first female of a round always finds a male, so every round pairs)
     }
-    wave_sync();
 }
 
-__global__ void __launch_bounds__(kWave) k_assort_pair(Ctx x, Prog p, StepArgs sa) {
-    __shared__ AssortLds lds;
+template <bool kProt>
+__global__ void __launch_bounds__(kActBlock, kProt ? 5 : 7) k_assort_pair(Ctx x, Prog p, StepArgs sa) {
+    __shared__ AssortLds<kProt> L;
+    const int par = (int)sa.parity;
     if (x.st->error) return;
-    const int64_t nocc = x.st->n_occ[sa.parity];
-    for (int k = threadIdx.x; k <= kAssortMaxDist; k += kWave)
-        lds.val[k] = (float)(1.0 - (1.0 * k) / (double)p.gen_size);
-    wave_sync();
-    for (int64_t i = blockIdx.x; i < nocc; i += gridDim.x) {
-        const OccCell e = x.occ_cur[i];
-        // the LDS form tabulates Hamming distances; AssortativePair's
-        // protein matches go through the general form
-        if (e.n <= (uint32_t)kWave && !p.assort_prot)
-            assort_cell_lds(x, p, sa, e.c, e.s, (int32_t)e.n, lds);
-        else
-            assort_cell(x, p, sa, e.c, e.s, (int32_t)e.n);
+    const int64_t ngrp = x.st->n_grp[par];
+    const int64_t mid = x.st->mid[par], nocc = x.st->n_occ[par];
+    for (int64_t g = blockIdx.x; g < ngrp; g += gridDim.x) {
+        const GroupDesc d0 = x.cur.grp[g], d1 = x.cur.grp[g + 1];
+        uint32_t i0 = readlane_u32(d0.first, 0), S0 = readlane_u32(d0.s, 0);
+        const uint32_t i1 = readlane_u32(d1.first, 0), S1 = readlane_u32(d1.s, 0);
+        while (i0 < i1) {
+            int tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));   // as in group_act
+            const uint32_t slot = S0 + (uint32_t)tid;
+            uint8_t life = 0, sex = 2;
+            int64_t id = 0;
+            int32_t h = 0;
+            if (slot < S1) {
+                life = x.cur.life[slot];
+                sex = x.cur.gender[slot];
+                id = x.cur.id[slot];
+                if (!kProt) h = x.cur.ghandle[slot];
+            }
+            int nc = (int)(i1 - i0);
+            OccCell e{0, 0, 0, 0};
+            if (tid < nc) e = x.occ_cur[i0 + (uint32_t)tid];
+            group_clear(L.gc, tid, nc);
+            for (int k = tid; k < nc * 2; k += kActBlock) (&L.cnt[0][0])[k] = 0u;
+            L.prt[tid] = -1;
+            if (tid == 0) L.npool = 0;
+            __syncthreads();
+            if (tid < nc) group_cell<kAssortCell>(L.gc, tid, e, S0);
+            __syncthreads();
+            nc = uniform_i32(L.gc.nfit);
+            if (nc == 0) {   // a cell too large for the block (assort_cell)
+                S0 += (uint32_t)uniform_i32((int)L.gc.n[0]);
+                i0++;
+                __syncthreads();
+                continue;
+            }
+            const uint32_t T = (uint32_t)uniform_i32((int)(L.gc.eb[nc - 1] + L.gc.n[nc - 1]));
+            const bool valid = (uint32_t)tid < T;
+            const int k = group_cell_of(L.gc, tid);
+            const int eb = (int)L.gc.eb[k], nk = (int)L.gc.n[k];
+            const bool isF = valid && life == QHG_LIFE_FERTILE && sex == 0;
+            const bool isM = valid && life == QHG_LIFE_FERTILE && sex == 1;
+            const int first = isF ? eb : eb + nk - 1, dirn = isF ? 1 : -1;
+            uint64_t w[4] = {0, 0, 0, 0};
+            int np = 0;
+            if (isF || isM) {
+                if (kProt) {
+                    np = x.gnprot[slot];
+                } else {
+                    const uint64_t *gw = x.gpool + (int64_t)h * x.gwords;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        if (q < 2 * p.assort_words) w[q] = gw[q];
+                }
+                const int r = (int)atomicAdd(&L.cnt[k][isF ? 0 : 1], 1u);
+                L.lid[first + dirn * r] = id;
+            }
+            __syncthreads();
+            int P = -1;
+            if (isF || isM) {
+                P = first + dirn * group_id_rank(L.lid, first, dirn, (int)L.cnt[k][isF ? 0 : 1], id);
+                L.srt[P] = (int16_t)tid;
+                if (kProt) {
+                    const int kept = np < kProtBudget ? np : kProtBudget;
+                    const int at = (int)atomicAdd(&L.npool, (uint32_t)kept);
+                    L.np[P] = (int16_t)np;
+                    L.poff[P] = (int16_t)((at + kept <= kProtPool) ? at : -1);
+                    if (at + kept <= kProtPool) {
+                        const Digest *d = reinterpret_cast<const Digest *>(x.gprot + (int64_t)slot * (4 * kProtBudget));
+                        for (int q = 0; q < kept; q++) L.pool[at + q] = d[q];
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) L.w[P][q] = w[q];
+                }
+            }
+            if (tid < kWave) {
+                // the cells' parts of the table
+                const uint32_t v = (tid < nc) ? L.cnt[tid][0] * ((L.cnt[tid][1] + 3u) & ~3u) : 0u;
+                const uint32_t incl = (uint32_t)wave_incl_scan_u64(v);
+                if (tid < nc) L.toff[tid] = incl - v;
+            }
+            __syncthreads();
+            for (int kk = tid / kSub; kk < nc; kk += kActBlock / kSub)
+                assort_rounds<kProt>(x, p, sa, L, kk, tid & (kSub - 1), S0);
+            __syncthreads();
+            if (valid) {
+                const int pp = (P >= 0) ? L.prt[P] : -1;
+                x.gmate[slot] = (pp >= 0) ? (int32_t)(S0 + (uint32_t)L.srt[pp]) : -1;
+            }
+            i0 += (uint32_t)nc;
+            S0 += T;
+            __syncthreads();   // the next pass writes the LDS read here
+        }
+    }
+    if (mid) {
+        const int lane = threadIdx.x & 63;
+        const int64_t wave = uniform_i64(((int64_t)blockIdx.x * kActBlock + threadIdx.x) / kWave);
+        const int64_t nwaves = (int64_t)gridDim.x * kActWaves;
+        for (int64_t base = wave; base < nocc; base += nwaves * kWave) {
+            OccCell e{0, 0, 0, 0};
+            if (base + lane * nwaves < nocc) e = x.occ_cur[base + lane * nwaves];
+            uint64_t left = __ballot(e.n > (uint32_t)kAssortCell);
+            while (left) {
+                const int q = __ffsll((unsigned long long)left) - 1;
+                left &= left - 1ull;
+                assort_cell(x, p, sa, (int32_t)readlane_u32((uint32_t)e.c, q), readlane_u32(e.s, q),
+                            (int32_t)readlane_u32(e.n, q));
+            }
+        }
+    }
+}
+
+// The protein digests of every FERTILE agent, before k_assort_pair: gnprot
+// and gprot by slot.  A thread finds the proteins of one strand (a walk over
+// the codons), then the block's threads hash the block's proteins, one each:
+// the hashes are most of the work and an agent's number of proteins varies,
+// so hashed agent by agent most lanes wait.  A codon is looked up in LDS (and
+// found to begin or end a protein by a mask), not in constant memory.
+constexpr int kProtAgents = kActBlock / 2;   // agents of a block
+
+struct ProteinItem {
+    uint32_t at;              // agent of the block | strand << 7 | protein of the strand << 8
+    uint32_t span;            // first codon | codons << 16
+};
+
+__global__ void __launch_bounds__(kActBlock, 3) k_proteins(Ctx x, Prog p, StepArgs sa) {
+    __shared__ ProteinItem items[kActBlock * kProtBudget];
+    __shared__ uint32_t nitems;
+    __shared__ int32_t found[2][kProtAgents], handle[kProtAgents];
+    __shared__ uint8_t amino[64];
+    const int tid = threadIdx.x;
+    const int a = tid >> 7, ag = tid & (kProtAgents - 1);   // strand, agent
+    if (x.st->error) return;
+    const int64_t n = x.st->n_alive[sa.parity];
+    const int nb = x.gwords / 2;
+    if (tid < 64) amino[tid] = codon_amino((uint32_t)tid);
+    for (int64_t base = (int64_t)blockIdx.x * kProtAgents; base < n; base += (int64_t)gridDim.x * kProtAgents) {
+        const int64_t slot = base + ag;
+        if (tid == 0) nitems = 0;
+        __syncthreads();
+        const bool lists = slot < n && x.cur.life[slot] == QHG_LIFE_FERTILE && x.cur.gender[slot] <= 1;
+        if (lists) {
+            const int32_t h = x.cur.ghandle[slot];
+            int np = 0;
+            protein_spans(x.gpool + (int64_t)h * x.gwords + (int64_t)a * nb, p.gen_size, [&](int start, int len) {
+                if (np < kProtBudget)
+                    items[atomicAdd(&nitems, 1u)] = ProteinItem{(uint32_t)ag | ((uint32_t)a << 7) | ((uint32_t)np << 8),
+                                                                (uint32_t)start | ((uint32_t)len << 16)};
+                np++;
+            });
+            found[a][ag] = np;
+            if (a == 0) handle[ag] = h;
+        }
+        __syncthreads();
+        if (lists && a == 0) x.gnprot[slot] = found[0][ag] + found[1][ag];
+        for (uint32_t t = tid; t < nitems; t += kActBlock) {
+            const ProteinItem it = items[t];
+            const int g = (int)(it.at & 127u), str = (int)(it.at >> 7) & 1;
+            const int k = (int)(it.at >> 8) + (str ? found[0][g] : 0);   // strand 1's proteins follow strand 0's
+            if (k >= kProtBudget) continue;
+            uint32_t st[4];
+            protein_md5(x.gpool + (int64_t)handle[g] * x.gwords + (int64_t)str * nb, nb, (int)(it.span & 0xFFFFu),
+                        (int)(it.span >> 16), amino, st);
+            uint32_t *out = x.gprot + (base + g) * (4 * kProtBudget) + 4 * k;
+#pragma unroll
+            for (int q = 0; q < 4; q++) out[q] = st[q];
+        }
+        __syncthreads();
     }
 }
 
@@ -1954,6 +2176,7 @@ __device__ __forceinline__ void tile_write(const CtxT &x, const StepArgs &sa, ui
             x.occ_nxt[orun] = OccCell{(int32_t)c, o, nn, 0u};
             group_ends(x.nxt.grp, x.grp_cap, sa.gdiv, (uint32_t)orun, o, nn);
             if (nn > (uint32_t)kGroupSlots) x.st->big[1 - sa.parity] = 1;
+            if (nn > (uint32_t)kAssortCell) x.st->mid[1 - sa.parity] = 1;
         }
     }
     if (threadIdx.x == 0) x.tact[tile] = 0u;

@@ -27,7 +27,7 @@ constexpr uint8_t kAaMet = 10, kAaStp = 20;
 
 // the genetic code in the reference's numbering (aTranslationTable,
 // ProteinBuilder.h:64-78): codon index -> amino acid 0..19, 20 = stop
-__constant__ uint8_t kAminoOf[64] = {
+constexpr uint8_t kAminoOf[64] = {
     8, 11, 8, 11, 16, 16, 16, 16, 14, 15, 14, 15, 7, 7, 10, 7,
     13, 6, 13, 6, 12, 12, 12, 12, 14, 14, 14, 14, 9, 9, 9, 9,
     3, 2, 3, 2, 0, 0, 0, 0, 5, 5, 5, 5, 17, 17, 17, 17,
@@ -80,36 +80,54 @@ __device__ __forceinline__ void md5_block(uint32_t (&st)[4], const uint32_t (&m)
     st[3] += d;
 }
 
-// amino acid of codon k of a strand (words w)
-__device__ __forceinline__ uint32_t codon_amino(const uint64_t *w, int32_t k) {
-    uint32_t idx = 0;
-#pragma unroll
-    for (int t = 0; t < 3; t++) {
-        const int32_t pos = 3 * k + t;
-        idx = (idx << 2) | (uint32_t)((w[pos >> 5] >> (2 * (pos & 31))) & 3u);
-    }
-    return kAminoOf[idx];
+// The 6 bits of a codon as a genome word holds them (first nucleotide lowest)
+// to its codon index, and, as masks over those bits, the codons that read as
+// amino acid aa.
+__host__ __device__ constexpr uint32_t codon_index(uint32_t v) { return ((v & 3u) << 4) | (v & 12u) | (v >> 4); }
+__host__ __device__ constexpr uint64_t codons_of(uint8_t aa) {
+    uint64_t m = 0;
+    for (uint32_t v = 0; v < 64; v++)
+        if (kAminoOf[codon_index(v)] == aa) m |= 1ull << v;
+    return m;
 }
 
-// MD5 of the protein of codons [s, e) of a strand
-__device__ __forceinline__ void protein_md5(const uint64_t *w, int32_t s, int32_t e, uint32_t (&st)[4]) {
+// the table protein_md5 reads: amino acid by a codon's 6 bits
+__device__ __forceinline__ uint8_t codon_amino(uint32_t v) {
+    uint8_t a = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 64; q++)
+        if (q == v) a = kAminoOf[codon_index(q)];
+    return a;
+}
+
+// MD5 of the protein of len codons from codon s of a strand (words w, nb of
+// them); amino: codon_amino(v) at v.
+__device__ __forceinline__ void protein_md5(const uint64_t *w, int nb, int32_t s, int32_t len, const uint8_t *amino,
+                                            uint32_t (&st)[4]) {
     st[0] = 0x67452301u;
     st[1] = 0xefcdab89u;
     st[2] = 0x98badcfeu;
     st[3] = 0x10325476u;
-    const int32_t len = e - s;
     const int32_t nblk = (len + 8) / 64 + 1;
     for (int32_t b = 0; b < nblk; b++) {
+        // the block's 64 codons from bit 0 on: every codon at a fixed place
+        const int at = 6 * (s + 64 * b), q0 = at >> 6, r = at & 63;
+        uint64_t c[7];
+#pragma unroll
+        for (int q = 0; q < 7; q++) c[q] = (q0 + q < nb) ? w[q0 + q] : 0ull;
+#pragma unroll
+        for (int q = 0; q < 6; q++) c[q] = r ? (c[q] >> r) | (c[q + 1] << (64 - r)) : c[q];
         uint32_t m[16];
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             uint32_t word = 0;
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const int32_t j = 64 * b + 4 * q + t;
-                uint32_t by = 0;
-                if (j < len) by = codon_amino(w, s + j);
-                else if (j == len) by = 0x80u;
+                const int i = 4 * q + t, lo = 6 * i, x = lo >> 6, y = lo & 63;
+                uint32_t v = (uint32_t)(c[x] >> y);
+                if (y > 58) v |= (uint32_t)(c[x + 1] << (64 - y));
+                const int32_t j = 64 * b + i;
+                const uint32_t by = (j < len) ? amino[v & 63u] : (j == len) ? 0x80u : 0u;
                 word |= by << (8 * t);
             }
             m[q] = word;
@@ -123,42 +141,39 @@ __device__ __forceinline__ void protein_md5(const uint64_t *w, int32_t s, int32_
     }
 }
 
-// Digests of an agent's proteins (genome g, gwords words, genome_size
-// nucleotides per strand) into out[4 * k] (at most kProtBudget); returns
-// the number of proteins, which may exceed the budget (then only the first
-// kProtBudget are written).  A genome of 3 nucleotides or fewer has none
-// (ProteinBuilder::init refuses it).
-__device__ __forceinline__ int32_t protein_digests(const uint64_t *g, int32_t gwords, int32_t genome_size,
-                                                   uint32_t *out) {
-    if (genome_size <= 3) return 0;
-    const int32_t nb = gwords / 2;
+// The proteins of a strand (words w, genome_size nucleotides): calls
+// found(first codon, codons) for each, in order.  A genome of 3 nucleotides or
+// fewer has none (ProteinBuilder::init refuses it).
+template <typename FoundF>
+__device__ __forceinline__ void protein_spans(const uint64_t *w, int32_t genome_size, FoundF found) {
+    if (genome_size <= 3) return;
+    constexpr uint64_t kMet = codons_of(kAaMet), kStp = codons_of(kAaStp);
     const int32_t C = genome_size / 3;
-    int32_t np = 0;
-    for (int a = 0; a < 2; a++) {
-        const uint64_t *w = g + (int64_t)a * nb;
-        bool building = false;
-        int32_t start = 0;
-        for (int32_t k = 0; k <= C; k++) {
-            // codon C stands for the strand's end
-            const uint32_t aa = (k < C) ? codon_amino(w, k) : kAaStp;
-            if (!building) {
-                if (k < C && aa == kAaMet) {
-                    building = true;
-                    start = k + 1;
-                }
-            } else if (aa == kAaStp) {
-                if (np < kProtBudget) {
-                    uint32_t st[4];
-                    protein_md5(w, start, k, st);
-#pragma unroll
-                    for (int q = 0; q < 4; q++) out[4 * np + q] = st[q];
-                }
-                np++;
-                building = false;
-            }
+    int32_t start = -1;
+    uint64_t cur = 0;       // bits read and not used yet, nbit of them
+    int nbit = 0;
+    int q = 0;
+    for (int32_t k = 0; k < C; k++) {
+        uint32_t v;
+        if (nbit >= 6) {
+            v = (uint32_t)cur & 63u;
+            cur >>= 6;
+            nbit -= 6;
+        } else {
+            const uint64_t nw = w[q++];
+            v = ((uint32_t)cur | (uint32_t)(nw << nbit)) & 63u;
+            const int used = 6 - nbit;
+            cur = nw >> used;
+            nbit = 64 - used;
+        }
+        if (start < 0) {
+            if ((kMet >> v) & 1ull) start = k + 1;
+        } else if ((kStp >> v) & 1ull) {
+            found(start, k - start);
+            start = -1;
         }
     }
-    return np;
+    if (start >= 0) found(start, C - start);   // the strand's end closes it
 }
 
 // countProtHashMatches: equal digest pairs of two agents' lists

@@ -51,9 +51,9 @@ namespace {
             return fail(QHG_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-enum KernelId { KB_ACT, KB_SCAN, KB_SCATTER, KB_GENOME, KB_CAPACITY, KB_EVAL, KB_GPOOL, KB_ASSORT, KB_COUNT };
+enum KernelId { KB_ACT, KB_SCAN, KB_SCATTER, KB_GENOME, KB_CAPACITY, KB_EVAL, KB_GPOOL, KB_ASSORT, KB_PROT, KB_COUNT };
 const char *kKernelNames[KB_COUNT] = {"k_cell_act", "k_cell_scan",     "k_cell_scatter", "k_genome",
-                                      "k_capacity", "k_eval", "k_gpool_compact", "k_assort_pair"};
+                                      "k_capacity", "k_eval", "k_gpool_compact", "k_assort_pair", "k_proteins"};
 
 constexpr int kRing = kStatusRing;
 #ifndef QHG_GROUP_AGENTS
@@ -565,6 +565,13 @@ int build_prog(qhg_pop *p) {
         g.assort_words = qhg_gpu_genome_words(blocks);
         g.assort_cutoff = (float)P.assort_cutoff;
         g.assort_permute = P.assort_permute != 0;
+        // the couples' match falls with their distance (at most 128 for the
+        // words compared): those up to dmax count
+        g.assort_dmax = -1;
+        for (int d = 0; d <= 64 * g.assort_words; d++) {
+            const float v = (float)(1.0 - (1.0 * d) / (double)P.gen_genome_size);
+            if (v >= g.assort_cutoff && v > 0.f) g.assort_dmax = d;
+        }
         g.assort_prot = p->has_prot ? 1 : 0;
     }
     p->has_me = has_kind(P, QHG_ACT_MULTIEVAL);
@@ -1199,8 +1206,14 @@ int phase_initialize(qhg_pop *p) {
     }
     if (p->has_assort) {
         // AssortativePairHam::initialize pairs in the initialize phase
-        const int grid = (int)std::min<int64_t>(p->ncells, (int64_t)p->max_grid);
-        rc = launch_bs(p, KB_ASSORT, k_assort_pair, grid, kWave, p->ctx(), p->prog, p->step_args());
+        const int kb = (int)(p->known_step & 1);
+        if (p->has_prot) {
+            const int64_t runs = (p->known.n_alive[kb] + kProtAgents - 1) / kProtAgents;
+            rc = launch_bs(p, KB_PROT, k_proteins, grid_items(p, runs), kActBlock, p->ctx(), p->prog, p->step_args());
+            if (rc) return rc;
+        }
+        rc = launch_bs(p, KB_ASSORT, p->has_prot ? k_assort_pair<true> : k_assort_pair<false>,
+                       grid_items(p, p->known.n_grp[kb]), kActBlock, p->ctx(), p->prog, p->step_args());
         if (rc) return rc;
     }
     p->initialized = true;
@@ -1552,8 +1565,11 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
     st.max_id[b] = max_id;
     st.gpool[b] = p->gwords ? n : 0;
     st.n_grp[b] = ngrp;
-    st.big[b] = 0;
-    for (const OccCell &e : occ) st.big[b] |= e.n > (uint32_t)kGroupSlots ? 1 : 0;
+    st.big[b] = st.mid[b] = 0;
+    for (const OccCell &e : occ) {
+        st.big[b] |= e.n > (uint32_t)kGroupSlots ? 1 : 0;
+        st.mid[b] |= e.n > (uint32_t)kAssortCell ? 1 : 0;
+    }
     st.step = p->steps_enqueued;
     st.error = 0;
     HIPCHK(hipMemcpyAsync(p->d_st, &st, sizeof(st), hipMemcpyHostToDevice, s));
@@ -1590,6 +1606,7 @@ int qhg_gpu_set_clock(qhg_pop *p, int64_t step, double t, int64_t max_id) {
         std::swap(st.gpool[0], st.gpool[1]);
         std::swap(st.n_grp[0], st.n_grp[1]);
         std::swap(st.big[0], st.big[1]);
+        std::swap(st.mid[0], st.mid[1]);
     }
     st.max_id[nb] = std::max(st.max_id[nb], max_id);
     st.step = step;
@@ -1799,6 +1816,7 @@ int qhg_gpu_env_event(qhg_pop *p, const qhg_env_desc *env, int32_t events) {
             std::swap(st.gpool[0], st.gpool[1]);
             std::swap(st.n_grp[0], st.n_grp[1]);
             std::swap(st.big[0], st.big[1]);
+            std::swap(st.mid[0], st.mid[1]);
             HIPCHK(hipMemcpyAsync(p->d_st, &st, sizeof(st), hipMemcpyHostToDevice, p->stream));
             HIPCHK(hipStreamSynchronize(p->stream));
             p->known = st;

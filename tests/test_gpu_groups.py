@@ -155,3 +155,57 @@ def test_scan_tiles_match_the_oracle(width, height):
         assert_same_state(gpu.agents(), ora.agents(), "step %d" % (3 * k + 3))
         assert np.array_equal(gpu.getNumAgentsArray(), ora.cell_counts())
     gpu.close()
+
+
+def _protein_genomes(rng, n, genome_size, proteins):
+    """Genomes of about that many proteins per agent: Met, a few codons and a
+    stop, again and again, with a few nucleotides changed per agent."""
+    words = 2 * abi.genome_words(genome_size)
+    nuc = rng.integers(0, 4, 32 * words)
+    per = (2 * genome_size // 3) // max(1, proteins)
+    for strand in range(2):
+        at = strand * 16 * words
+        for k in range(0, genome_size // 3 - 3, max(3, per)):
+            nuc[at + 3 * k:at + 3 * k + 3] = (0, 3, 2)                    # Met
+            nuc[at + 3 * (k + 2):at + 3 * (k + 2) + 3] = (3, 0, 0)        # stop
+    g = np.tile(nuc, (n, 1))
+    for _ in range(3):
+        g[np.arange(n), rng.integers(0, 32 * words, n)] = rng.integers(0, 4, n)
+    g = g.reshape(n, words, 32).astype(np.uint64) << (2 * np.arange(32)).astype(np.uint64)
+    return np.ascontiguousarray(g.sum(axis=2, dtype=np.uint64).ravel())
+
+
+@pytest.mark.parametrize("kind", ["edges", "ones", "sixes", "hundreds", "mixed", "alone"])
+@pytest.mark.parametrize("model", ["hamming", "hamming_noperm", "hamming_long", "protein", "protein_many"])
+def test_assortative_groups_match_the_oracle(kind, model):
+    """k_assort_pair at the same edges: 16 lanes per cell, tables of several
+    cells, cells too large for a block; digests in the block's pool and past it."""
+    rng = np.random.default_rng(51)
+    prot = model.startswith("protein")
+    size = 1100 if model == "hamming_long" else 256
+    sc = scenarios.c2(seed=51, level=3, n_agents=10, patch_cells=5, genetics=True, genome_size=size, protein=prot,
+                      assort=((1.0, 1) if prot else (0.9, 0 if model == "hamming_noperm" else 1)))
+    sc["params"].npp_k_max = 600.0
+    n = _counts(kind, sc["grid"]["num_cells"], rng)
+    cell = np.repeat(np.arange(len(n)), n).astype(np.int32)
+    m = len(cell)
+    age = rng.uniform(0, 40, m)
+    sc["agents"] = {
+        "id": rng.permutation(np.arange(1, 3 * m + 1, dtype=np.int64))[:m], "cell": cell,
+        "life": np.full(m, abi.QHG_LIFE_FERTILE, dtype=np.uint8), "gender": (rng.random(m) < 0.5).astype(np.uint8),
+        "birth_time": -age, "age": age, "last_birth": np.full(m, -5.0), "mate_id": np.full(m, -3, dtype=np.int64),
+        "num_babies": np.zeros(m, dtype=np.int32),
+        "genome": (_protein_genomes(rng, m, size, 12 if model == "protein_many" else 4) if prot
+                   else scenarios.initial_genomes(rng, m, size))}
+    gpu, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    gpu.preLoop()
+    ora.pre_loop()
+    paired = 0
+    for k in range(5):
+        gpu.run(1)
+        ora.run(1)
+        got = gpu.agents()
+        assert_same_state(got, ora.agents(), "%s %s step %d" % (kind, model, k))
+        paired += int((got["mate_id"] >= 0).sum())
+    assert paired > 0 or kind in ("ones", "alone")
+    gpu.close()
