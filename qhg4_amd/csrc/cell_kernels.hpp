@@ -64,7 +64,6 @@ constexpr int kScanPer = 1;           // cells per k_cell_scan thread
 constexpr int kCellTile = kScanBlock * kScanPer;   // cells per look-back tile
 constexpr int kMaxCross = 32;         // device limit on Genetics_num_crossover
 constexpr int kStatusRing = 8;        // host-mapped status snapshots
-constexpr int kStatusSealEvery = 4;   // steps whose snapshot k_cell_scatter seals for the host
 
 constexpr int32_t kErrCapacity = 1;   // the next population does not fit
 constexpr int32_t kErrGather = 8;     // an internal count disagreed
@@ -2309,6 +2308,17 @@ __global__ void __launch_bounds__(kScanBlock) k_cell_scan(Ctx x, StepArgs sa) {
 // ---------------------------------------------------------------------------
 // k_cell_scatter: every agent's record to its place in the next buffer
 // ---------------------------------------------------------------------------
+// A step's status snapshot for the host: its words go straight to host memory
+// (system-scope stores), and once they are there the step's number into the
+// seal word of the snapshot's slot (after the kStatusRing snapshots).  The
+// host polls the seal, while the step's agents are still being moved, and
+// nothing has to mark the stream.  No cache is written back for it: only
+// these words are meant for the host.
+__device__ __forceinline__ void host_store(uint64_t *at, uint64_t v) {
+    __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void host_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // an agent's record as it leaves the current buffer
 struct ScatItem {
     uint64_t w;               // outcome word
@@ -2439,16 +2449,10 @@ __global__ void __launch_bounds__(kScatterBlock) k_cell_scatter(Ctx x, StepArgs 
                                   readlane_u32((uint32_t)w, kStep);
             const int64_t slot = (int64_t)(step % (uint64_t)kStatusRing);
             uint64_t *dst = reinterpret_cast<uint64_t *>(x.hring + slot);
-            if (lane < kWords) dst[lane] = w;
-            if (step % (uint64_t)kStatusSealEvery == 0) {
-                // the seal words follow the kStatusRing snapshots: the step
-                // goes there once the snapshot is visible to the host (a
-                // system-scope release), and the host polls it instead of
-                // waiting on an event between two steps' kernels
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-                int64_t *seal = reinterpret_cast<int64_t *>(x.hring + kStatusRing) + slot;
-                if (lane == 0) __hip_atomic_store(seal, (int64_t)step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+            if (lane < kWords) host_store(&dst[lane], w);
+            host_stores_done();
+            int64_t *seal = reinterpret_cast<int64_t *>(x.hring + kStatusRing) + slot;
+            if (lane == 0) host_store(reinterpret_cast<uint64_t *>(seal), step);
         }
         return;
     }
@@ -2916,19 +2920,17 @@ __global__ void __launch_bounds__(kScatterBlock) k_batch_scatter(BatchArgs B) {
             if (hr) {
                 const uint64_t *srcw = reinterpret_cast<const uint64_t *>(st);
                 uint64_t *dstw = reinterpret_cast<uint64_t *>(hr + (st->step % kStatusRing));
-                for (int w = 0; w < (int)(sizeof(DevStatus) / 8); w++) dstw[w] = srcw[w];
+                for (int w = 0; w < (int)(sizeof(DevStatus) / 8); w++) host_store(&dstw[w], srcw[w]);
             }
         }
-        // every member's snapshot of a step divisible by kStatusSealEvery is
-        // sealed with its step, as k_cell_scatter does, once all of them are
-        // visible to the host (one system-scope release for the wave)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+        // every member's snapshot is sealed with its step, as k_cell_scatter does
+        host_stores_done();
         for (int r = lane; r < B.npops; r += kWave) {
             const int64_t step = pop_desc(B, r).ctx[0].st->step;
             DevStatus *hr = pop_desc(B, r).ctx[0].hring;
-            if (hr && step % kStatusSealEvery == 0) {
+            if (hr) {
                 int64_t *seal = reinterpret_cast<int64_t *>(hr + kStatusRing) + step % kStatusRing;
-                __hip_atomic_store(seal, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(reinterpret_cast<uint64_t *>(seal), (uint64_t)step);
             }
         }
         return;

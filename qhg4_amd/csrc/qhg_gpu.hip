@@ -183,6 +183,7 @@ struct qhg_pop {
     bool me_done = false;
     bool acted = false;       // k_cell_act launched for the current step
     bool initialized = false; // initialize phase done for the current step
+    bool snap_ok = false;     // the last step's snapshot is the status (nothing changed it since)
     bool looked = false;      // the current step's outcomes were written into the records (k_act_commit)
     double t_next = 0.0;      // time of the next step
 
@@ -758,7 +759,43 @@ int run_evaluators(qhg_pop *p) {
     return 0;
 }
 
+int64_t seal_of(const qhg_pop *p, int k) { return __atomic_load_n(p->h_seal + k, __ATOMIC_ACQUIRE); }
+
+// Wait until the snapshot of `step` is sealed (0), or the stream has drained
+// without it (1: a step that finds the device error flag set writes no
+// snapshot, and a batch member's step no longer advances).  The stream is
+// asked only every 2 ms of waiting: each query puts a marker into the stream,
+// which holds the GPU idle like an event does.
+int wait_sealed(qhg_pop *p, int64_t step) {
+    using clk = std::chrono::steady_clock;
+    const int k = (int)(step % kRing);
+    if (seal_of(p, k) == step) return 0;
+    auto next_query = clk::now() + std::chrono::milliseconds(2);
+    for (uint32_t spin = 1;; spin++) {
+        if (seal_of(p, k) == step) return 0;
+        if (spin % 1024 == 0 && clk::now() >= next_query) {
+            const hipError_t e = hipStreamQuery(p->stream);
+            if (e == hipSuccess) return seal_of(p, k) == step ? 0 : 1;
+            if (e != hipErrorNotReady) return fail(QHG_ERR_HIP, std::string("status wait: ") + hipGetErrorString(e));
+            next_query = clk::now() + std::chrono::milliseconds(2);
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// The status as of everything enqueued.  After a step it is the snapshot the
+// step's scatter writes to the host, complete before the scatter is (20 us per
+// call with a copy and a synchronization, 1-2 us beyond the step's own time
+// with it); otherwise it is copied.
 int read_status_sync(qhg_pop *p, DevStatus *out) {
+    if (p->snap_ok && !p->acted && !p->initialized) {
+        const int rc = wait_sealed(p, p->steps_enqueued);
+        if (rc < 0) return rc;
+        if (rc == 0) {
+            std::memcpy(out, (const void *)&p->h_ring[p->steps_enqueued % kRing], sizeof(*out));
+            return 0;
+        }
+    }
     HIPCHK(hipMemcpyAsync(out, p->d_st, sizeof(DevStatus), hipMemcpyDeviceToHost, p->stream));
     HIPCHK(hipStreamSynchronize(p->stream));
     return 0;
@@ -987,6 +1024,7 @@ int compact_pool(qhg_pop *p, int64_t new_gcap) {
         HIPCHK(hipMalloc(&p->d_gpool[other], (size_t)new_gcap * p->gwords * 8));
     }
     const int32_t par = p->cur();
+    p->snap_ok = false;
     int rc = launch(p, KB_GPOOL, k_gpool_compact, p->num_cu * 8, p->ctx(), p->d_gpool[other], par);
     if (rc) return rc;
     hipLaunchKernelGGL(k_gpool_commit, dim3(p->num_cu * 4), dim3(256), 0, p->stream, p->ctx(), par);
@@ -1041,8 +1079,6 @@ int grow_agents(qhg_pop *p, int64_t new_cap, int64_t n) {
     return alloc_slot_scratch(p, new_cap);
 }
 
-int64_t seal_of(const qhg_pop *p, int k) { return __atomic_load_n(p->h_seal + k, __ATOMIC_ACQUIRE); }
-
 void clear_seals(qhg_pop *p) {
     for (int k = 0; k < kRing; k++) __atomic_store_n(p->h_seal + k, (int64_t)-1, __ATOMIC_RELAXED);
 }
@@ -1068,27 +1104,13 @@ void poll_ring(qhg_pop *p) {
         if (p->ring_step[k] >= 0 && p->ring_step[k] <= p->known_step) p->ring_step[k] = -1;
 }
 
-// Wait until slot k is sealed.  A step that finds the device error flag set
-// writes no snapshot (a batch member's step no longer advances): once the
-// stream has drained, the status itself is read.  The stream is asked only every 2 ms of waiting: each query puts a
-// marker into the stream, which holds the GPU idle like an event does.
+// Wait until slot k is sealed, or read the status itself once the stream has
+// drained without it.
 int wait_seal(qhg_pop *p, int k) {
-    using clk = std::chrono::steady_clock;
-    auto next_query = clk::now() + std::chrono::milliseconds(2);
-    for (uint32_t spin = 1;; spin++) {
-        if (seal_of(p, k) == p->ring_step[k]) return 0;
-        if (spin % 1024 == 0 && clk::now() >= next_query) {
-            const hipError_t e = hipStreamQuery(p->stream);
-            if (e == hipSuccess) {
-                if (seal_of(p, k) == p->ring_step[k]) return 0;
-                for (int j = 0; j < kRing; j++) p->ring_step[j] = -1;
-                return refresh_known(p);
-            }
-            if (e != hipErrorNotReady) return fail(QHG_ERR_HIP, std::string("status wait: ") + hipGetErrorString(e));
-            next_query = clk::now() + std::chrono::milliseconds(2);
-        }
-        __builtin_ia32_pause();
-    }
+    const int rc = wait_sealed(p, p->ring_step[k]);
+    if (rc != 1) return rc;
+    for (int j = 0; j < kRing; j++) p->ring_step[j] = -1;
+    return refresh_known(p);
 }
 
 // oldest step whose snapshot the host has not consumed (or -1)
@@ -1175,13 +1197,13 @@ int ensure_capacity(qhg_pop *p) {
     return 0;
 }
 
-// Every step's scatter writes its status snapshot into the ring and seals
-// it every kStatusSealEvery steps; the host reads the sealed ones.  No event
+// Every step's scatter writes its status snapshot into the ring and seals it;
+// the host looks at every kRingEvery-th while it runs ahead.  No event
 // marks them: an event is a packet of its own between two steps' kernels and
 // holds the GPU idle for a few microseconds (the kernel trace shows ~5.6 us
 // before a step's first kernel after each one), and a snapshot a few steps
 // old bounds the capacity just as well.
-constexpr int kRingEvery = kStatusSealEvery;
+constexpr int kRingEvery = 4;
 static_assert(kRing % kRingEvery == 0 && kRing / kRingEvery >= 2, "ring slots for the sealed steps");
 
 int enqueue_readback(qhg_pop *p) {
@@ -1262,6 +1284,7 @@ int phase_finalize(qhg_pop *p) {
     p->initialized = false;
     p->steps_enqueued++;
     p->t_next += 1.0;
+    p->snap_ok = true;
     return enqueue_readback(p);
 }
 
@@ -1558,6 +1581,7 @@ int qhg_gpu_upload_agents(qhg_pop *p, const qhg_agents *a) {
         }
     }
     DevStatus st;
+    p->snap_ok = false;
     HIPCHK(hipMemcpyAsync(&st, p->d_st, sizeof(st), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     st.n_alive[b] = n;
@@ -1591,6 +1615,7 @@ int qhg_gpu_set_clock(qhg_pop *p, int64_t step, double t, int64_t max_id) {
     for (int k = 0; k < kRing; k++) p->ring_step[k] = -1;
     // the steps may run again from an earlier one: no old seal may match
     clear_seals(p);
+    p->snap_ok = false;
     DevStatus st;
     int rc = read_status_sync(p, &st);
     if (rc) return rc;
@@ -1793,6 +1818,7 @@ int qhg_gpu_env_event(qhg_pop *p, const qhg_env_desc *env, int32_t events) {
         if (rc) return rc;
         const int b = p->cur();
         if (st.n_occ[b] > 0) {
+            p->snap_ok = false;
             // d_tmp (ncells doubles) holds the kept cells' old segment starts
             uint32_t *src_s = reinterpret_cast<uint32_t *>(p->d_tmp);
             rc = launch_bs(p, KB_CAPACITY, k_env_kill, 1, kKillBlock, (const OccCell *)p->d_occ[b], st.n_occ[b],
@@ -2069,6 +2095,7 @@ int qhg_gpu_autotune(qhg_pop *p, int32_t trial_steps, qhg_tuning *chosen, int32_
         r = qhg_gpu_run(p, trial_steps);
         if (r) return r;
         HIPCHK(hipEventRecord(tm.e1, p->stream));
+        HIPCHK(hipEventSynchronize(tm.e1));
         r = refresh_known(p);
         if (r) return r;
         float ms = 0;
@@ -2441,6 +2468,7 @@ int qhg_batch_run(qhg_batch *b, int32_t nsteps) {
         for (qhg_pop *p : b->pops) {
             p->steps_enqueued++;
             p->t_next += 1.0;
+            p->snap_ok = true;
         }
         // each member's snapshots are sealed by k_batch_scatter; no event
         // goes into the stream
