@@ -92,9 +92,9 @@ def kernel_bytes(bm, d, grid, ops, gwords):
     per_surv = bm["SCAT_SURVIVOR"] + (bm["SCAT_SURVIVOR_GEN"] if gwords else 0)
     per_birth = bm["SCAT_BIRTH"] + (bm["SCAT_BIRTH_GEN"] if gwords else 0)
     scat = occ * bm["SCAT_OCC"] + live * bm["SCAT_LIVE"] + survivors * per_surv + births * per_birth
-    out = {"k_cell_act": act, "k_cell_scan": scan, "k_cell_scatter": scat}
     if gwords:
-        out["k_genome"] = births * bm["SCAT_GENOME_WORDS"] * gwords * 8
+        scat += births * bm["SCAT_GENOME_WORDS"] * gwords * 8
+    out = {"k_cell_act": act, "k_cell_scan": scan, "k_cell_scatter": scat}
     if abi.ACT_ASSORTPAIR in ops and gwords:
         # words per strand position the distance compares (the block count
         # read as a genome size, as AssortativePairHam passes it)

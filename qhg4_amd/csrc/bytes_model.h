@@ -56,7 +56,7 @@
 #define QHG_B_ASSORT_LIVE       14  /* life r 1 + gender r 1 + id r 8 + partner slot w 4    */
 #define QHG_B_ASSORT_FERTILE     4  /* genome handle r 4, + 2 x D x 8 genome words r          */
 
-/* k_genome (Genetics::makeOffspring), per birth */
+/* and, with Genetics (Genetics::makeOffspring), per birth */
 #define QHG_B_SCAT_GENOME_WORDS  3  /* x gwords x 8: two parent genomes r + child w          */
 
 #endif

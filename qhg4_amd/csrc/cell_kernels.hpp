@@ -5,8 +5,8 @@
 // next, swapped every step).  Inside a segment the order is the one the
 // previous step wrote (stayers, then arrivals per incoming neighbour slot,
 // then newborns); every order-dependent rule sorts by agent id itself, so
-// results do not depend on it.  A step is three launches (four with
-// Genetics), none with global atomics on agent data:
+// results do not depend on it.  A step is three launches, none with global
+// atomics on agent data:
 //
 //   k_cell_act      one block per group of consecutive occupied cells:
 //                   RandomPair::initialize / findMates on the cells' segments
@@ -26,15 +26,16 @@
 //                   plus its place, a mother's newborn after the arrivals of
 //                   its cell in mother-id order (performMoves,
 //                   recycleDeadSpaceNew, createAgentAtIndex,
-//                   makePopSpecificOffspring; SPopulation.cpp:596-918).
-//   k_genome        one thread per birth: Genetics::makeOffspring
-//                   (Genetics.cpp:285-337) into the genome pool.
+//                   makePopSpecificOffspring; SPopulation.cpp:596-918),
+//                   with Genetics its genome (Genetics::makeOffspring,
+//                   Genetics.cpp:285-337) into the genome pool.
 //
 // Per-cell tables (count, K, weights, neighbours) are read once per cell.
 // Genomes live in a pool addressed by a per-agent handle, so they are only
 // touched at births and at occasional pool compactions.
 #pragma once
 #include <cstddef>
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -165,7 +166,6 @@ struct Ctx {
     int64_t grp_cap;          // entries of a buffer's group list
     uint64_t *dec;            // per slot of the current buffer: outcome word
     uint64_t *brank;          // per mother's slot: cell | rank among the cell's births << 32
-    int32_t *brec;            // per birth: mother slot, father slot (Genetics)
     int32_t *gmate;           // per slot: the partner's slot, -1 unpaired
     int32_t *gfu, *gmu, *gfs, *gms;           // per-slot list scratch of large cells
     int64_t *gfid, *gmid;
@@ -2306,6 +2306,92 @@ __global__ void __launch_bounds__(kScanBlock) k_cell_scan(Ctx x, StepArgs sa) {
 }
 
 // ---------------------------------------------------------------------------
+// genetics: GeneUtils::makeMultiMask / crossOver / freeReco / mutateNucs
+// (GeneUtils.cpp:112-246, :322-360), one genome word per lane
+// ---------------------------------------------------------------------------
+
+// bits lo..hi (inclusive, lo <= hi <= 63)
+__device__ __forceinline__ uint64_t bit_range(int lo, int hi) {
+    const uint64_t up = (hi >= 63) ? ~0ull : ((1ull << (hi + 1)) - 1ull);
+    return up & ~((1ull << lo) - 1ull);
+}
+
+// The draws of a child genome follow makeOffspring's order (Genetics.cpp:
+// 285-337): i1, i2, the mother's crossover draws, the father's, the mutation
+// count, then (position, mask) pairs.  The number of the mutation count:
+__device__ __forceinline__ uint32_t mutation_draw(int cross, int nbk) {
+    return cross > 0 ? 2 + 2 * (uint32_t)cross : cross == -1 ? 2 + 4 * (uint32_t)nbk : 2;
+}
+
+// Word w of a child genome: strand s = w / nbk comes from parent s (0 mother,
+// 1 father), block b = w % nbk; g0, g1: block b of that parent's strands; D:
+// the child's draws (sel_draw: number s of them, i1 for the mother, i2 for the
+// father); k: its mutations; those that hit this word apply here.
+template <typename ProgT, typename DrawF>
+__device__ __forceinline__ uint64_t child_word(const ProgT &p, DrawF D, uint32_t sel_draw, int k, uint64_t g0, uint64_t g1,
+                                               int s, int b, int nbk, int w) {
+    const int sel = (int)(2 * 1.0 * wrandd(sel_draw));
+    const int C = p.gen_cross;
+    uint64_t word;
+    const uint32_t nmut = mutation_draw(C, nbk);
+    if (C > 0) {
+        // GeneUtils::crossOver (GeneUtils.cpp:184-246) restricted to block b:
+        // this parent's breaks are draws 2 + s*C + q, q < C
+        const uint32_t nbits = (uint32_t)nbk * 64u;
+        int before = 0, in = 0;
+        for (int q = 0; q < C; q++) {
+            const uint32_t bp = wrandi(0, nbits, 2, D(2 + (uint32_t)(s * C + q)));
+            before += (int)(bp >> 6) < b;
+            in += (int)(bp >> 6) == b;
+        }
+        const bool cur = before & 1;
+        const uint64_t gc = cur ? g1 : g0, go = cur ? g0 : g1;
+        uint64_t L = ~0ull;
+        if (in) {
+            // makeMultiMask (GeneUtils.cpp:156-175) over the block's breaks in
+            // draw order, walked from the last: bit 63-j takes the current
+            // value; a break at bit v flips it at j = 64-v, but only if that j
+            // is still ahead, otherwise the walk stops there (unsorted breaks,
+            // repeats and breaks at bit 0 included)
+            uint32_t on = 1u - (uint32_t)(in % 2);
+            int jc = 0;
+            uint64_t m = 0;
+            for (int q = C - 1; q >= 0; q--) {
+                const uint32_t bp = wrandi(0, nbits, 2, D(2 + (uint32_t)(s * C + q)));
+                if ((int)(bp >> 6) != b) continue;
+                const int t = 64 - (int)(bp & 63u);
+                if (t > 63 || t <= jc) break;
+                if (on) m |= bit_range(64 - t, 63 - jc);
+                on = 1u - on;
+                jc = t;
+            }
+            if (on) m |= bit_range(0, 63 - jc);
+            L = m;
+        }
+        word = (sel == 0) ? ((L & gc) | (~L & go)) : ((L & go) | (~L & gc));
+    } else if (C == -1) {
+        // freeReco + makeFreeMask (GeneUtils.cpp:322-360): two draws per block
+        const uint32_t n0 = 2 + (uint32_t)(s * 2 * nbk + 2 * b);
+        uint64_t v = ((uint64_t)D(n0) << 32) + D(n0 + 1);
+        v &= 0x5555555555555555ull;
+        v += v << 1;
+        word = (sel == 0) ? ((v & g0) | (~v & g1)) : ((v & g1) | (~v & g0));
+    } else {
+        word = sel ? g1 : g0;
+    }
+    // GeneUtils::mutateNucs (GeneUtils.cpp:112-141)
+    const uint32_t nbits_all = 2u * 2u * (uint32_t)p.gen_size;
+    for (int j = 0; j < k; j++) {
+        const uint32_t bp = wrandi(0, nbits_all, 2, D(nmut + 1 + 2 * (uint32_t)j));
+        if ((int)(bp >> 6) == w) {
+            const uint64_t mk = (uint64_t)wrandi(1, 4, 1, D(nmut + 2 + 2 * (uint32_t)j));
+            word ^= mk << (bp & 63u);
+        }
+    }
+    return word;
+}
+
+// ---------------------------------------------------------------------------
 // k_cell_scatter: every agent's record to its place in the next buffer
 // ---------------------------------------------------------------------------
 // A step's status snapshot for the host: its words go straight to host memory
@@ -2348,36 +2434,56 @@ __device__ __forceinline__ void scatter_load(const CtxT &x, const StepArgs &sa, 
     if (x.gwords) a.gh = x.cur.ghandle[i];
 }
 
-// One agent, and its newborn: createAgentAtIndex + makePopSpecificOffspring
-// (SPopulation.cpp:880-918); new ids rank births by (cell, mother id).
+// Where a record and a newborn go (-1: nowhere).
+struct ScatPlan {
+    int64_t to, nto;          // next-buffer slots of the agent and of its newborn
+    int64_t rg;               // the newborn's rank among the step's births
+    int32_t fh;               // Genetics: the father's handle
+};
+
 template <typename CtxT>
-__device__ __forceinline__ void scatter_agent(const CtxT &x, const StepArgs &sa, int64_t i, const ScatItem &a,
-                                              int64_t max_id, int64_t gbase) {
+__device__ __forceinline__ ScatPlan scatter_plan(const CtxT &x, const StepArgs &sa, int64_t i, ScatItem &a) {
+    ScatPlan pl{-1, -1, -1, 0};
     const uint32_t kind = (uint32_t)(a.w >> kDecKindAt) & 3u;
     const bool birth = (a.w & kDecBirth) != 0;
     uint64_t br = 0;
-    if (birth) br = x.brank[i];
+    if (birth) {
+        br = x.brank[i];
+        if (x.gwords) pl.fh = x.cur.ghandle[a.gmate];
+    }
+    if (sa.mates && a.gmate >= 0) a.mate = x.cur.id[a.gmate];
     if (kind != kDecDead) {
         const uint32_t *table = (kind == kDecStay) ? x.off_nxt : (kind == kDecMove) ? x.rpos : x.nav.rpos;
-        const uint32_t at = table[(uint32_t)a.w];
-        int64_t mate = a.mate;
-        if (sa.mates && a.gmate >= 0) mate = x.cur.id[a.gmate];
-        const int64_t to = (int64_t)at + ((uint32_t)(a.w >> kDecRankAt) & kDecRankMask);
+        pl.to = (int64_t)table[(uint32_t)a.w] + ((uint32_t)(a.w >> kDecRankAt) & kDecRankMask);
+    }
+    if (birth) {
+        const uint32_t c = (uint32_t)br, r = (uint32_t)(br >> 32);
+        pl.nto = (int64_t)x.bpos[c] + r;
+        pl.rg = (int64_t)x.birth_off[c] + r;
+    }
+    return pl;
+}
+
+// One agent, and its newborn: createAgentAtIndex + makePopSpecificOffspring
+// (SPopulation.cpp:880-918); new ids rank births by (cell, mother id).
+template <typename CtxT>
+__device__ __forceinline__ void scatter_write(const CtxT &x, const StepArgs &sa, const ScatItem &a, const ScatPlan &pl,
+                                              int64_t max_id, int64_t gbase) {
+    if (pl.to >= 0) {
+        const int64_t to = pl.to;
         x.nxt.id[to] = a.id;
         x.nxt.birth[to] = a.birth;
         x.nxt.age[to] = sa.sets_age ? sa.t - a.birth : a.age;
         x.nxt.lastb[to] = a.lastb;
-        x.nxt.nbabies[to] = a.nbab + ((birth && !(a.w & kDecCounted)) ? 1 : 0);
+        x.nxt.nbabies[to] = a.nbab + ((pl.rg >= 0 && !(a.w & kDecCounted)) ? 1 : 0);
         x.nxt.gender[to] = a.g;
         x.nxt.life[to] = !sa.sets_life ? a.life : (a.w & kDecFertile) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
         if (x.gwords) x.nxt.ghandle[to] = a.gh;
-        x.nxt.mate_id[to] = mate;
+        x.nxt.mate_id[to] = a.mate;
     }
-    if (birth) {
-        const uint32_t c = (uint32_t)br, r = (uint32_t)(br >> 32);
-        const int64_t to = (int64_t)x.bpos[c] + r;
-        const int64_t rg = (int64_t)x.birth_off[c] + r;
-        const int64_t nid = max_id + 1 + rg;
+    if (pl.rg >= 0) {
+        const int64_t to = pl.nto;
+        const int64_t nid = max_id + 1 + pl.rg;
         x.nxt.id[to] = nid;
         x.nxt.mate_id[to] = -3;
         x.nxt.birth[to] = sa.t;
@@ -2388,11 +2494,79 @@ __device__ __forceinline__ void scatter_agent(const CtxT &x, const StepArgs &sa,
         const uint8_t gg = (uint8_t)(2 * wrandd(u));
         x.nxt.gender[to] = gg;
         x.nxt.life[to] = (gg == 0) ? QHG_LIFE_FERTILE : QHG_LIFE_ALIVE;
-        if (x.gwords) {
-            x.nxt.ghandle[to] = (int32_t)(gbase + rg);
-            x.brec[2 * rg] = (int32_t)i;
-            x.brec[2 * rg + 1] = a.gmate;
+        if (x.gwords) x.nxt.ghandle[to] = (int32_t)(gbase + pl.rg);
+    }
+}
+
+// The genomes of a wave's newborns, by all its lanes.  rg: this lane's newborn
+// (ScatPlan), gh, fh: its parents' handles.  A lane per genome word, as many
+// births at once as fit the wave; a birth's lanes first draw for it together,
+// four numbers each, kept in the wave's part of LDS (sd), and search the
+// binomial table together.  Here, beside the records, the births need no list
+// and no launch of their own.  Bound by instructions (about a thousand per
+// pass of a wave, half of them draws and f64 conversions), not by the rows or
+// the occupancy: limits of 6 to 8 waves per SIMD spill and are slower.  With
+// 16 words per genome, at 369 k agents (1.39 M) records and genomes in two
+// kernels, every word's lane drawing for itself, took 36 us (82); one kernel
+// in which each mother's lane drew, 31 (84); so 21 (74).
+template <typename CtxT, typename ProgT>
+__device__ __forceinline__ void scatter_genomes(const CtxT &x, const ProgT &p, const StepArgs &sa, int64_t rg, int32_t gh,
+                                                int32_t fh, int64_t max_id, int64_t gbase, uint32_t *sd) {
+    const int lane = threadIdx.x & 63;
+    uint64_t left = __ballot(rg >= 0);
+    if (!left) return;
+    const int gw = x.gwords, nbk = gw / 2;
+    const int per_lane = (gw <= kWave) ? gw : kWave;      // lanes per birth
+    const int per = kWave / per_lane, pb = lane / per_lane, li = lane - pb * per_lane;
+    const uint64_t lanes = (per_lane == kWave) ? ~0ull : (1ull << per_lane) - 1ull;
+    const uint32_t nd = 4u * (uint32_t)per_lane;
+    while (left) {
+        const bool on = pb < per && pb < __popcll(left);
+        const int src = select_bit(left, on ? pb : 0);
+        const int64_t r = (int64_t)__shfl((long long)rg, src, 64);
+        const int64_t hm = __shfl(gh, src, 64), hf = __shfl(fh, src, 64);
+        const uint64_t nid = (uint64_t)(max_id + 1 + r);
+        int w = li, s = (w >= nbk) ? 1 : 0, b = w - s * nbk;
+        uint64_t g0 = 0, g1 = 0;
+        if (on) {
+            const uint64_t *par = x.gpool + (s ? hf : hm) * gw + b;
+            g0 = par[0];
+            g1 = par[nbk];
         }
+        uint32_t o[4];
+        draw4(x.seed, sa.step, QHG_STREAM_GENETICS, nid, (uint32_t)li, o);
+        wave_sync();
+        *reinterpret_cast<uint4 *>(&sd[4 * lane]) = make_uint4(o[0], o[1], o[2], o[3]);
+        wave_sync();
+        const uint32_t *mine = sd + (on ? (uint32_t)pb * nd : 0u);
+        auto D = [&](uint32_t n) -> uint32_t {
+            return (n < nd) ? mine[n] : draw(x.seed, sa.step, QHG_STREAM_GENETICS, nid, n);
+        };
+        int k = 0;
+        if (p.nbino > 0) {
+            // BinomialDist::getN: the first entry that the draw does not exceed
+            const double v = wrandd(D(mutation_draw(p.gen_cross, nbk)));
+            k = -1;
+            for (int e = li; __ballot(on && k < 0); e += per_lane) {
+                const double cdf = (e < p.nbino) ? p.bino[e] : 2.0;
+                const uint64_t ok = (__ballot(!(v > cdf)) >> (pb * per_lane)) & lanes;
+                if (k < 0 && ok) k = e - li + __ffsll((unsigned long long)ok) - 1;
+            }
+        }
+        if (on) {
+            uint64_t *out = x.gpool + (gbase + r) * gw;
+            for (;;) {
+                out[w] = child_word(p, D, mine[s], k, g0, g1, s, b, nbk, w);
+                w += per_lane;
+                if (w >= gw) break;
+                s = (w >= nbk) ? 1 : 0;
+                b = w - s * nbk;
+                const uint64_t *par = x.gpool + (s ? hf : hm) * gw + b;
+                g0 = par[0];
+                g1 = par[nbk];
+            }
+        }
+        for (int q = 0; q < per && left; q++) left &= left - 1ull;
     }
 }
 
@@ -2403,7 +2577,10 @@ __device__ __forceinline__ void scatter_agent(const CtxT &x, const StepArgs &sa,
 // 55 us at 1.39 M agents, 18.4 at 369 k and 6.4 at 6 k; so 41, 12.7 and 5.
 // (Non-temporal stores: 95 and 26; a line is written in pieces, by several
 // waves, and must stay in the cache until it is whole.)
-__global__ void __launch_bounds__(kScatterBlock) k_cell_scatter(Ctx x, StepArgs sa) {
+template <bool kGen>
+__global__ void __launch_bounds__(kScatterBlock) k_cell_scatter(Ctx x, std::conditional_t<kGen, Prog, int32_t> p,
+                                                                StepArgs sa) {
+    __shared__ __align__(16) uint32_t sd[kGen ? 4 * kScatterBlock : 4];   // scatter_genomes
     const int tid = threadIdx.x, lane = tid & 63;
     const int pr = (int)sa.parity;
     const int64_t stride = (int64_t)(gridDim.x - 1) * kScatterBlock;
@@ -2456,149 +2633,14 @@ __global__ void __launch_bounds__(kScatterBlock) k_cell_scatter(Ctx x, StepArgs 
         }
         return;
     }
-    for (bool first = true; i < n; i += stride, first = false) {
-        if (!first) scatter_load(x, sa, i, a);
-        scatter_agent(x, sa, i, a, max_id, gbase);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// genetics: GeneUtils::makeMultiMask / crossOver / freeReco / mutateNucs
-// (GeneUtils.cpp:112-246, :322-360), one genome word per lane
-// ---------------------------------------------------------------------------
-
-// bits lo..hi (inclusive, lo <= hi <= 63)
-__device__ __forceinline__ uint64_t bit_range(int lo, int hi) {
-    const uint64_t up = (hi >= 63) ? ~0ull : ((1ull << (hi + 1)) - 1ull);
-    return up & ~((1ull << lo) - 1ull);
-}
-
-// Word w of a child genome (Genetics::makeOffspring, Genetics.cpp:285-337):
-// strand s = w / nbk comes from parent s (0 mother, 1 father), block
-// b = w % nbk.  The draws follow makeOffspring's order: i1, i2, the mother's
-// crossover draws, the father's, the mutation count, then (position, mask)
-// pairs; mutations that hit this word are applied here.  Draws 0-3 and the
-// block holding the mutation count are computed once.
-template <typename CtxT, typename ProgT>
-__device__ uint64_t child_word(const CtxT &x, const ProgT &p, uint32_t step, uint64_t nid, const uint64_t *par,
-                               int s, int b, int nbk, int w) {
-    uint32_t d0[4];
-    draw4(x.seed, step, QHG_STREAM_GENETICS, nid, 0, d0);
-    auto D = [&](uint32_t n) -> uint32_t {
-        if (n < 4) {
-            uint32_t v = d0[0];
-#pragma unroll
-            for (int q = 1; q < 4; q++) if ((uint32_t)q == n) v = d0[q];
-            return v;
+    for (bool first = true; i - tid < n; i += stride, first = false) {   // whole waves: they share the genomes
+        ScatPlan pl{-1, -1, -1, 0};
+        if (i < n) {
+            if (!first) scatter_load(x, sa, i, a);
+            pl = scatter_plan(x, sa, i, a);
         }
-        return draw(x.seed, step, QHG_STREAM_GENETICS, nid, n);
-    };
-    const int sel = (int)(2 * 1.0 * wrandd(s ? d0[1] : d0[0]));   // i1 for the mother, i2 for the father
-    const int C = p.gen_cross;
-    uint64_t word;
-    uint32_t nmut;
-    if (C > 0) {
-        // GeneUtils::crossOver (GeneUtils.cpp:184-246) restricted to block b:
-        // this parent's breaks are draws 2 + s*C + q, q < C
-        const uint32_t nbits = (uint32_t)nbk * 64u;
-        int before = 0, in = 0;
-        for (int q = 0; q < C; q++) {
-            const uint32_t bp = wrandi(0, nbits, 2, D(2 + (uint32_t)(s * C + q)));
-            before += (int)(bp >> 6) < b;
-            in += (int)(bp >> 6) == b;
-        }
-        const int cur = before & 1;
-        const uint64_t gc = par[cur * nbk + b], go = par[(1 - cur) * nbk + b];
-        uint64_t L = ~0ull;
-        if (in) {
-            // makeMultiMask (GeneUtils.cpp:156-175) over the block's breaks in
-            // draw order, walked from the last: bit 63-j takes the current
-            // value; a break at bit v flips it at j = 64-v, but only if that j
-            // is still ahead, otherwise the walk stops there (unsorted breaks,
-            // repeats and breaks at bit 0 included)
-            uint32_t k = 1u - (uint32_t)(in % 2);
-            int jc = 0;
-            uint64_t m = 0;
-            for (int q = C - 1; q >= 0; q--) {
-                const uint32_t bp = wrandi(0, nbits, 2, D(2 + (uint32_t)(s * C + q)));
-                if ((int)(bp >> 6) != b) continue;
-                const int t = 64 - (int)(bp & 63u);
-                if (t > 63 || t <= jc) break;
-                if (k) m |= bit_range(64 - t, 63 - jc);
-                k = 1u - k;
-                jc = t;
-            }
-            if (k) m |= bit_range(0, 63 - jc);
-            L = m;
-        }
-        word = (sel == 0) ? ((L & gc) | (~L & go)) : ((L & go) | (~L & gc));
-        nmut = 2 + 2 * (uint32_t)C;
-    } else if (C == -1) {
-        // freeReco + makeFreeMask (GeneUtils.cpp:322-360): two draws per block
-        const uint32_t n0 = 2 + (uint32_t)(s * 2 * nbk + 2 * b);
-        uint64_t v = ((uint64_t)D(n0) << 32) + D(n0 + 1);
-        v &= 0x5555555555555555ull;
-        v += v << 1;
-        const uint64_t a0 = par[b], a1 = par[nbk + b];
-        word = (sel == 0) ? ((v & a0) | (~v & a1)) : ((v & a1) | (~v & a0));
-        nmut = 2 + 4 * (uint32_t)nbk;
-    } else {
-        word = par[sel * nbk + b];
-        nmut = 2;
-    }
-    if (p.nbino > 0) {
-        // BinomialDist::getN then GeneUtils::mutateNucs (GeneUtils.cpp:112-141)
-        uint32_t dm[4];
-        const uint32_t mb = nmut >> 2;
-        draw4(x.seed, step, QHG_STREAM_GENETICS, nid, mb, dm);
-        auto M = [&](uint32_t n) -> uint32_t {
-            if ((n >> 2) == mb) {
-                uint32_t v = dm[0];
-#pragma unroll
-                for (int q = 1; q < 4; q++) if ((uint32_t)q == (n & 3u)) v = dm[q];
-                return v;
-            }
-            return draw(x.seed, step, QHG_STREAM_GENETICS, nid, n);
-        };
-        const double um = wrandd(M(nmut));
-        int k = 0;
-        while (k < p.nbino && um > p.bino[k]) k++;
-        const uint32_t nbits_all = 2u * 2u * (uint32_t)p.gen_size;
-        for (int j = 0; j < k; j++) {
-            const uint32_t bp = wrandi(0, nbits_all, 2, M(nmut + 1 + 2 * (uint32_t)j));
-            if ((int)(bp >> 6) == w) {
-                const uint64_t mk = (uint64_t)wrandi(1, 4, 1, M(nmut + 2 + 2 * (uint32_t)j));
-                word ^= mk << (bp & 63u);
-            }
-        }
-    }
-    return word;
-}
-
-// k_genome: the step's births, one lane per genome word (64 / gwords births
-// per wave when a genome has at most 64 words)
-__global__ void __launch_bounds__(kWave) k_genome(Ctx x, Prog p, StepArgs sa) {
-    if (x.st->error) return;
-    const int lane = threadIdx.x;
-    const int pr = (int)sa.parity;
-    const int64_t B = x.st->births_last;
-    const int64_t max_id = x.st->max_id[pr];
-    const int64_t gbase = x.st->gpool[pr];
-    const int gw = x.gwords, nbk = gw / 2;
-    const int per = (gw <= kWave) ? kWave / gw : 1;
-    const int pb = (gw <= kWave) ? lane / gw : 0;
-    for (int64_t base = (int64_t)blockIdx.x * per; base < B; base += (int64_t)gridDim.x * per) {
-        const int64_t rg = base + pb;
-        if (pb >= per || rg >= B) continue;
-        const int32_t ms = x.brec[2 * rg], fs = x.brec[2 * rg + 1];
-        const int64_t hm = x.cur.ghandle[ms], hf = x.cur.ghandle[fs];
-        const uint64_t nid = (uint64_t)(max_id + 1 + rg);
-        uint64_t *out = x.gpool + (gbase + rg) * gw;
-        for (int w = (gw <= kWave) ? lane % gw : lane; w < gw; w += (gw <= kWave) ? gw : kWave) {
-            const int s = w / nbk, b = w % nbk;
-            const uint64_t *par = x.gpool + (s ? hf : hm) * gw;
-            out[w] = child_word(x, p, sa.step, nid, par, s, b, nbk, w);
-        }
+        if constexpr (kGen) scatter_genomes(x, p, sa, pl.rg, a.gh, pl.fh, max_id, gbase, sd + 4 * (tid & ~63));
+        scatter_write(x, sa, a, pl, max_id, gbase);
     }
 }
 
@@ -2622,12 +2664,12 @@ struct PopDesc {
 };
 
 // The batch step index lives in device memory, one copy per kernel of the
-// step (act, scan, scatter, genome), so the launch arguments stay the same
+// step (act, scan, scatter), so the launch arguments stay the same
 // from step to step and one step can be captured in a graph and replayed.
 // Every kernel reads its own copy; block 0 sets the next kernel's copy, which
 // no running kernel reads, and the last kernel of the step advances the act
 // kernel's copy for the next step.
-enum BatchCounter { BC_ACT, BC_SCAN, BC_SCATTER, BC_GENOME, BC_COUNT };
+enum BatchCounter { BC_ACT, BC_SCAN, BC_SCATTER, BC_COUNT };
 
 struct BatchArgs {
     const PopDesc *pops;
@@ -2638,14 +2680,14 @@ struct BatchArgs {
     uint64_t *tiles2;         //   ... and occupied-cell totals (k_batch_scan_sums)
     int64_t *bctr;            // BC_COUNT copies of the batch step index
     uint32_t gdiv;            // as StepArgs
-    int32_t genome;           // k_batch_genome runs in this step
+    int32_t pad;
 };
 
 __device__ __forceinline__ int64_t batch_step_in(const BatchArgs &B, int k, int next) {
     const int64_t b = uniform_i64(B.bctr[k]);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (next >= 0) B.bctr[next] = b;
-        if (next < 0 || (k == BC_SCATTER && !B.genome)) B.bctr[BC_ACT] = b + 1;
+        if (next < 0) B.bctr[BC_ACT] = b + 1;
     }
     return b;
 }
@@ -2898,9 +2940,11 @@ __global__ void __launch_bounds__(kScanBlock) k_batch_scan(BatchArgs B) {
     }
 }
 
+template <bool kGen>
 __global__ void __launch_bounds__(kScatterBlock) k_batch_scatter(BatchArgs B) {
+    __shared__ __align__(16) uint32_t sd[kGen ? 4 * kScatterBlock : 4];   // scatter_genomes
     const int tid = threadIdx.x, lane = tid & 63;
-    const int64_t bstep = batch_step_in(B, BC_SCATTER, BC_GENOME);
+    const int64_t bstep = batch_step_in(B, BC_SCATTER, -1);
     if (blockIdx.x == 0) {
         if (tid >= kWave) return;
         // close every member's step and copy its status into host memory,
@@ -2947,55 +2991,16 @@ __global__ void __launch_bounds__(kScatterBlock) k_batch_scatter(BatchArgs B) {
         const StepArgs sa = pop_step_args_uniform(*dp, bstep, B.gdiv);
         ConstCtx &x = dp->ctx[sa.parity];
         const DevStatus *st = x.st;
+        const int64_t max_id = st->max_id[sa.parity], gbase = st->gpool[sa.parity];
+        ScatPlan pl{-1, -1, -1, 0};
+        ScatItem a;
         if (i < st->n_alive[sa.parity]) {
-            ScatItem a;
             scatter_load(x, sa, i, a);
-            scatter_agent(x, sa, i, a, st->max_id[sa.parity], st->gpool[sa.parity]);
+            pl = scatter_plan(x, sa, i, a);
         }
-    }
-}
-
-// births of every member with Genetics, one lane per genome word
-__global__ void __launch_bounds__(kWave) k_batch_genome(BatchArgs B) {
-    const int lane = threadIdx.x;
-    const int64_t bstep = batch_step_in(B, BC_GENOME, -1);
-    int64_t cnt[4], base[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int r = lane + 64 * k;
-        cnt[k] = 0;
-        if (r < B.npops) {
-            ConstCtx &x0 = pop_desc(B, r).ctx[0];
-            if (x0.gwords && !x0.st->error) {
-                const int per = (x0.gwords <= kWave) ? kWave / x0.gwords : 1;
-                cnt[k] = (x0.st->births_last + per - 1) / per;   // births of the step just scanned
-            }
-        }
-    }
-    const int64_t total = pop_prefix(cnt, base);
-    for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
-        const int r = pop_of(base, B.npops, g);
-        const int64_t gl = g - lane_value(base, r);
-        const DevStatus *st = pop_desc(B, r).ctx[0].st;
-        const StepArgs sa = pop_step_args_uniform(pop_desc(B, r), bstep, B.gdiv);
-        const int par = (int)sa.parity;
-        ConstCtx &x = *uniform_ptr(&pop_desc(B, r).ctx[par]);
-        ConstProg &pg = *uniform_ptr(&pop_desc(B, r).prog);
-        const int gw = x.gwords, nbk = gw / 2;
-        const int per = (gw <= kWave) ? kWave / gw : 1;
-        const int pb = (gw <= kWave) ? lane / gw : 0;
-        const int64_t rg = gl * per + pb;
-        if (pb >= per || rg >= st->births_last) continue;
-        const int64_t max_id = st->max_id[par], gbase = st->gpool[par];
-        const int32_t ms = x.brec[2 * rg], fs = x.brec[2 * rg + 1];
-        const int64_t hm = x.cur.ghandle[ms], hf = x.cur.ghandle[fs];
-        const uint64_t nid = (uint64_t)(max_id + 1 + rg);
-        uint64_t *out = x.gpool + (gbase + rg) * gw;
-        for (int w = (gw <= kWave) ? lane % gw : lane; w < gw; w += (gw <= kWave) ? gw : kWave) {
-            const int s = w / nbk, b = w % nbk;
-            const uint64_t *par_g = x.gpool + (s ? hf : hm) * gw;
-            out[w] = child_word(x, pg, sa.step, nid, par_g, s, b, nbk, w);
-        }
+        if (kGen && x.gwords)
+            scatter_genomes(x, dp->prog, sa, pl.rg, a.gh, pl.fh, max_id, gbase, sd + 4 * (tid & ~63));
+        scatter_write(x, sa, a, pl, max_id, gbase);
     }
 }
 

@@ -47,7 +47,9 @@ QHG_HD void draw4(uint64_t seed, uint32_t step, uint32_t stream, uint64_t id,
 QHG_HD uint32_t draw(uint64_t seed, uint32_t step, uint32_t stream, uint64_t id, uint32_t n) {
     uint32_t o[4];
     draw4(seed, step, stream, id, n >> 2, o);
-    return o[n & 3];
+    // (selects: an index would put the four words into memory)
+    const uint32_t lo = (n & 1) ? o[1] : o[0], hi = (n & 1) ? o[3] : o[2];
+    return (n & 2) ? hi : lo;
 }
 
 // WELL512::wrandd: double in [0,1)

@@ -51,8 +51,8 @@ namespace {
             return fail(QHG_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-enum KernelId { KB_ACT, KB_SCAN, KB_SCATTER, KB_GENOME, KB_CAPACITY, KB_EVAL, KB_GPOOL, KB_ASSORT, KB_PROT, KB_COUNT };
-const char *kKernelNames[KB_COUNT] = {"k_cell_act", "k_cell_scan",     "k_cell_scatter", "k_genome",
+enum KernelId { KB_ACT, KB_SCAN, KB_SCATTER, KB_CAPACITY, KB_EVAL, KB_GPOOL, KB_ASSORT, KB_PROT, KB_COUNT };
+const char *kKernelNames[KB_COUNT] = {"k_cell_act", "k_cell_scan",     "k_cell_scatter",
                                       "k_capacity", "k_eval", "k_gpool_compact", "k_assort_pair", "k_proteins"};
 
 constexpr int kRing = kStatusRing;
@@ -128,7 +128,6 @@ struct qhg_pop {
     // per-slot step scratch (cap entries)
     uint64_t *d_dec = nullptr;
     uint8_t *d_gflag = nullptr;
-    int32_t *d_brec = nullptr;
     int32_t *d_gfu = nullptr, *d_gmu = nullptr, *d_gfs = nullptr, *d_gms = nullptr, *d_gmate = nullptr;
     int64_t *d_gfid = nullptr, *d_gmid = nullptr;
     uint32_t *d_gprot = nullptr;   // AssortativePair: kProtBudget digests per slot
@@ -237,7 +236,6 @@ struct qhg_pop {
         x.grp_cap = group_entries(cap, ncells);
         x.dec = d_dec;
         x.brank = reinterpret_cast<uint64_t *>(d_gmid);   // the lists of k_cell_act are done when it is written
-        x.brec = d_brec;
         x.gfu = d_gfu;
         x.gmu = d_gmu;
         x.gfs = d_gfs;
@@ -317,7 +315,7 @@ int grid_items(const qhg_pop *p, int64_t items) {
 // slots), genome pools, per-cell tables, fixed-size scratch
 int64_t device_bytes(const qhg_pop *p) {
     const int64_t g = p->gwords ? 1 : 0;
-    const int64_t per_slot = 2 * (46 + 4 * g) + 45 + 8 * g + (p->has_prot ? 16 * kProtBudget + 4 : 0);
+    const int64_t per_slot = 2 * (46 + 4 * g) + 45 + (p->has_prot ? 16 * kProtBudget + 4 : 0);
     int64_t b = p->cap * per_slot + 2 * group_entries(p->cap, p->ncells) * (int64_t)sizeof(GroupDesc);
     for (int k = 0; k < 2; k++)
         if (p->d_gpool[k]) b += p->gcap * p->gwords * 8;
@@ -447,13 +445,13 @@ int collect_timing(qhg_pop *p) {
 }
 
 void free_slot_scratch(qhg_pop *p) {
-    void *ptrs[] = {p->d_dec, p->d_gflag, p->d_brec, p->d_gfu, p->d_gmu, p->d_gfs, p->d_gms,
+    void *ptrs[] = {p->d_dec, p->d_gflag, p->d_gfu, p->d_gmu, p->d_gfs, p->d_gms,
                     p->d_gmate, p->d_gfid, p->d_gmid, p->d_gprot, p->d_gnprot};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     p->d_dec = nullptr;
     p->d_gflag = nullptr;
-    p->d_brec = p->d_gfu = p->d_gmu = p->d_gfs = p->d_gms = p->d_gmate = nullptr;
+    p->d_gfu = p->d_gmu = p->d_gfs = p->d_gms = p->d_gmate = nullptr;
     p->d_gfid = p->d_gmid = nullptr;
     p->d_gprot = nullptr;
     p->d_gnprot = nullptr;
@@ -473,7 +471,6 @@ int alloc_slot_scratch(qhg_pop *p, int64_t cap) {
     HIPCHK(hipMalloc(&p->d_gmate, n * 4));
     HIPCHK(hipMalloc(&p->d_gfid, n * 8));
     HIPCHK(hipMalloc(&p->d_gmid, n * 8));
-    if (p->gwords) HIPCHK(hipMalloc(&p->d_brec, n * 8));
     if (p->has_prot) {
         HIPCHK(hipMalloc(&p->d_gprot, n * 16 * kProtBudget));
         HIPCHK(hipMalloc(&p->d_gnprot, n * 4));
@@ -1274,12 +1271,10 @@ int phase_finalize(qhg_pop *p) {
     if (rc) return rc;
     // one more block than the agents use: the step's bookkeeping
     const int64_t runs = (p->known.n_alive[p->known_step & 1] + kScatterBlock - 1) / kScatterBlock;
-    rc = launch_bs(p, KB_SCATTER, k_cell_scatter, grid_items(p, runs) + 1, kScatterBlock, x, sa);
+    const int sgrid = grid_items(p, runs) + 1;
+    rc = p->gwords ? launch_bs(p, KB_SCATTER, k_cell_scatter<true>, sgrid, kScatterBlock, x, p->prog, sa)
+                   : launch_bs(p, KB_SCATTER, k_cell_scatter<false>, sgrid, kScatterBlock, x, (int32_t)0, sa);
     if (rc) return rc;
-    if (p->gwords) {
-        rc = launch_bs(p, KB_GENOME, k_genome, p->num_cu * 16, kWave, x, p->prog, sa);
-        if (rc) return rc;
-    }
     p->acted = false;
     p->initialized = false;
     p->steps_enqueued++;
@@ -2118,13 +2113,13 @@ int qhg_gpu_autotune(qhg_pop *p, int32_t trial_steps, qhg_tuning *chosen, int32_
 // ===========================================================================
 // Batched stepping (many populations per launch)
 // ===========================================================================
-enum BatchKernelId { BK_ACT, BK_SCAN, BK_SCATTER, BK_GENOME, BK_SCAN_SUMS, BK_COUNT };
+enum BatchKernelId { BK_ACT, BK_SCAN, BK_SCATTER, BK_SCAN_SUMS, BK_COUNT };
 
 struct qhg_batch {
     hipStream_t stream = nullptr;
     int device = 0;
     int num_cu = 256;
-    int scan_grid = 1, genome_grid = 1;
+    int scan_grid = 1;
     int act_per_cu[3] = {1, 1, 1};   // blocks of the act kernels (plain, age deaths, Navigate) a CU holds
     std::vector<qhg_pop *> pops;
     std::vector<int64_t> gens, step0, join;
@@ -2189,7 +2184,6 @@ BatchArgs batch_args(const qhg_batch *b) {
     A.tiles2 = b->d_tiles2;
     A.bctr = b->d_bctr;
     A.gdiv = b->gdiv;
-    A.genome = b->any_genetics ? 1 : 0;
     return A;
 }
 
@@ -2216,10 +2210,8 @@ int batch_launch_step(qhg_batch *b) {
     rc = blaunch(b, BK_SCAN, k_batch_scan, sg, kScanBlock, A);
     if (rc) return rc;
     // one more block than the agents use: the members' bookkeeping
-    rc = blaunch(b, BK_SCATTER, k_batch_scatter, cg + 1, kScatterBlock, A);
-    if (rc) return rc;
-    if (b->any_genetics) return blaunch(b, BK_GENOME, k_batch_genome, b->genome_grid, kWave, A);
-    return 0;
+    return b->any_genetics ? blaunch(b, BK_SCATTER, k_batch_scatter<true>, cg + 1, kScatterBlock, A)
+                           : blaunch(b, BK_SCATTER, k_batch_scatter<false>, cg + 1, kScatterBlock, A);
 }
 
 void batch_drop_graph(qhg_batch *b) {
@@ -2360,7 +2352,6 @@ int qhg_batch_create(qhg_batch **out) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, act[k], kActBlock, 0) == hipSuccess && n > 1)
             b->act_per_cu[k] = n;
     }
-    b->genome_grid = b->num_cu * 16;
     *out = b;
     return 0;
 }
@@ -2574,8 +2565,7 @@ int qhg_batch_set_timing(qhg_batch *b, int32_t enable) {
 }
 
 const char *qhg_batch_kernel_name(int32_t index) {
-    static const char *names[BK_COUNT] = {"k_batch_act", "k_batch_scan", "k_batch_scatter", "k_batch_genome",
-                                          "k_batch_scan_sums"};
+    static const char *names[BK_COUNT] = {"k_batch_act", "k_batch_scan", "k_batch_scatter", "k_batch_scan_sums"};
     if (index < 0 || index >= BK_COUNT) return "";
     return names[index];
 }

@@ -209,3 +209,44 @@ def test_assortative_groups_match_the_oracle(kind, model):
         paired += int((got["mate_id"] >= 0).sum())
     assert paired > 0 or kind in ("ones", "alone")
     gpu.close()
+
+
+@pytest.mark.parametrize("genome_size,crossovers,rate", [
+    (4, 1, 0.2), (32, 5, 0.3), (32, 0, 0.0), (33, -1, 0.1), (97, 9, 0.1), (192, 3, 0.05), (500, 1, 0.02), (1024, -1, 1e-3),
+    (1025, 32, 1e-3), (2048, 2, 5e-3)])
+def test_genome_draws_match_the_oracle(genome_size, crossovers, rate):
+    """Genomes of 2 to 128 words (32 births a pass of a wave to one birth in
+    two passes, widths that do not divide a wave); draws within a birth's
+    lanes' numbers and past them; mutation counts in and past the binomial
+    table's first entries; alone and as a batch's members."""
+    print("case: genome size %d, crossovers %d, rate %g" % (genome_size, crossovers, rate), flush=True)
+    scs = []
+    for seed in (61, 62):
+        sc = scenarios.c2(seed=seed, level=3, n_agents=2500, patch_cells=60, genetics=True, genome_size=genome_size)
+        p = sc["params"]
+        p.gen_num_crossover, p.gen_mutation_rate = crossovers, rate
+        words = 2 * abi.genome_words(genome_size)
+        rng = np.random.default_rng(seed + genome_size)
+        sc["agents"]["genome"] = rng.integers(0, 2**63, len(sc["agents"]["id"]) * words, dtype=np.uint64)
+        scs.append(sc)
+    gpu, oras = GpuPopulation.from_scenario(scs[0]), [Oracle(sc) for sc in scs]
+    members = [GpuPopulation.from_scenario(sc) for sc in scs]
+    for pop in [gpu] + members:
+        pop.preLoop()
+    for ora in oras:
+        ora.pre_loop()
+    batch = GpuBatch()
+    for m in members:
+        batch.add(m)
+    for k in range(3):
+        gpu.run(8)
+        batch.run(8)
+        for ora in oras:
+            ora.run(8)
+        assert_same_state(gpu.agents(), oras[0].agents(), "alone, step %d" % (8 * k + 8))
+        for m, ora in zip(members, oras):
+            assert_same_state(m.agents(), ora.agents(), "in a batch, step %d" % (8 * k + 8))
+    assert oras[0].agents()["id"].max() > 2700      # (births: ids past the first 2500)
+    batch.close()
+    for pop in [gpu] + members:
+        pop.close()
