@@ -277,13 +277,21 @@ AGENT_FIELDS = {
 }
 
 
+class _AgentAddresses(C.Structure):
+    """Agents with plain addresses: ten pointer objects cost 20 us to make."""
+    _fields_ = [(name, C.c_int64 if name == "n" else C.c_void_p) for name, _ in Agents._fields_]
+
+
 def agents_struct(arrays, n):
     """Build an Agents struct pointing into a dict of numpy arrays."""
-    a = Agents()
-    a.n = n
-    for name, (_, ct) in AGENT_FIELDS.items():
-        setattr(a, name, ptr(arrays.get(name), ct))
-    a.genome = ptr(arrays.get("genome"), C.c_uint64)
+    raw = _AgentAddresses(n)
+    for name, _ in Agents._fields_[1:]:
+        arr = arrays.get(name)
+        if arr is not None:
+            assert arr.flags["C_CONTIGUOUS"]
+            setattr(raw, name, arr.ctypes.data)
+    a = Agents.from_buffer(raw)
+    a._arrays = arrays          # what it points into lives as long as it does
     return a
 
 

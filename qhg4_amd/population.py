@@ -145,12 +145,12 @@ class GpuPopulation:
         return out
 
     def capacities(self):
-        out = np.zeros(self.grid["num_cells"], dtype=np.float64)
+        out = np.empty(self.grid["num_cells"], dtype=np.float64)
         check(lib().qhg_gpu_capacities(self.h, abi.ptr(out, C.c_double)), "qhg_gpu_capacities")
         return out
 
     def env_weights(self):
-        out = np.zeros(self.grid["num_cells"] * (self.grid["connectivity"] + 1), dtype=np.float64)
+        out = np.empty(self.grid["num_cells"] * (self.grid["connectivity"] + 1), dtype=np.float64)
         check(lib().qhg_gpu_env_weights(self.h, abi.ptr(out, C.c_double)), "qhg_gpu_env_weights")
         return out
 

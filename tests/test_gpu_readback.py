@@ -58,3 +58,49 @@ def test_agents_come_back_in_id_order(kind, gwords):
         if gwords:
             assert np.array_equal(got["genome"], agents["genome"].reshape(n, gwords)[back])
     pop.close()
+
+
+@pytest.mark.parametrize("n,gwords", [(60000, 0), (85000, 0), (524287, 0), (524289, 0), (1572900, 0), (24575, 16),
+                                      (24576, 16), (32768, 16), (32769, 16), (131073, 16)])
+def test_large_reads_arrive_whole(n, gwords):
+    """Reads around the sizes at which they leave through the copying threads
+    (3 MB), at a chunk's end (4 MB), and round the ring of three chunks."""
+    from qhg4_amd.population import GpuPopulation
+    print("case: %d agents, %d genome words" % (n, gwords), flush=True)
+    rng = np.random.default_rng(n)
+    grid = rect_grid(101, 97)
+    agents = {
+        "id": rng.permutation(n).astype(np.int64), "cell": rng.integers(0, grid["num_cells"], n).astype(np.int32),
+        "life": rng.choice([1, 5], n).astype(np.uint8), "gender": rng.integers(0, 2, n).astype(np.uint8),
+        "birth_time": rng.uniform(-40, 0, n), "age": rng.uniform(0, 40, n), "last_birth": rng.uniform(-9, 0, n),
+        "num_babies": rng.integers(0, 9, n).astype(np.int32), "mate_id": np.full(n, -3, dtype=np.int64),
+    }
+    actions = [(abi.ACT_GETOLD, 1)]
+    kw = {}
+    if gwords:
+        actions.append((abi.ACT_GENETICS, 2))
+        kw = dict(gen_genome_size=32 * gwords // 2, gen_num_crossover=1, gen_mutation_rate=0.0)
+        agents["genome"] = rng.integers(0, 1 << 62, n * gwords, dtype=np.int64).astype(np.uint64)
+    pop = GpuPopulation(grid, {}, scenarios.make_params(1, actions, **kw), agents, capacity=n + 64)
+    pop.preLoop(0.0)
+    back = np.argsort(agents["id"])
+    got = pop.agents()
+    for k in abi.AGENT_FIELDS:
+        assert np.array_equal(got[k], agents[k][back]), k
+    if gwords:
+        assert np.array_equal(got["genome"], agents["genome"].reshape(n, gwords)[back])
+    pop.close()
+
+
+@pytest.mark.parametrize("level", [6, 7])
+def test_large_tables_arrive_whole(level):
+    """Movement weights of 2.3 MB (one copy) and 9.2 MB (three chunks)."""
+    from oracle.oracle import Oracle
+    from qhg4_amd.population import GpuPopulation
+    sc = scenarios.c2(seed=5, level=level, n_agents=200, patch_cells=50)
+    pop, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    pop.preLoop()
+    ora.pre_loop()
+    assert np.array_equal(pop.env_weights(), ora.env_weights())
+    assert np.array_equal(pop.capacities(), ora.capacities())
+    pop.close()
