@@ -1026,7 +1026,11 @@ struct GroupActLds {
 // used, each costs a trip to the scalar cache on the chain).  With one wave
 // per group of ~4 cells, 60 % of the lanes filled and the picks one after
 // another, the kernel took 137 us at 1.39 M agents, 38.5 at 369 k and 15.5 at
-// 6 k; in this form 55, 20 and 10.
+// 6 k; in this form 55, 20 and 10, and with its registers held to five blocks
+// per CU instead of four (the compiler's own choice; no spills) 47 at 1.39 M:
+// 3.6 waves per SIMD had left a third of the issue slots idle.  Six blocks
+// spill: 47 and 21 at 369 k.  Navigation and the batch, whose contexts lie in
+// memory, take four instead of three: 31 to 27 us and 54 to 45.
 template <bool kRare, bool kAssort, bool kNav>
 __device__ __forceinline__ void group_act(ConstCtx *xp, ConstProg *pp, uint32_t step, double t, GroupDesc d0,
                                           GroupDesc d1, GroupActLds &G, uint32_t &my_deaths, uint32_t &my_moves,
@@ -1345,12 +1349,12 @@ __device__ __forceinline__ void cell_act_kernel() {
 }
 
 template <bool kRare, bool kAssort>
-__global__ void __launch_bounds__(kActBlock) k_cell_act(ActArgs) {
+__global__ void __launch_bounds__(kActBlock, kRare ? 4 : 5) k_cell_act(ActArgs) {
     cell_act_kernel<kRare, kAssort, false>();
 }
 
 template <bool kRare, bool kAssort>
-__global__ void __launch_bounds__(kActBlock) k_cell_act_nav(ActArgs) {
+__global__ void __launch_bounds__(kActBlock, 4) k_cell_act_nav(ActArgs) {
     cell_act_kernel<kRare, kAssort, true>();
 }
 
@@ -2791,7 +2795,7 @@ __device__ __forceinline__ void batch_items(const BatchArgs &B, int64_t bstep, i
 }
 
 template <bool kRare, bool kNav = false>
-__global__ void __launch_bounds__(kActBlock) k_batch_act(BatchArgs B) {
+__global__ void __launch_bounds__(kActBlock, kRare ? 3 : 4) k_batch_act(BatchArgs B) {
     __shared__ GroupActLds lds;
     __shared__ uint32_t part[kParts];
     const int tid = threadIdx.x;

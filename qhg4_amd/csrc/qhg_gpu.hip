@@ -122,6 +122,8 @@ struct qhg_pop {
     int num_cu = 256;
     int max_grid = 1;         // blocks of k_cell_act and k_cell_scatter, at most
     int act_grid = 1;         // blocks of the current step's k_cell_act
+    void (*act_kern)(ActArgs) = nullptr;   // that kernel, and its resident blocks per CU
+    int act_per_cu = 1;
     int scan_grid = 1, ntiles = 1;
     // launch shapes (results do not depend on them)
     double group_agents = QHG_GROUP_AGENTS;
@@ -1386,7 +1388,16 @@ int phase_act(qhg_pop *p) {
                                           : (p->has_assort ? k_cell_act_nav<false, true> : k_cell_act_nav<false, false>))
               : p->has_rare ? (p->has_assort ? k_cell_act<true, true> : k_cell_act<true, false>)
                             : (p->has_assort ? k_cell_act<false, true> : k_cell_act<false, false>);
-    p->act_grid = grid_items(p, p->known.n_grp[p->known_step & 1]);
+    // no more blocks than are resident at once: a block takes its next group
+    // without a launch and a prologue (with 16 per CU 19.2 us at 369 k agents,
+    // so 17.5; at 1.39 M the same)
+    if (p->act_kern != kern) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, kActBlock, 0) != hipSuccess || n < 1) n = 1;
+        p->act_kern = kern;
+        p->act_per_cu = n;
+    }
+    p->act_grid = std::min(grid_items(p, p->known.n_grp[p->known_step & 1]), p->num_cu * p->act_per_cu);
     int rc = launch_bs(p, KB_ACT, kern, p->act_grid, kActBlock, ActArgs{p->ctx(), p->prog, p->step_args()});
     if (rc) return rc;
     p->acted = true;
