@@ -1403,9 +1403,13 @@ __global__ void __launch_bounds__(256) k_act_commit(Ctx x, StepArgs sa, int32_t 
 // two full lists, as 255, which no lists give); 0 does not count.  The
 // rounds are serial within a cell and short, so 16 lanes take a cell and a
 // block its ~14 cells at once; a wave per cell left most lanes idle and took
-// 55 us at 369 k agents against 25.6 here (7 blocks per CU; 29.5 at 5), the
-// protein matches, recomputed from global memory in every round, 913 us at
-// 80 k agents against 51 and k_proteins' 28.
+// 55 us at 369 k agents against 25.6 with the table in LDS (7 blocks per CU;
+// 29.5 at 5), the protein matches, recomputed from global memory in every
+// round, 913 us at 80 k agents against 51 and k_proteins' 28.  With the
+// rounds of cells up to 16 x 16 in registers 20.4 and, digests compared four
+// by four as well, 31: cells of a dozen fertile agents are the rule (none
+// beyond 14 females or 13 males at 348 k), and the kernel lasts as long as
+// its longest chains.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int bitcount2(uint64_t v) {   // GeneUtils::bitcount2
     return __popcll((v | (v >> 1)) & 0x5555555555555555ull);
@@ -1617,6 +1621,16 @@ struct AssortLds {
 };
 
 constexpr int kSub = 16;   // lanes per cell in the rounds
+constexpr int kProtStep = 4;
+
+// the largest value of a row of 16 lanes (non-negative values)
+__device__ __forceinline__ int row_max16(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true));   // row_ror:8
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, true));   // row_ror:4
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, true));   // row_ror:2
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, true));   // row_ror:1
+    return v;
+}
 
 __device__ __forceinline__ int select16(uint32_t v, int k) {
     int pos = 0, c = __popc(v & 0xFFu);
@@ -1626,6 +1640,134 @@ __device__ __forceinline__ int select16(uint32_t v, int k) {
     c = __popc(v & 0x3u);
     if (k >= c) { k -= c; v >>= 2; pos += 2; }
     return pos + ((k >= (int)(v & 1u)) ? 1 : 0);
+}
+
+// lane N's value in the whole row of 16
+template <int N>
+__device__ __forceinline__ uint32_t row_bcast16(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + N, 0xf, 0xf, true);   // row_newbcast
+}
+
+// f(I), f(I + 1), ... below N, as constants, until one returns false
+template <int I, int N, typename F>
+__device__ __forceinline__ void each_lane16(F &f) {
+    if constexpr (I < N)
+        if (f(std::integral_constant<int, I>{})) each_lane16<I + 1, N>(f);
+}
+
+// bits of the bytes of v that equal b (its copy in every byte), lowest first
+__device__ __forceinline__ uint32_t equal_bytes4(uint32_t v, uint32_t b) {
+    const uint32_t d = v ^ b;
+    const uint32_t z = ~(((d & 0x7f7f7f7fu) + 0x7f7f7f7fu) | d | 0x7f7f7f7fu);   // 0x80 where d is 0
+    return (((z >> 7) * 0x01020408u) >> 24) & 15u;
+}
+
+// A cell's draws in order, a window of 16 (lane l: the l-th next) at a time.
+struct RowDraws {
+    uint32_t u0, u1, base, at, have;   // draws base + l and base + 16 + l (have of them); the next to use
+
+    template <typename DrawF>
+    __device__ __forceinline__ uint32_t window(int l, int sh, uint32_t need, DrawF draw_of) {
+        if (at - base >= 16u) {
+            u0 = (have > 16u) ? u1 : draw_of(base + 16u + (uint32_t)l);
+            base += 16u;
+            have = 16u;
+        }
+        if (at - base + need > 16u && have == 16u) {
+            u1 = draw_of(base + 16u + (uint32_t)l);
+            have = 32u;
+        }
+        const uint32_t k = at - base + (uint32_t)l;
+        const uint32_t a = (uint32_t)__shfl((int)u0, sh + (int)(k & 15u), 64);
+        if (have == 16u) return a;
+        const uint32_t b = (uint32_t)__shfl((int)u1, sh + (int)(k & 15u), 64);
+        return (k < 16u) ? a : b;
+    }
+};
+
+// The rounds of a cell of at most 16 females and 16 males, in registers: lane
+// l holds female l's row of the table (four words), and what one lane has the
+// others read by row broadcasts (one instruction, where a shuffle or a table
+// in LDS costs some 100 cycles; the rounds are one chain of such steps).
+// order[] of a round as in assort_rounds: the swaps move positions, so every
+// female follows her own.
+template <bool kProt>
+__device__ __forceinline__ void assort_rounds16(const Ctx &x, const Prog &p, const StepArgs &sa, AssortLds<kProt> &L,
+                                                int32_t c, int F, int Mw, const uint32_t *Tw, int f0, int m0, int l,
+                                                int sh) {
+    const uint32_t lt = (1u << l) - 1u;
+    const auto votes = [&](bool v) -> uint32_t { return (uint32_t)(__ballot(v) >> sh) & 0xFFFFu; };
+    const auto draw_of = [&](uint32_t j) -> uint32_t { return assort_draw(x.seed, sa.step, c, j); };
+    uint32_t row[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) row[j] = (l < F && j < Mw) ? Tw[l * Mw + j] : 0u;
+    RowDraws ds{draw_of((uint32_t)l), 0u, 0u, 0u, 16u};
+    uint32_t free_males = 0xFFFFu;
+    for (;;) {
+        int mine = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t v = row[j];
+            mine = max(mine, (int)max(max(v & 255u, (v >> 8) & 255u), max((v >> 16) & 255u, v >> 24)));
+        }
+        const int top = row_max16(mine);
+        if (top == 0) break;
+        const uint32_t reach = votes(mine == top);
+        const int np = __popc(reach);
+        // her place among those that reach it, in id order; the others after them
+        int pos = (mine == top) ? __popc(reach & lt) : np + __popc(~reach & lt);
+        if (p.assort_permute && np > 2) {
+            // for i = np-1 down to 2: swap entry i with entry wrandi(0, i)
+            const uint32_t u = ds.window(l, sh, (uint32_t)(np - 2), draw_of);
+            const uint32_t to = __umulhi((uint32_t)(np - 1 - l), u);   // (used from lanes below np - 2)
+            auto swap = [&](auto s) -> bool {
+                constexpr int S = decltype(s)::value;
+                if (S >= np - 2) return false;
+                const int i = np - 1 - S, q = (int)row_bcast16<S>(to);
+                pos = (pos == i) ? q : (pos == q) ? i : pos;
+                return true;
+            };
+            each_lane16<0, 14>(swap);
+            ds.at += (uint32_t)(np - 2);
+        }
+        // by position: the female and the males at that value
+        uint32_t males = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) males |= equal_bytes4(row[j], (uint32_t)top * 0x01010101u) << (4 * j);
+        const uint32_t turn =
+            (uint32_t)__builtin_amdgcn_ds_permute((sh + pos) * 4, (int)(males | ((uint32_t)l << 16)));
+        uint32_t u = ds.window(l, sh, (uint32_t)np, draw_of);
+        uint32_t got = 0;              // her male's bit
+        const uint32_t before = free_males;
+        // each female in turn: a random unpaired male at that value
+        auto pair = [&](auto q) -> bool {
+            constexpr int Q = decltype(q)::value;
+            if (Q >= np) return false;
+            const uint32_t v = row_bcast16<Q>(turn);
+            const uint32_t mk = v & free_males;
+            if (mk & 0xFFFFu) {
+                const int sel = (int)__umulhi((uint32_t)__popc(mk & 0xFFFFu), row_bcast16<0>(u));
+                const uint32_t bit = votes(((mk >> l) & 1u) && __popc(mk & lt) == sel);
+                free_males &= ~bit;
+                if ((v >> 16) == (uint32_t)l) got = bit;
+                u = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, 0x101, 0xf, 0xf, true);   // row_shl:1
+                ds.at++;
+            }
+            return true;
+        };
+        each_lane16<0, 16>(pair);
+        const uint32_t taken = before & ~free_males;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t m = (((taken >> (4 * j)) & 15u) * 0x00204081u) & 0x01010101u;
+            row[j] = got ? 0u : row[j] & ~(m * 255u);
+        }
+        if (got) {
+            const int jm = __ffs((int)got) - 1;
+            L.prt[f0 + l] = (int16_t)(m0 - jm);
+            L.prt[m0 - jm] = (int16_t)(f0 + l);
+        }
+    }
 }
 
 // The table and the rounds of group cell k, by the 16 lanes (l) of a quarter
@@ -1656,11 +1798,21 @@ __device__ __forceinline__ void assort_rounds(const Ctx &x, const Prog &p, const
             const int nf = min((int)L.np[f0 + i], kProtBudget), nm = min((int)L.np[m0 - j], kProtBudget);
             const int of = L.poff[f0 + i], om = L.poff[m0 - j];
             if (of >= 0 && om >= 0) {
-                for (int q = 0; q < nf; q++) {
-                    const Digest df = L.pool[of + q];
-                    for (int r = 0; r < nm; r++) {
-                        const Digest dm = L.pool[om + r];
-                        v += (df.lo == dm.lo && df.hi == dm.hi) ? 1 : 0;
+                // four of each at a time, their reads in flight together (past
+                // a list's end its first one, not counted)
+                for (int q0 = 0; q0 < nf; q0 += kProtStep) {
+                    Digest df[kProtStep];
+#pragma unroll
+                    for (int q = 0; q < kProtStep; q++) df[q] = L.pool[of + (q0 + q < nf ? q0 + q : 0)];
+                    for (int r0 = 0; r0 < nm; r0 += kProtStep) {
+                        Digest dm[kProtStep];
+#pragma unroll
+                        for (int r = 0; r < kProtStep; r++) dm[r] = L.pool[om + (r0 + r < nm ? r0 + r : 0)];
+#pragma unroll
+                        for (int q = 0; q < kProtStep; q++)
+#pragma unroll
+                            for (int r = 0; r < kProtStep; r++)
+                                v += (q0 + q < nf && r0 + r < nm && df[q].lo == dm[r].lo && df[q].hi == dm[r].hi) ? 1 : 0;
                     }
                 }
             } else {
@@ -1675,6 +1827,10 @@ __device__ __forceinline__ void assort_rounds(const Ctx &x, const Prog &p, const
         T[t] = (uint8_t)v;
     }
     wave_sync();
+    if (F <= kSub && M <= kSub) {
+        assort_rounds16<kProt>(x, p, sa, L, c, F, Mw, Tw, f0, m0, l, sh);
+        return;
+    }
     // the cell's draws, computed 16 at a time and taken in order
     uint32_t dj = 0, ubase = 0;
     uint32_t U = assort_draw(x.seed, sa.step, c, (uint32_t)l);
@@ -1701,11 +1857,7 @@ __device__ __forceinline__ void assort_rounds(const Ctx &x, const Prog &p, const
             L.rmax[f0 + i] = (uint8_t)rm;
             top = rm > top ? rm : top;
         }
-#pragma unroll
-        for (int d = kSub / 2; d >= 1; d >>= 1) {
-            const int o = __shfl_xor(top, d, 64);
-            top = o > top ? o : top;
-        }
+        top = row_max16(top);
         if (top == 0) break;
         wave_sync();
         // females reaching it, in id order

@@ -250,3 +250,47 @@ def test_genome_draws_match_the_oracle(genome_size, crossovers, rate):
     batch.close()
     for pop in [gpu] + members:
         pop.close()
+
+
+@pytest.mark.parametrize("changed", [0, 1, 4])
+@pytest.mark.parametrize("model", ["hamming", "hamming_noperm", "protein"])
+def test_assortative_rounds_match_the_oracle(model, changed):
+    """Rounds of cells up to and past 16 females or males (16 lanes' registers
+    and the table in LDS): all matches equal (every female in one round, the
+    draws past a window of 16), and few to many different values."""
+    rng = np.random.default_rng(57)
+    prot = model == "protein"
+    sc = scenarios.c2(seed=57, level=3, n_agents=10, patch_cells=5, genetics=True, protein=prot,
+                      assort=((1.0, 1) if prot else (0.5, 0 if model == "hamming_noperm" else 1)))
+    sc["params"].npp_k_max = 600.0
+    sizes = [(1, 1), (1, 16), (16, 1), (2, 3), (3, 2), (4, 5), (7, 8), (8, 7), (9, 12), (15, 16), (16, 15), (16, 16),
+             (16, 17), (17, 16), (17, 17), (1, 17), (17, 1), (14, 16), (16, 4), (20, 30)] * 3
+    cells = rng.choice(sc["grid"]["num_cells"], len(sizes), replace=False)
+    cell = np.concatenate([np.full(f + m, c) for (f, m), c in zip(sizes, cells)]).astype(np.int32)
+    gender = np.concatenate([rng.permutation([0] * f + [1] * m) for f, m in sizes]).astype(np.uint8)
+    n = len(cell)
+    if prot:
+        genome = _protein_genomes(np.random.default_rng(3), 1, 256, 4).reshape(1, -1)
+    else:
+        genome = scenarios.initial_genomes(np.random.default_rng(3), 1, 256).reshape(1, -1)
+    genome = np.repeat(genome, n, axis=0)
+    for _ in range(changed):
+        genome[np.arange(n), rng.integers(0, genome.shape[1], n)] ^= np.uint64(1) << rng.integers(0, 64, n).astype(np.uint64)
+    age = rng.uniform(0, 40, n)
+    sc["agents"] = {
+        "id": rng.permutation(np.arange(1, 3 * n + 1, dtype=np.int64))[:n], "cell": cell,
+        "life": np.full(n, abi.QHG_LIFE_FERTILE, dtype=np.uint8), "gender": gender, "birth_time": -age, "age": age,
+        "last_birth": np.full(n, -5.0), "mate_id": np.full(n, -3, dtype=np.int64),
+        "num_babies": np.zeros(n, dtype=np.int32), "genome": np.ascontiguousarray(genome.ravel())}
+    gpu, ora = GpuPopulation.from_scenario(sc), Oracle(sc)
+    gpu.preLoop()
+    ora.pre_loop()
+    paired = 0
+    for k in range(4):
+        gpu.run(1)
+        ora.run(1)
+        got = gpu.agents()
+        assert_same_state(got, ora.agents(), "%s %d step %d" % (model, changed, k))
+        paired += int((got["mate_id"] >= 0).sum())
+    assert paired > 0
+    gpu.close()
