@@ -294,9 +294,8 @@ namespace qhg {
 // Every pass is a stream over the agents or over the bitmap.  At 369 k and
 // 1.39 M agents a read took 39 and 215 ms with the order, the mates' liveness
 // and the gather on the host (an indirect std::sort and a binary search per
-// agent), 1.3 and 4.0 ms with them here (1.39 M with 128-byte genomes: 341 ->
-// 13.7 ms); what is left is the copy to the caller's pageable arrays at
-// 15-20 GB/s.
+// agent), 0.6 and 1.9 ms with them here (1.39 M with 128-byte genomes: 341 ->
+// 5.4 ms); what is left is the copy to the caller's pageable arrays (copy_out).
 // ---------------------------------------------------------------------------
 constexpr int kRankBlock = 256;
 constexpr int kRankPer = 8;                          // bitmap words per thread
@@ -440,6 +439,141 @@ __global__ void __launch_bounds__(kRankBlock) k_read_agents(RankMap m, AgentBuf 
         if (o.age) o.age[r] = a.age[i];
         if (o.lastb) o.lastb[r] = a.lastb[i];
         if (o.nbabies) o.nbabies[r] = a.nbabies[i];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Small reads in one launch.  Every block keeps the whole bitmap in LDS, from
+// the lowest live id on, and finds the agents of its kReadOut ranks itself:
+// reading all ids (from L2, up to kReadIds per thread, once) costs less than
+// the five dependent launches before.  At 6 k agents the call took 52 us with
+// them, 35 with this one (a step and its read 90 and 70 us; with twice the ids
+// per thread, for up to 32 k agents, 36).  Ids that span more than the bitmap
+// holds leave *how set, and the caller takes the launches above.
+// ---------------------------------------------------------------------------
+constexpr int kReadBlock = 1024;
+constexpr int kReadIds = 16;                          // ids per thread
+constexpr int kReadOut = 256;                         // agents a block writes
+constexpr int kReadWords = 4096;                      // bitmap words in LDS
+constexpr int64_t kReadSmall = kReadBlock * kReadIds; // agents at most
+
+__global__ void __launch_bounds__(kReadBlock) k_read_small(AgentBuf a, const OccCell *occ, int64_t nocc, int32_t ncells,
+                                                           int32_t n, uint32_t *slot_of, ReadOut o, int32_t *how) {
+    constexpr int kWaves = kReadBlock / kWave, kPer = kReadWords / kReadBlock;
+    __shared__ unsigned long long bits[kReadWords];
+    __shared__ uint16_t pre[kReadWords];              // live ids before a word (n at most kReadSmall)
+    __shared__ uint32_t list[kReadOut];
+    __shared__ long long wmin[kWaves];
+    __shared__ uint32_t wsum[kWaves];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    int64_t id[kReadIds];
+    int64_t low = INT64_MAX;
+#pragma unroll
+    for (int k = 0; k < kReadIds; k++) {
+        const int i = k * kReadBlock + tid;
+        id[k] = (i < n) ? a.id[i] : INT64_MAX;
+    }
+#pragma unroll
+    for (int k = 0; k < kReadIds; k++) low = id[k] < low ? id[k] : low;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) bits[k * kReadBlock + tid] = 0ull;
+    if (tid < kReadOut) list[tid] = 0xFFFFFFFFu;
+#pragma unroll
+    for (int d = kWave / 2; d >= 1; d >>= 1) {
+        const int64_t v = __shfl_xor((long long)low, d, kWave);
+        low = v < low ? v : low;
+    }
+    if (lane == 0) wmin[wave] = low;
+    __syncthreads();
+    low = wmin[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; w++) low = wmin[w] < low ? wmin[w] : low;
+    bool wide = low < 0;
+    low &= ~63ll;
+#pragma unroll
+    for (int k = 0; k < kReadIds; k++) {
+        if (k * kReadBlock + tid >= n) continue;
+        const uint64_t at = (uint64_t)(id[k] - low);
+        if (at >= 64ull * kReadWords) wide = true;
+        else atomicOr(&bits[at >> 6], 1ull << (at & 63));
+    }
+    if (__syncthreads_or(wide)) {
+        if (tid == 0) *how = 1;
+        return;
+    }
+    uint32_t c[kPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        c[k] = (uint32_t)__popcll(bits[tid * kPer + k]);
+        sum += c[k];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += y;
+    }
+    if (lane == kWave - 1) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t before = incl - sum;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) before += (w < wave) ? wsum[w] : 0u;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        pre[tid * kPer + k] = (uint16_t)before;
+        before += c[k];
+    }
+    __syncthreads();
+    const int r0 = (int)blockIdx.x * kReadOut;
+#pragma unroll
+    for (int k = 0; k < kReadIds; k++) {
+        const int i = k * kReadBlock + tid;
+        if (i >= n) continue;
+        const uint64_t at = (uint64_t)(id[k] - low);
+        const int r = (int)pre[at >> 6] + __popcll(bits[at >> 6] & ((1ull << (at & 63)) - 1ull)) - r0;
+        if (r >= 0 && r < kReadOut) list[r] = (uint32_t)i;
+    }
+    __syncthreads();
+    // a quarter of the block per group of fields
+    const int q = tid / kReadOut, r = tid & (kReadOut - 1);
+    static_assert(kReadBlock == 4 * kReadOut, "four groups of fields");
+    const int64_t out = r0 + r;
+    if (out >= n) return;
+    const uint32_t i = list[r];
+    if (i >= (uint32_t)n) {
+        *how = 1;
+        return;
+    }
+    if (q == 0) {
+        if (slot_of) slot_of[out] = i;
+        if (o.cell) {
+            int64_t lo = 0, hi = nocc;   // occ[lo].s <= i < occ[hi].s
+            while (hi - lo > 1) {
+                const int64_t mid = (lo + hi) / 2;
+                if (occ[mid].s <= i) lo = mid;
+                else hi = mid;
+            }
+            const OccCell e = occ[lo];
+            if (i < e.s || i >= e.s + e.n || e.c < 0 || e.c >= ncells) *how = 1;
+            o.cell[out] = e.c;
+        }
+    } else if (q == 1) {
+        if (o.id) o.id[out] = a.id[i];
+        if (o.mate) {
+            // the partner's id while it lives, -1 once it has died
+            const int64_t v = a.mate_id[i];
+            const uint64_t at = (uint64_t)(v - low);
+            const bool alive = v >= low && at < 64ull * kReadWords && ((bits[at >> 6] >> (at & 63)) & 1ull);
+            o.mate[out] = (v >= 0 && !alive) ? -1 : v;
+        }
+        if (o.nbabies) o.nbabies[out] = a.nbabies[i];
+    } else if (q == 2) {
+        if (o.birth) o.birth[out] = a.birth[i];
+        if (o.age) o.age[out] = a.age[i];
+    } else {
+        if (o.lastb) o.lastb[out] = a.lastb[i];
+        if (o.life) o.life[out] = a.life[i];
+        if (o.gender) o.gender[out] = a.gender[i];
     }
 }
 

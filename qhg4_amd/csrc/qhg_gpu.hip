@@ -170,6 +170,7 @@ struct qhg_pop {
     size_t read_bytes = 0;
     char *h_copy = nullptr;   // copy_out's pinned ring and its slots' events (made by the first large copy)
     hipEvent_t copy_ev[kCopySlots] = {};
+    std::atomic<bool> read_wide{false};   // a one-launch read found ids too far apart
     std::mutex read_mu;       // readers on several threads share the scratch above
     DevStatus *d_st = nullptr;
 
@@ -988,10 +989,13 @@ int copy_out(qhg_pop *p, const CopyPiece *pieces, int count) {
     return 0;
 }
 
+constexpr int kReadAgain = 1;   // the ids do not fit the one-launch read
+
 // The live agents in id order, ordered on the device (aux_kernels.hpp).  The
 // buffer the next step writes is free between steps and takes the arrays;
-// the list scratch takes the order and the cells.
-int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
+// the list scratch takes the order and the cells.  small: in one launch if
+// the agents are few.
+int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a, bool small) {
     std::lock_guard<std::mutex> lock(p->read_mu);
     const int b = p->cur();
     const int64_t n = s.n_alive[b];
@@ -1007,8 +1011,9 @@ int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
     const bool pinned = want + 64 <= kReadPinned;
     int rc = read_buffer(p, pinned ? want + 64 : 64);
     if (rc) return rc;
+    small = small && pinned && n <= kReadSmall;
     RankMap m{};
-    rc = rank_map(p, s.max_id[b], &m);
+    if (!small) rc = rank_map(p, s.max_id[b], &m);
     if (rc) return rc;
     // the pool a compaction writes next takes the ordered genome rows
     uint64_t *&rows = p->d_gpool[1 - p->gp_cur];
@@ -1028,15 +1033,21 @@ int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
     const dim3 blk(kRankBlock);
     const int ga = grid_for(n, p->num_cu * 8);
     hipStream_t st = p->stream;
-    hipLaunchKernelGGL(k_rank_clear, dim3(grid_for(m.words, p->num_cu * 8)), blk, 0, st, m);
-    hipLaunchKernelGGL(k_rank_mark, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n);
-    hipLaunchKernelGGL(k_rank_tiles, dim3(std::min(m.tiles, p->num_cu * 8)), blk, 0, st, m);
-    hipLaunchKernelGGL(k_rank_base, dim3(1), blk, 0, st, m);
-    hipLaunchKernelGGL(k_rank_slots, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n, slot_of, d_bad);
     ReadOut o{(int64_t *)to[0], (int64_t *)to[1], (int32_t *)to[5], (int32_t *)to[6], (uint8_t *)to[7],
               (uint8_t *)to[8], (double *)to[2],  (double *)to[3],  (double *)to[4]};
-    hipLaunchKernelGGL(k_read_agents, dim3(ga), blk, 0, st, m, d, (const OccCell *)p->d_occ[b], s.n_occ[b], p->ncells,
-                       (const uint32_t *)slot_of, n, o, d_bad);
+    if (small) {
+        hipLaunchKernelGGL(k_read_small, dim3((unsigned)((n + kReadOut - 1) / kReadOut)), dim3(kReadBlock), 0, st, d,
+                           (const OccCell *)p->d_occ[b], s.n_occ[b], p->ncells, (int32_t)n, genomes ? slot_of : nullptr, o,
+                           d_bad);
+    } else {
+        hipLaunchKernelGGL(k_rank_clear, dim3(grid_for(m.words, p->num_cu * 8)), blk, 0, st, m);
+        hipLaunchKernelGGL(k_rank_mark, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n);
+        hipLaunchKernelGGL(k_rank_tiles, dim3(std::min(m.tiles, p->num_cu * 8)), blk, 0, st, m);
+        hipLaunchKernelGGL(k_rank_base, dim3(1), blk, 0, st, m);
+        hipLaunchKernelGGL(k_rank_slots, dim3(ga), blk, 0, st, m, (const int64_t *)d.id, n, slot_of, d_bad);
+        hipLaunchKernelGGL(k_read_agents, dim3(ga), blk, 0, st, m, d, (const OccCell *)p->d_occ[b], s.n_occ[b], p->ncells,
+                           (const uint32_t *)slot_of, n, o, d_bad);
+    }
     if (genomes)
         hipLaunchKernelGGL(k_read_genomes, dim3(grid_for(n * p->gwords, p->num_cu * 16)), blk, 0, st,
                            (const int32_t *)d.ghandle, (const uint64_t *)p->d_gpool[p->gp_cur], s.gpool[b], p->gwords,
@@ -1050,6 +1061,7 @@ int read_agents_ranked(qhg_pop *p, const DevStatus &s, qhg_agents *a) {
     if (genomes) large[pieces++] = {a->genome, rows, (size_t)n * p->gwords * 8};
     rc = copy_out(p, large, pieces);
     if (rc) return rc;
+    if (*bad && small) return kReadAgain;
     if (*bad) return fail(QHG_ERR_STATE, "download: the agents, the cell list or the genome handles disagree");
     if (pinned) {
         at = 64;
@@ -1828,7 +1840,16 @@ int qhg_gpu_download_agents(qhg_pop *p, qhg_agents *a) {
     rc = look_inside(p);
     if (rc) return rc;
     if (n > 0) {
-        rc = s.max_id[b] < kRankIdLimit ? read_agents_ranked(p, s, a) : QHG_ERR_NOMEM;
+        rc = QHG_ERR_NOMEM;
+        if (s.max_id[b] < kRankIdLimit) {
+            rc = read_agents_ranked(p, s, a, !p->read_wide);
+            if (rc == kReadAgain) {
+                // ids spread that widely stay so (the oldest agents live on):
+                // the next reads do not try again
+                p->read_wide = true;
+                rc = read_agents_ranked(p, s, a, false);
+            }
+        }
         if (rc == QHG_ERR_NOMEM) {
             (void)hipGetLastError();   // a failed allocation's error is not the next launch's
             rc = read_agents_sorted(p, s, a);

@@ -104,3 +104,46 @@ def test_large_tables_arrive_whole(level):
     assert np.array_equal(pop.env_weights(), ora.env_weights())
     assert np.array_equal(pop.capacities(), ora.capacities())
     pop.close()
+
+
+SPAN = 64 * 4096      # ids that one launch's bitmap holds
+
+
+@pytest.mark.parametrize("gwords", [0, 4])
+@pytest.mark.parametrize("n,first,span", [(1, 5, 1), (2, 63, SPAN - 63), (2, 64, SPAN), (2, 64, SPAN + 1), (255, 0, 300),
+                                          (256, 1000, 256), (257, 1, 4096), (1024, 77, 5000), (1025, 77, 1025),
+                                          (5000, 1 << 20, SPAN - 64), (5000, (1 << 20) + 1, SPAN + 64),
+                                          (16383, 129, SPAN - 200), (16384, 3, 16384), (16385, 3, 16385)])
+def test_small_reads_match(n, first, span, gwords):
+    """Reads of one launch at the edges of its blocks, its agents and its ids,
+    and past them (partners are not uploaded: none)."""
+    from qhg4_amd.population import GpuPopulation
+    print("case: %d agents, ids %d..%d" % (n, first, first + span - 1), flush=True)
+    rng = np.random.default_rng(n + span)
+    inner = rng.choice(max(0, span - 2), max(0, n - 2), replace=False) + first + 1 if n > 2 else np.zeros(0, np.int64)
+    ids = np.unique(np.concatenate([[first], inner, [first + span - 1]]).astype(np.int64))
+    assert len(ids) == n
+    order = rng.permutation(n)
+    grid = rect_grid(23, 19)
+    agents = {
+        "id": ids[order], "cell": rng.integers(0, grid["num_cells"], n).astype(np.int32),
+        "life": rng.choice([1, 5], n).astype(np.uint8), "gender": rng.integers(0, 2, n).astype(np.uint8),
+        "birth_time": rng.uniform(-40, 0, n), "age": rng.uniform(0, 40, n), "last_birth": rng.uniform(-9, 0, n),
+        "num_babies": rng.integers(0, 9, n).astype(np.int32), "mate_id": np.full(n, -3, dtype=np.int64),
+    }
+    actions = [(abi.ACT_GETOLD, 1)]
+    kw = {}
+    if gwords:
+        actions.append((abi.ACT_GENETICS, 2))
+        kw = dict(gen_genome_size=32 * gwords // 2, gen_num_crossover=1, gen_mutation_rate=0.0)
+        agents["genome"] = rng.integers(0, 1 << 62, n * gwords, dtype=np.int64).astype(np.uint64)
+    pop = GpuPopulation(grid, {}, scenarios.make_params(1, actions, **kw), agents, capacity=n + 64)
+    pop.preLoop(0.0)
+    back = np.argsort(agents["id"])
+    for _ in range(2):
+        got = pop.agents()
+        for k in abi.AGENT_FIELDS:
+            assert np.array_equal(got[k], agents[k][back]), k
+        if gwords:
+            assert np.array_equal(got["genome"], agents["genome"].reshape(n, gwords)[back])
+    pop.close()
